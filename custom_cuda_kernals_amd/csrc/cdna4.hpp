@@ -17,6 +17,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "fp8_codec.hpp"
 
 namespace cck {
@@ -479,5 +481,95 @@ struct RowBuf<false, SPOL> {
   __device__ void st8(const u32x2& v, uint32_t off) const { st_stream(v, reinterpret_cast<u32x2*>(p + off)); }
   __device__ void st4(uint32_t v, uint32_t off) const { st_stream(v, reinterpret_cast<uint32_t*>(p + off)); }
 };
+
+// ---------------------------------------------------------------------------
+// Rows that start at any element boundary (odd lengths, sliced buffers). A
+// row is still taken as 16-byte vectors from its own first element, so vector
+// v holds the same elements as in an aligned row: global accesses of gfx950
+// may start at any byte. Measured on MI355X, a 256 MiB copy by 16-byte vectors
+// (nontemporal): aligned 84.0 us; loads 8 / 4 / 2 bytes off 85.1 / 84.9 /
+// 86.8; stores off 87.6 / 87.6 / 88.2; both off 88.8 / 88.8 / 91.9. The last
+// n < VEC elements of such a row are a partial vector, moved one by one.
+// ---------------------------------------------------------------------------
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+typedef u32x2 u32x2_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint16_t u16_any __attribute__((aligned(1)));
+
+// RowBuf's interface (nontemporal) over a row that starts at any byte.
+struct RowAny {
+  char* p;
+  __device__ RowAny(const void* base, uint32_t) : p(static_cast<char*>(const_cast<void*>(base))) {}
+  __device__ u32x4 ld16(uint32_t off) const {
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p + off));
+  }
+  // Cached: for rows that every workgroup reads.
+  __device__ u32x4 ld16_cached(uint32_t off) const { return *reinterpret_cast<const u32x4_any*>(p + off); }
+  __device__ void st16(const u32x4& v, uint32_t off) const {
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any*>(p + off));
+  }
+  __device__ void st8(const u32x2& v, uint32_t off) const {
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x2_any*>(p + off));
+  }
+  __device__ void st4(uint32_t v, uint32_t off) const {
+    __builtin_nontemporal_store(v, reinterpret_cast<u32_any*>(p + off));
+  }
+};
+
+// Byte offset at which vector v of a ragged row of `nwhole` whole vectors is
+// loaded. The partial vector (v == nwhole, npart elements) is loaded as the
+// row's last VEC elements, so its load is an ordinary one inside the row;
+// partial_vector then drops the VEC - npart elements of its neighbour.
+// Loading the elements one by one instead took up to 58 VGPRs more than
+// the widest rows have. Rows have at least VEC elements.
+template <class C>
+__device__ inline uint32_t ragged_offset(uint32_t v, int nwhole, int npart) {
+  return v * 16u - (v == (uint32_t)nwhole ? (uint32_t)((C::VEC - npart) * C::kBytes) : 0u);
+}
+// The last npart elements of w moved to the front, zeros after them.
+template <class C>
+__device__ inline u32x4 partial_vector(u32x4 w, int npart) {
+  const int drop = (C::VEC - npart) * C::kBytes;
+  if (drop & 8) w = (u32x4){w[2], w[3], 0u, 0u};
+  if (drop & 4) w = (u32x4){w[1], w[2], w[3], 0u};
+  if (C::kBytes == 2 && (drop & 2)) {
+    w = (u32x4){w[0] >> 16 | w[1] << 16, w[1] >> 16 | w[2] << 16, w[2] >> 16 | w[3] << 16, w[3] >> 16};
+  }
+  return w;
+}
+// The first n elements of v (1 <= n < VEC) to p: at most one store of 8, one
+// of 4 and one of 2 bytes.
+template <class C>
+__device__ inline void store_partial(const u32x4& v, int n, char* p) {
+  const int bytes = n * C::kBytes;
+  u32x2 lo = {v[0], v[1]};
+  if (bytes & 8) {
+    *reinterpret_cast<u32x2_any*>(p) = lo;
+    lo = (u32x2){v[2], v[3]};
+    p += 8;
+  }
+  if (bytes & 4) {
+    *reinterpret_cast<u32_any*>(p) = lo[0];
+    lo[0] = lo[1];
+    p += 4;
+  }
+  if (C::kBytes == 2 && (bytes & 2)) *reinterpret_cast<u16_any*>(p) = (uint16_t)lo[0];
+}
+// The first n of VEC packed codes (1 <= n < VEC) to q.
+template <int VEC>
+__device__ inline void store_codes_partial(const uint32_t (&w)[VEC / 4], int n, uint8_t* q) {
+  uint32_t c = w[0];
+  if (VEC == 8 && (n & 4)) {
+    *reinterpret_cast<u32_any*>(q) = c;
+    c = w[VEC / 4 - 1];
+    q += 4;
+  }
+  if (n & 2) {
+    *reinterpret_cast<u16_any*>(q) = (uint16_t)c;
+    c >>= 16;
+    q += 2;
+  }
+  if (n & 1) *q = (uint8_t)c;
+}
 
 }  // namespace cck

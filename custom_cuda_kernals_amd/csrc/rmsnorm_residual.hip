@@ -56,13 +56,27 @@ __device__ inline void scale_round_mul(float (&f)[C::VEC], float inv, const floa
 // row length, the per-vector bounds checks and the whole summation plan are
 // compile-time constants. Measured on MI355X at [16384, 4096] bf16,
 // per-token FP8: see the launcher.
-template <class C, int THREADS, int ITEMS, int MODE, int FMT, bool FULL>
-__global__ __launch_bounds__(THREADS) void rmsnorm_resident(
+//
+// RAGGED: any row length from VEC elements up and any element-aligned
+// pointers. The row is taken as VEC-element vectors from its own start (see
+// RowAny), the last one partial, so every step is the aligned kernel's and
+// the bits are too; only the accesses differ. The partial vector's absent
+// elements are zeros to the sum and to the amax and are not stored. What bounds
+// it beyond the aligned rows' traffic is occupancy (64-bit row addresses): the
+// wave floor below and y held packed took 256 x 3 per-token rows from 141 to 116
+// VGPRs and 256 x 2 from 103 to 90, [3001, 4100] from 25.4 to 23.1 us.
+enum RowForm : int { kRowGeneral, kRowFull, kRowRagged };
+
+constexpr int min_waves(RowForm form, int items) { return form != kRowRagged ? 1 : items == 2 ? 5 : items == 1 ? 6 : 4; }
+
+template <class C, int THREADS, int ITEMS, int MODE, int FMT, RowForm FORM>
+__global__ __launch_bounds__(THREADS, min_waves(FORM, ITEMS)) void rmsnorm_resident(
     const void* __restrict__ x, const void* __restrict__ res, const void* __restrict__ w,
     void* __restrict__ y, uint8_t* __restrict__ yq, float* __restrict__ scale,
     void* __restrict__ ro, int64_t rows, int64_t cols_arg, float eps, float static_scale) {
   constexpr int NW = THREADS / 64;
   constexpr int VEC = C::VEC;
+  constexpr bool FULL = FORM == kRowFull, RAGGED = FORM == kRowRagged;
   constexpr int NREG = (THREADS * ITEMS * VEC + kRegionAddends - 1) / kRegionAddends;
   __shared__ uint32_t lds[2 * NW];
   using RowSum = ResidentRowSum<VEC, THREADS, ITEMS, FULL>;
@@ -70,7 +84,9 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
   __shared__ float sum_blocks[2 * NREG * kFoldLanes];
   __shared__ float sum_tail[FULL ? 1 : 2 * kTailWords];
   const int64_t cols = FULL ? (int64_t)THREADS * ITEMS * VEC : cols_arg;
-  const int nvec = (int)(cols / VEC);
+  const int nwhole = (int)(cols / VEC);                // whole vectors
+  const int npart = RAGGED ? (int)(cols % VEC) : 0;    // elements of the partial vector after them
+  const int nvec = nwhole + (RAGGED && npart != 0 ? 1 : 0);
   // Vector v of the row exists (always, for a full row).
   auto in_row = [&](uint32_t v) { return FULL || v < (uint32_t)nvec; };
   const AtenSumPlan plan(cols);
@@ -78,14 +94,16 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
   const uint32_t row_bytes = (uint32_t)(cols * C::kBytes);
   auto load_row = [&](int64_t row, u32x4 (&xa)[ITEMS], u32x4 (&ra)[ITEMS]) {
     const int64_t off = row * cols * C::kBytes;
-    const RowBuf<true> bx(static_cast<const char*>(x) + off, row_bytes);
-    const RowBuf<true> br(static_cast<const char*>(res) + off, row_bytes);
+    using Row = std::conditional_t<RAGGED, RowAny, RowBuf<true>>;
+    const Row bx(static_cast<const char*>(x) + off, row_bytes);
+    const Row br(static_cast<const char*>(res) + off, row_bytes);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const uint32_t v = threadIdx.x + k * THREADS;
       if (in_row(v)) {
-        xa[k] = bx.ld16(v * 16u);
-        ra[k] = br.ld16(v * 16u);
+        const uint32_t at = RAGGED ? ragged_offset<C>(v, nwhole, npart) : v * 16u;
+        xa[k] = bx.ld16(at);
+        ra[k] = br.ld16(at);
       }
     }
   };
@@ -96,11 +114,20 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
   // row loads do not wait for it, measured 1.5-5 % slower on MI355X.
   constexpr bool kHoistW = ITEMS <= 2;
   u32x4 wreg[kHoistW ? ITEMS : 1];
+  auto load_w = [&](int v) {
+    if constexpr (RAGGED) {
+      // As loaded: moving the partial vector to the front here would wait for
+      // this load before the row loads go out.
+      return RowAny(w, 0).ld16_cached(ragged_offset<C>((uint32_t)v, nwhole, npart));
+    } else {
+      return wv[v];
+    }
+  };
   if constexpr (kHoistW) {
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const int v = threadIdx.x + k * THREADS;
-      if (in_row(v)) wreg[k] = wv[v];
+      if (in_row(v)) wreg[k] = load_w(v);
     }
   }
   // A workgroup's first row is loaded at kernel entry, ahead of the loop
@@ -123,7 +150,8 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
   // contiguous block of rows (65 % vs 75 % of peak at [8192, 4096] bf16).
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x, parity ^= 1) {
     const int64_t off = row * cols * C::kBytes;
-    const RowBuf<true, ro_store_policy(MODE)> bro(static_cast<char*>(ro) + off, row_bytes);
+    const std::conditional_t<RAGGED, RowAny, RowBuf<true, ro_store_policy(MODE)>> bro(static_cast<char*>(ro) + off,
+                                                                                     row_bytes);
     if (!kPrefetch && row != (int64_t)blockIdx.x) load_row(row, xa, ra);
     u32x4 rov[ITEMS];
     // torch-CPU's summation order, which does not depend on the launch
@@ -138,12 +166,26 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
       for (int i = 0; i < VEC; ++i) sq[i] = 0.0f;
       if (in_row(v)) {
         float fx[VEC], fr[VEC], fo[VEC];
+        if constexpr (RAGGED) {
+          if (v == nwhole) {
+            xa[k] = partial_vector<C>(xa[k], npart);
+            ra[k] = partial_vector<C>(ra[k], npart);
+          }
+        }
         C::unpack(xa[k], fx);
         C::unpack(ra[k], fr);
 #pragma unroll
         for (int i = 0; i < VEC; ++i) fo[i] = fx[i] + fr[i];
         rov[k] = C::pack(fo);
-        bro.st16(rov[k], (uint32_t)v * 16u);
+        if constexpr (RAGGED) {
+          if (v == nwhole) {
+            store_partial<C>(rov[k], npart, bro.p + v * 16);
+          } else {
+            bro.st16(rov[k], (uint32_t)v * 16u);
+          }
+        } else {
+          bro.st16(rov[k], (uint32_t)v * 16u);
+        }
         C::unpack(rov[k], fo);
 #pragma unroll
         for (int i = 0; i < VEC; ++i) sq[i] = fo[i] * fo[i];
@@ -163,7 +205,8 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
     const float inv = 1.0f / __builtin_sqrtf(variance + eps);
 
     if constexpr (MODE == 0) {
-      const RowBuf<true, out_store_policy(MODE)> by(static_cast<char*>(y) + off, row_bytes);
+      const std::conditional_t<RAGGED, RowAny, RowBuf<true, out_store_policy(MODE)>> by(static_cast<char*>(y) + off,
+                                                                                       row_bytes);
 #pragma unroll
       for (int k = 0; k < ITEMS; ++k) {
         const int v = threadIdx.x + k * THREADS;
@@ -174,11 +217,20 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
           // is not hoisted above the loop as well: that made every
           // workgroup wait for its weight load before issuing its row loads
           // (43.4 vs 43.9 us at [8192, 4096] bf16 on MI355X).
-          u32x4 wk = kHoistW ? wreg[kHoistW ? k : 0] : wv[v];
+          u32x4 wk = kHoistW ? wreg[kHoistW ? k : 0] : load_w(v);
           asm("" : "+v"(wk));
+          if (RAGGED && v == nwhole) wk = partial_vector<C>(wk, npart);
           C::unpack(wk, fw);
           scale_round_mul<C>(fo, inv, fw);
-          by.st16(C::pack(fo), (uint32_t)v * 16u);
+          if constexpr (RAGGED) {
+            if (v == nwhole) {
+              store_partial<C>(C::pack(fo), npart, by.p + v * 16);
+            } else {
+              by.st16(C::pack(fo), (uint32_t)v * 16u);
+            }
+          } else {
+            by.st16(C::pack(fo), (uint32_t)v * 16u);
+          }
         }
       }
     } else {
@@ -190,7 +242,7 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
       // 52.5, 512 x 3 at 12288 124.1 vs 122.1 (but 512 x 4 at 16384 163.5 vs
       // 166.8).
       constexpr bool kPackY =
-          (MODE == 1 && ITEMS >= 4) || (MODE == 2 && (ITEMS == 3 || (ITEMS == 4 && THREADS == 1024)));
+          (RAGGED && ITEMS >= 2) || (MODE == 1 && ITEMS >= 4) || (MODE == 2 && (ITEMS == 3 || (ITEMS == 4 && THREADS == 1024)));
       float yv[kPackY ? 1 : ITEMS][VEC];
       u32x4 yp[kPackY ? ITEMS : 1];
       float amax = 0.0f;
@@ -210,10 +262,18 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
           // static 96.9 vs 98.3; 256 x 2 at [16384, 4096] per-token 76.6 vs
           // 77.0, static 74.6 vs 75.5.
           constexpr bool kOpaqueW = THREADS == 512 || (THREADS > 512 && MODE == 1);
-          u32x4 wk = kHoistW ? wreg[kHoistW ? k : 0] : wv[v];
-          if constexpr (kOpaqueW) asm("" : "+v"(wk));
+          u32x4 wk = kHoistW ? wreg[kHoistW ? k : 0] : load_w(v);
+          if constexpr (kOpaqueW || RAGGED) asm("" : "+v"(wk));
+          if (RAGGED && v == nwhole) wk = partial_vector<C>(wk, npart);
           C::unpack(wk, fw);
           scale_round_mul<C>(f, inv, fw);
+          if constexpr (RAGGED) {
+            // 0 * inv is NaN where inv is not finite: absent elements stay out of the amax.
+            if (v == nwhole) {
+#pragma unroll
+              for (int i = 0; i < VEC; ++i) f[i] = i < npart ? f[i] : 0.0f;
+            }
+          }
 #pragma unroll
           for (int i = 0; i < VEC; i += 2) {
             C::round2(f[i], f[i + 1]);
@@ -240,7 +300,8 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
       }
       const float r = 1.0f / s;
       const bool fast = fast_path_ok<FMT>(s, r, amax);
-      const RowBuf<true, out_store_policy(MODE)> bq(yq + row * cols, (uint32_t)cols);
+      const std::conditional_t<RAGGED, RowAny, RowBuf<true, out_store_policy(MODE)>> bq(yq + row * cols,
+                                                                                       (uint32_t)cols);
 #pragma unroll
       for (int k = 0; k < ITEMS; ++k) {
         const int v = threadIdx.x + k * THREADS;
@@ -258,7 +319,9 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
           } else {
             quant_exact<FMT, VEC>(f, s, wq);
           }
-          if constexpr (VEC == 8) {
+          if (RAGGED && v == nwhole) {
+            store_codes_partial<VEC>(wq, npart, yq + row * cols + (int64_t)v * VEC);
+          } else if constexpr (VEC == 8) {
             bq.st8((u32x2){wq[0], wq[1]}, (uint32_t)v * 8u);
           } else {
             bq.st4(wq[0], (uint32_t)v * 4u);
@@ -269,7 +332,8 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_resident(
   }
 }
 
-// Any alignment / row length: scalar accesses, four waves. The sum of squares
+// Rows under one vector or longer than the register-resident shapes, of any
+// alignment: scalar accesses, four waves. The sum of squares
 // follows torch-CPU's order exactly (aten_sum.hpp), so this path gives the
 // same bits as the register-resident kernel for any alignment or row length:
 // the row is cut into blocks of 2^P steps (4 * 2^P vectors of 8 addends,
@@ -393,9 +457,9 @@ int32_t launch_rmsnorm(const void* x, const void* res, const void* w, void* y, u
   const bool vec_ok = (cols % C::VEC == 0) && host_aligned(x, 16) && host_aligned(res, 16) &&
                       host_aligned(w, 16) && host_aligned(ro, 16) &&
                       (MODE == 0 ? host_aligned(y, 16) : host_aligned(yq, C::VEC));
-  const int64_t nvec = cols / C::VEC;
+  const int64_t nvec = (cols + C::VEC - 1) / C::VEC;
   const unsigned g = row_grid(rows);
-  auto run = [&](auto shape) {
+  auto launch = [&](auto shape, auto form) {
     using S = decltype(shape);
     // Wide FP8 rows run on a grid of the workgroups the device holds at once,
     // each looping over rows (no idle CU between rows, one weight load per
@@ -408,19 +472,21 @@ int32_t launch_rmsnorm(const void* x, const void* res, const void* w, void* y, u
     // 74.9 at [16384, 4096].
     constexpr int kCap = S::kThreads * S::kItems;
     constexpr bool kLoop = (MODE == 1 && kCap >= 1536) || (MODE == 2 && kCap >= 3072);
-    auto go = [&](auto full) {
-      constexpr auto kernel = rmsnorm_resident<C, S::kThreads, S::kItems, MODE, FMT, decltype(full)::value>;
-      const int64_t resident = kLoop ? resident_groups<kernel>(S::kThreads) : 0;
-      const unsigned grid = resident > 0 && resident < (int64_t)g ? (unsigned)resident : g;
-      kernel<<<grid, S::kThreads, 0, st>>>(x, res, w, y, yq, scale, ro, rows, cols, eps, static_scale);
-    };
+    constexpr auto kernel = rmsnorm_resident<C, S::kThreads, S::kItems, MODE, FMT, (RowForm)decltype(form)::value>;
+    const int64_t resident = kLoop ? resident_groups<kernel>(S::kThreads) : 0;
+    const unsigned grid = resident > 0 && resident < (int64_t)g ? (unsigned)resident : g;
+    kernel<<<grid, S::kThreads, 0, st>>>(x, res, w, y, yq, scale, ro, rows, cols, eps, static_scale);
+  };
+  auto run = [&](auto shape) {
+    constexpr int kCap = decltype(shape)::kThreads * decltype(shape)::kItems;
     // A row that fills the shape exactly in whole 512-addend regions takes
     // the compile-time-planned kernel (no per-vector bounds checks, no tail).
     if constexpr (C::VEC == 8 && (kCap * 8) % kRegionAddends == 0) {
-      if (nvec == kCap) return go(std::true_type{});
+      if (nvec == kCap) return launch(shape, IntC<kRowFull>{});
     }
-    go(std::false_type{});
+    launch(shape, IntC<kRowGeneral>{});
   };
+  auto run_ragged = [&](auto shape) { launch(shape, IntC<kRowRagged>{}); };
   // 16-byte rows (f16 / bf16): the shapes come from a sweep over every
   // THREADS in 64..1024 (step 64) x ITEMS in 1..4 holding the row, on MI355X
   // at 8192 bf16 rows of 2048..16384 elements (graph-replayed, 2 GiB
@@ -439,25 +505,51 @@ int32_t launch_rmsnorm(const void* x, const void* res, const void* w, void* y, u
   // MI355X against 1024 x 1 and 1024 x 2: 172.8 vs 196.3 us at [16384, 4096],
   // 44.2 vs 53.5 at [4096, 4096], 58.2 vs 63.4 at [4096, 5120], 177.2 vs
   // 184.6 at [8192, 8192]; 256 x 2 lost to 512 x 1 at 2048 columns).
-  bool done;
-  if constexpr (MODE == 0 && C::VEC == 8) {
-    done = vec_ok && pick_row_shape<RowShape<64, 1>, RowShape<128, 1>, RowShape<256, 1>, RowShape<320, 1>,
+  // Ragged rows (RAGGED above) of at least one vector take shapes from the
+  // same lists. The FP8 variants stop at 1024 x 3: with 64-bit row addresses
+  // 1024 x 4 spills. Longer rows, and rows under one vector, take the looping
+  // kernel, which every ragged row took before (4 waves, 2- or 4-byte
+  // accesses, residual_out read back and y formed twice). Measured on MI355X,
+  // through the Python API, looping kernel vs these, bf16 per-token FP8:
+  // [3001, 4100] 59.4 vs 23.1 us (3.7 TB/s; 20.6 for aligned rows of 4104),
+  // [16384, 101] 51.0 vs 14.3, [16384, 1005] 100.7 vs 28.1, [1524, 11005] 97.0 vs
+  // 34.8, [838, 20005] 123.6 vs 41.3; plain [4091, 4101] 76.7 vs 35.2; fp32
+  // per-token [8184, 2050] 129.8 vs 54.1.
+  bool done = false;
+  if (!vec_ok) {
+    if (cols < C::VEC) {
+    } else if constexpr (MODE == 0 && C::VEC == 8) {
+      done = pick_row_shape<RowShape<64, 1>, RowShape<128, 1>, RowShape<256, 1>, RowShape<320, 1>, RowShape<512, 1>,
+                            RowShape<768, 1>, RowShape<512, 2>, RowShape<768, 2>, RowShape<512, 4>,
+                            RowShape<1024, 4>>(nvec, run_ragged);
+    } else if constexpr (MODE == 0) {
+      done = pick_row_shape<RowShape<64, 1>, RowShape<128, 1>, RowShape<256, 1>, RowShape<512, 1>, RowShape<512, 2>,
+                            RowShape<512, 4>, RowShape<1024, 4>>(nvec, run_ragged);
+    } else if constexpr (C::VEC == 8) {
+      done = pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<256, 1>, RowShape<192, 2>, RowShape<256, 2>,
+                            RowShape<256, 3>, RowShape<512, 2>, RowShape<512, 3>, RowShape<1024, 2>, RowShape<1024, 3>>(nvec, run_ragged);
+    } else {
+      done = pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<128, 2>, RowShape<256, 2>, RowShape<512, 2>,
+                            RowShape<512, 4>, RowShape<1024, 3>>(nvec, run_ragged);
+    }
+  } else if constexpr (MODE == 0 && C::VEC == 8) {
+    done = pick_row_shape<RowShape<64, 1>, RowShape<128, 1>, RowShape<256, 1>, RowShape<320, 1>,
                                     RowShape<384, 1>, RowShape<448, 1>, RowShape<512, 1>, RowShape<768, 1>,
                                     RowShape<512, 2>, RowShape<768, 2>, RowShape<512, 4>,
                                     RowShape<1024, 4>>(nvec, run);
   } else if constexpr (MODE == 0) {
-    done = vec_ok && pick_row_shape<RowShape<64, 1>, RowShape<128, 1>, RowShape<256, 1>, RowShape<512, 1>,
+    done = pick_row_shape<RowShape<64, 1>, RowShape<128, 1>, RowShape<256, 1>, RowShape<512, 1>,
                                     RowShape<512, 2>, RowShape<512, 4>, RowShape<1024, 3>,
                                     RowShape<1024, 4>>(nvec, run);
   } else if constexpr (C::VEC == 8) {
-    done = vec_ok && pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<256, 1>, RowShape<192, 2>,
+    done = pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<256, 1>, RowShape<192, 2>,
                                     RowShape<256, 2>, RowShape<256, 3>, RowShape<512, 2>, RowShape<512, 3>,
                                     RowShape<512, 4>, RowShape<1024, 4>>(nvec, run);
   } else {
     // fp32 FP8 rows of 1025-2048 vectors: 512 x 4 against 1024 x 2, per-token
     // 53.7 vs 62.1 us at [4096, 5120], 117.6 vs 127.4 at [8192, 6144] (159.2
     // vs 157.4 at [8192, 8192]); static 147.4 vs 157.5 at [8192, 8192].
-    done = vec_ok && pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<128, 2>, RowShape<256, 2>,
+    done = pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<128, 2>, RowShape<256, 2>,
                                     RowShape<512, 2>, RowShape<512, 4>, RowShape<1024, 3>,
                                     RowShape<1024, 4>>(nvec, run);
   }

@@ -1,0 +1,105 @@
+"""Rows whose length is no multiple of a 16-byte vector, or whose buffers start
+off a 16-byte boundary, through the register-resident row kernels: bit for bit
+against the oracle at the edges of the row shapes (one vector, one element
+either side of a shape's capacity, the widest shapes and past them), with the
+memory around every output untouched.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from custom_cuda_kernals_amd import _native as native
+from oracle import eager, inputs
+from tests._parity import assert_codes_equal, assert_f32_bits_equal, bits_equal
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float32, torch.float16, torch.bfloat16]
+F8 = {"e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}
+# Row capacities of the shapes, in vectors; a row is one element short of one,
+# or one element longer, so its last vector is partial on either side.
+CAPACITIES = [1, 64, 128, 256, 320, 384, 512, 768, 1024, 1536, 2048, 3072, 4096]
+
+
+class Guarded:
+    """A device tensor `offset` elements into a buffer whose other bytes must
+    keep a pattern."""
+
+    def __init__(self, shape, dtype, offset: int) -> None:
+        n = int(np.prod(shape))
+        self.flat = torch.full(((n + offset + 64) * dtype.itemsize,), 0xA5, dtype=torch.uint8, device="cuda")
+        self.lo, self.hi = offset * dtype.itemsize, (n + offset) * dtype.itemsize
+        self.t = self.flat[self.lo:self.hi].view(dtype).view(shape)
+
+    def check(self) -> None:
+        rest = torch.cat([self.flat[:self.lo], self.flat[self.hi:]])
+        assert bool((rest == 0xA5).all()), "written outside the output"
+
+
+def _off(t: torch.Tensor, offset: int) -> torch.Tensor:
+    view = torch.empty(t.numel() + offset, dtype=t.dtype, device="cuda")[offset:].view(t.shape)
+    view.copy_(t.cuda())
+    return view
+
+
+def _lengths(vec: int) -> list[int]:
+    return [c * vec + d for c in CAPACITIES for d in (-1, 1) if c * vec + d >= 1]
+
+
+def _check_norm(x, r, w, static, offset=0):
+    """Plain (static is False), per-token (None) or static-scale RMSNorm."""
+    ro = Guarded(x.shape, x.dtype, offset)
+    xd, rd, wd = _off(x, offset), _off(r, offset), _off(w, offset)
+    if static is False:
+        y = Guarded(x.shape, x.dtype, offset)
+        native.rmsnorm_residual_fwd(xd, rd, wd, y.t, ro.t, 1e-5)
+        y_ref, ro_ref = eager.rmsnorm_residual(x, r, w, 1e-5)
+        assert bits_equal(y.t, y_ref).all()
+        y.check()
+    else:
+        q = Guarded(x.shape, F8["e4m3"], offset)
+        s = torch.empty(x.shape[0], dtype=torch.float32, device="cuda") if static is None else None
+        native.rmsnorm_residual_fp8_fwd(xd, rd, wd, q.t, s, ro.t, 1e-5, "e4m3", static)
+        codes, s_ref, ro_ref, _ = eager.rmsnorm_residual_fp8(x, r, w, 1e-5, "e4m3", static)
+        assert_codes_equal(q.t, codes)
+        if static is None:
+            assert_f32_bits_equal(s, s_ref)
+        q.check()
+    assert bits_equal(ro.t, ro_ref).all()
+    ro.check()
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("static", [False, None, 0.05], ids=["plain", "token", "static"])
+def test_rmsnorm(dtype, static):
+    vec = 16 // dtype.itemsize
+    for cols in _lengths(vec):
+        x, r, w = inputs.rmsnorm_inputs(5, cols, dtype, seed=cols)
+        _check_norm(x, r, w, static, offset=cols % 3)
+    # Whole vectors from an unaligned start, and every remainder after whole vectors.
+    for cols in [256 * vec, *range(600 * vec, 601 * vec)]:
+        x, r, w = inputs.rmsnorm_inputs(3, cols, dtype, seed=cols + 1)
+        _check_norm(x, r, w, static, offset=1)
+
+
+def test_rmsnorm_absent_elements_stay_out_of_the_amax():
+    """Rows whose variance underflows at eps = 0: 1 / sqrt(0) is infinite, so
+    present elements give infinities (a zero element NaN) and an infinite
+    scale; the partial vector's absent elements must not add a NaN."""
+    x = torch.full((3, 1003), 1e-30, dtype=torch.float32).to(torch.bfloat16)
+    x[1, 5] = 0.0
+    x[2] = 1.0
+    r, w = torch.zeros_like(x), torch.ones(1003, dtype=torch.bfloat16)
+    q = torch.empty(x.shape, dtype=F8["e4m3"], device="cuda")
+    s = torch.empty(3, dtype=torch.float32, device="cuda")
+    native.rmsnorm_residual_fp8_fwd(x.cuda(), r.cuda(), w.cuda(), q, s, torch.empty_like(x, device="cuda"), 0.0,
+                                    "e4m3", None)
+    codes, s_ref, _, _ = eager.rmsnorm_residual_fp8(x, r, w, 0.0, "e4m3", None)
+    assert_f32_bits_equal(s, s_ref)
+    assert np.isinf(s_ref.reshape(-1)[0]) and np.isnan(s_ref.reshape(-1)[1])
+    got = q.view(torch.uint8).cpu().numpy()
+    nan = (codes & 0x7F) == 0x7F
+    assert np.array_equal((got & 0x7F) == 0x7F, nan) and np.array_equal(got[~nan], codes[~nan])
