@@ -526,6 +526,15 @@ template <class C>
 __device__ inline uint32_t ragged_offset(uint32_t v, int nwhole, int npart) {
   return v * 16u - (v == (uint32_t)nwhole ? (uint32_t)((C::VEC - npart) * C::kBytes) : 0u);
 }
+// For steps that treat every element alike and write it once per value: the
+// first element of vector v of a ragged row of `cols` elements, the last
+// vector taken whole as the row's last VEC elements. It repeats up to VEC - 1
+// elements of its neighbour, with the same results.
+template <class C>
+__device__ inline uint32_t overlap_first(uint32_t v, uint32_t cols) {
+  const uint32_t e = v * C::VEC;
+  return e < cols - C::VEC ? e : cols - C::VEC;
+}
 // The last npart elements of w moved to the front, zeros after them.
 template <class C>
 __device__ inline u32x4 partial_vector(u32x4 w, int npart) {

@@ -176,7 +176,16 @@ constexpr int kPolQ = kPolSC1 | kPolNT;
 // vectors hold rows of 65536 bf16 / fp16 (32768 fp32) elements in 128 KB.
 // The raw registers are then free after the SiLU, so the next row's loads go
 // out before the amax reduction.
-template <class C, int THREADS, int ITEMS, int FMT, bool TAB, bool STATIC, bool LDSY = false>
+// RAGGED: any row length from VEC elements up and any element-aligned
+// pointers, by vectors from the row's own start (RowAny), the last one
+// overlapping its neighbour (overlap_first): y, the amax and the codes are per
+// element, so the repeated elements change nothing. Bound by HBM like the
+// aligned rows, plus the cache lines that neighbouring rows share: bf16,
+// against the two-pass scalar kernel / aligned rows of the next whole vector,
+// [2048, 5461] 24.3 vs 12.8 us, [12291, 1365] 37.7 vs 19.2 / 17.7, [3072, 5461]
+// 40.5 vs 18.1 / 17.9, [1228, 13653] 50.2 vs 18.9 / 18.0, [585, 28665] 94.5 vs
+// 25.4 / 20.1, [256, 40001] 119.7 vs 14.4; fp32 [3072, 5461] 60.8 vs 26.8.
+template <class C, int THREADS, int ITEMS, int FMT, bool TAB, bool STATIC, bool LDSY = false, bool RAGGED = false>
 __global__ __launch_bounds__(THREADS) void swiglu_fp8_resident(
     const void* __restrict__ gate, const void* __restrict__ up, uint8_t* __restrict__ yq,
     float* __restrict__ scale, float static_scale, int64_t rows, int64_t cols) {
@@ -185,7 +194,16 @@ __global__ __launch_bounds__(THREADS) void swiglu_fp8_resident(
   constexpr int VEC = C::VEC;
   __shared__ uint32_t lds[2 * NW];
   __shared__ __attribute__((aligned(16))) float tab[TAB ? SiluTableBF16::kEntries : 1];
-  const int nvec = (int)(cols / VEC);
+  const int nvec = (int)((cols + (RAGGED ? VEC - 1 : 0)) / VEC);
+  // First element of vector v.
+  auto first = [&](uint32_t v) { return RAGGED ? overlap_first<C>(v, (uint32_t)cols) : v * VEC; };
+  // The same for this thread's item k, formed anew (opaque to the optimiser):
+  // kept from the loads, the offsets took the ragged 1024 x 2 rows past 64 VGPRs.
+  auto first_again = [&](int k) {
+    uint32_t v = threadIdx.x;
+    if constexpr (RAGGED) asm("" : "+v"(v));
+    return first(v + k * THREADS);
+  };
   int parity = 0;
   // A static scale goes to scale[0] when the caller passed a scale word.
   if (STATIC && scale != nullptr && blockIdx.x == 0 && threadIdx.x == 0) scale[0] = static_scale;
@@ -195,14 +213,15 @@ __global__ __launch_bounds__(THREADS) void swiglu_fp8_resident(
   u32x4 graw[ITEMS], uraw[ITEMS];
   auto load = [&](int64_t row) {
     const int64_t off = row * cols * C::kBytes;
-    const RowBuf<false> bg(static_cast<const char*>(gate) + off, row_bytes);
-    const RowBuf<false> bu(static_cast<const char*>(up) + off, row_bytes);
+    using Row = std::conditional_t<RAGGED, RowAny, RowBuf<false>>;
+    const Row bg(static_cast<const char*>(gate) + off, row_bytes);
+    const Row bu(static_cast<const char*>(up) + off, row_bytes);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const uint32_t v = threadIdx.x + k * THREADS;
       if (v < (uint32_t)nvec) {
-        graw[k] = bg.ld16(v * 16u);
-        uraw[k] = bu.ld16(v * 16u);
+        graw[k] = bg.ld16(first(v) * C::kBytes);
+        uraw[k] = bu.ld16(first(v) * C::kBytes);
       }
     }
   };
@@ -273,7 +292,7 @@ __global__ __launch_bounds__(THREADS) void swiglu_fp8_resident(
     }
     const float r = 1.0f / s;
     const bool fast = fast_path_ok<FMT>(s, r, amax);
-    const RowBuf<kRsrcQ, kPolQ> bq(yq + row * cols, (uint32_t)cols);
+    const std::conditional_t<RAGGED, RowAny, RowBuf<kRsrcQ, kPolQ>> bq(yq + row * cols, (uint32_t)cols);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const uint32_t v = threadIdx.x + k * THREADS;
@@ -287,9 +306,9 @@ __global__ __launch_bounds__(THREADS) void swiglu_fp8_resident(
           quant_exact<FMT, VEC>(yk, s, wq);
         }
         if constexpr (VEC == 8) {
-          bq.st8((u32x2){wq[0], wq[1]}, v * 8u);
+          bq.st8((u32x2){wq[0], wq[1]}, first_again(k));
         } else {
-          bq.st4(wq[0], v * 4u);
+          bq.st4(wq[0], first_again(k));
         }
       }
     }
@@ -299,8 +318,8 @@ __global__ __launch_bounds__(THREADS) void swiglu_fp8_resident(
   }
 }
 
-// Per-token FP8 variant, any alignment / row length: y is recomputed in the
-// second pass.
+// Per-token FP8 rows that no register-resident shape holds (under one vector,
+// or past the widest): y is recomputed in the second pass.
 template <class C, int FMT>
 __global__ __launch_bounds__(256) void swiglu_fp8_generic(
     const void* __restrict__ gate, const void* __restrict__ up, uint8_t* __restrict__ yq,
@@ -329,15 +348,17 @@ __global__ __launch_bounds__(256) void swiglu_fp8_generic(
 }
 
 // Register-resident rows: one workgroup per row for the row-length buckets
-// below; false (nothing launched) when no bucket holds the row or the
-// buffers are not aligned for 16-byte access. STATIC rows are used only with
-// the bf16 table and 768 or more threads per row.
-template <class C, int FMT, bool STATIC>
+// below; false (nothing launched) when no bucket holds the row. STATIC rows
+// are used only with the bf16 table and 768 or more threads per row, and only
+// for whole vectors at 16-byte alignment; RAGGED ones are the rest of the
+// per-token rows.
+template <class C, int FMT, bool STATIC, bool RAGGED = false>
 bool launch_swiglu_fp8_rows(const void* gate, const void* up, uint8_t* yq, float* scale, float static_scale,
                             int64_t rows, int64_t cols, hipStream_t st) {
-  const bool vec_ok = (cols % C::VEC == 0) && host_aligned(gate, 16) && host_aligned(up, 16) &&
-                      host_aligned(yq, C::VEC);
-  const int64_t nvec = cols / C::VEC;
+  const bool ok = RAGGED ? cols >= C::VEC
+                         : (cols % C::VEC == 0) && host_aligned(gate, 16) && host_aligned(up, 16) &&
+                               host_aligned(yq, C::VEC);
+  const int64_t nvec = (cols + C::VEC - 1) / C::VEC;
   const unsigned g = row_grid(rows);
   bool launched = false;
   auto run = [&](auto shape) {
@@ -347,7 +368,7 @@ bool launch_swiglu_fp8_rows(const void* gate, const void* up, uint8_t* yq, float
     constexpr bool kTab = std::is_same_v<C, CodecBF16> && S::kThreads * S::kItems >= 1152;
     auto go = [&](auto ldsy) {
       constexpr bool kLdsY = decltype(ldsy)::value;
-      constexpr auto kernel = swiglu_fp8_resident<C, S::kThreads, S::kItems, FMT, kTab, STATIC, kLdsY>;
+      constexpr auto kernel = swiglu_fp8_resident<C, S::kThreads, S::kItems, FMT, kTab, STATIC, kLdsY, RAGGED>;
       // bf16 rows with y in LDS run on a grid of the workgroups the device
       // holds at once, each looping over rows: one SiLU table fill per
       // workgroup instead of per row, no idle CU between rows, and the next
@@ -362,7 +383,8 @@ bool launch_swiglu_fp8_rows(const void* gate, const void* up, uint8_t* yq, float
       launched = true;
     };
     if constexpr (S::kItems > 4) {
-      if constexpr (!STATIC) go(std::true_type{});
+      // (Ragged rows of 1024 x 8 would spill registers.)
+      if constexpr (!STATIC && !(RAGGED && S::kItems > 6)) go(std::true_type{});
     } else if constexpr (kTab && !STATIC && S::kThreads == 1024 && S::kItems >= 3) {
       // bf16 per-token rows of three and four vectors per thread park y in
       // LDS (48 / 64 KB) on the looping grid too, where the grid loops (more
@@ -375,7 +397,7 @@ bool launch_swiglu_fp8_rows(const void* gate, const void* up, uint8_t* yq, float
       // 168.5, 31744 236.0 / 231.3, 32768 238.0 / 230.5 (24576 tied); so
       // did a grid that does not loop (256 rows of 28672: 9.5 / 9.0) and
       // fp16 and fp32 rows (1-4 %).
-      constexpr auto kParked = swiglu_fp8_resident<C, S::kThreads, S::kItems, FMT, kTab, STATIC, true>;
+      constexpr auto kParked = swiglu_fp8_resident<C, S::kThreads, S::kItems, FMT, kTab, STATIC, true, RAGGED>;
       const int64_t last = nvec - (int64_t)(S::kItems - 1) * S::kThreads;  // threads holding a last vector
       const int64_t resident = resident_groups<kParked>(S::kThreads);
       if (4 * last <= 3 * S::kThreads && resident > 0 && resident < rows) {
@@ -400,7 +422,7 @@ bool launch_swiglu_fp8_rows(const void* gate, const void* up, uint8_t* yq, float
   // 166.3 against 170.7; 256 x 3 at 5632, 39.5 against 41.0; 512 x 2 at 8192
   // (57.5; 62.8 for 384 x 3). fp32 rows keep two vectors per thread up to
   // 1024 x 2. Wider rows of every type take 1024 x 6 or 8 with y in LDS.
-  if (vec_ok) {
+  if (ok) {
     if constexpr (std::is_same_v<C, CodecBF16>) {
       if (nvec > 896 && nvec <= 1152) {
         run(RowShape<384, 3>{});
@@ -424,7 +446,8 @@ bool launch_swiglu_fp8_rows(const void* gate, const void* up, uint8_t* yq, float
 template <class C, int FMT>
 int32_t launch_swiglu_fp8_token(const void* gate, const void* up, uint8_t* yq, float* scale, int64_t rows,
                                 int64_t cols, hipStream_t st) {
-  if (!launch_swiglu_fp8_rows<C, FMT, false>(gate, up, yq, scale, 0.0f, rows, cols, st)) {
+  if (!launch_swiglu_fp8_rows<C, FMT, false>(gate, up, yq, scale, 0.0f, rows, cols, st) &&
+      !launch_swiglu_fp8_rows<C, FMT, false, true>(gate, up, yq, scale, 0.0f, rows, cols, st)) {
     swiglu_fp8_generic<C, FMT><<<row_grid(rows), 256, 0, st>>>(gate, up, yq, scale, rows, cols);
   }
   return launch_status();

@@ -103,3 +103,24 @@ def test_rmsnorm_absent_elements_stay_out_of_the_amax():
     got = q.view(torch.uint8).cpu().numpy()
     nan = (codes & 0x7F) == 0x7F
     assert np.array_equal((got & 0x7F) == 0x7F, nan) and np.array_equal(got[~nan], codes[~nan])
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).split(".")[-1])
+def test_swiglu_fp8_token(dtype):
+    """Per-token SwiGLU + FP8: the last vector overlaps its neighbour, on every
+    shape, on parked rows (more rows than resident workgroups) and past the
+    widest shape."""
+    vec = 16 // dtype.itemsize
+    shapes = [(5, c) for c in _lengths(vec) + [256 * vec, 6144 * vec - 1, 6144 * vec + 1]]
+    if dtype == torch.bfloat16:
+        shapes += [(600, 17001), (300, 28665)]
+    for rows, cols in shapes:
+        g, u = inputs.swiglu_inputs(rows, cols, dtype, seed=cols)
+        offset = cols % 3
+        q = Guarded(g.shape, F8["e5m2"], offset)
+        s = torch.empty(rows, dtype=torch.float32, device="cuda")
+        native.swiglu_fp8_fwd(_off(g, offset), _off(u, offset), q.t, s, "e5m2", None)
+        codes, s_ref, _ = eager.swiglu_fp8(g, u, "e5m2", None)
+        assert_codes_equal(q.t, codes)
+        assert_f32_bits_equal(s, s_ref)
+        q.check()
