@@ -49,6 +49,26 @@ __device__ inline void quant_vec(const u32x4& raw, float s, float r, bool fast, 
   store_codes<C::VEC>(q, off, w);
 }
 
+// The same to any address, the first `part` codes only if part != 0.
+template <class C, int FMT>
+__device__ inline void quant_vec_any(const u32x4& raw, float s, float r, bool fast, uint8_t* q, int part) {
+  float f[C::VEC];
+  C::unpack(raw, f);
+  uint32_t w[C::VEC / 4];
+  if (fast) {
+    quant_fast<FMT, C::VEC>(f, s, r, w);
+  } else {
+    quant_exact<FMT, C::VEC>(f, s, w);
+  }
+  if (part) {
+    store_codes_partial<C::VEC>(w, part, q);
+  } else if constexpr (C::VEC == 8) {
+    RowAny(q, 0).st8((u32x2){w[0], w[1]}, 0u);
+  } else {
+    RowAny(q, 0).st4(w[0], 0u);
+  }
+}
+
 template <int FMT>
 __device__ inline uint8_t quant1(float v, float s, float r, bool fast) {
   if (fast) {
@@ -72,16 +92,30 @@ constexpr int kPolTokenQ = kBufStorePolicy;
 // ---------------------------------------------------------------------------
 // Token granularity, register-resident rows: one workgroup per row, each
 // thread holds ITEMS 16-byte vectors. Requires cols % VEC == 0 and 16-byte
-// aligned x, VEC-aligned q.
+// aligned x, VEC-aligned q, or RAGGED: any row length from VEC elements up and
+// any element-aligned pointers, by vectors from the row's own start (RowAny),
+// the last one overlapping its neighbour (overlap_first; the max and the codes
+// are per element).
 // ---------------------------------------------------------------------------
-template <class C, int FMT, int THREADS, int ITEMS>
+template <class C, int FMT, int THREADS, int ITEMS, bool RAGGED = false>
 __global__ __launch_bounds__(THREADS) void fp8_token_resident(const void* __restrict__ x,
                                                               uint8_t* __restrict__ q,
                                                               float* __restrict__ scale,
                                                               int64_t rows, int64_t cols) {
   constexpr int NW = THREADS / 64;
   __shared__ uint32_t lds[2 * NW];
-  const int nvec = (int)(cols / C::VEC);
+  const int nvec = (int)((cols + (RAGGED ? C::VEC - 1 : 0)) / C::VEC);
+  // First element of this thread's item k.
+  auto first = [&](int k) {
+    const uint32_t v = threadIdx.x + k * THREADS;
+    return RAGGED ? overlap_first<C>(v, (uint32_t)cols) : v * C::VEC;
+  };
+  // The same, formed anew (opaque to the optimiser) instead of kept in registers from the loads.
+  auto first_again = [&](int k) {
+    uint32_t t = threadIdx.x;
+    if constexpr (RAGGED) asm("" : "+v"(t));
+    return RAGGED ? overlap_first<C>(t + k * THREADS, (uint32_t)cols) : (t + k * THREADS) * C::VEC;
+  };
   int parity = 0;
   // Buffer-resource row access (no per-lane 64-bit addressing): 6.6 vs 6.8 us
   // at [2048, 4096] bf16 on MI355X.
@@ -96,11 +130,12 @@ __global__ __launch_bounds__(THREADS) void fp8_token_resident(const void* __rest
   constexpr bool kAhead = ITEMS <= 4;
   u32x4 nxt[ITEMS];
   auto issue = [&](int64_t row) {
-    const RowBuf<true> bx(static_cast<const char*>(x) + row * cols * C::kBytes, row_bytes);
+    const std::conditional_t<RAGGED, RowAny, RowBuf<true>> bx(static_cast<const char*>(x) + row * cols * C::kBytes,
+                                                              row_bytes);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const uint32_t v = threadIdx.x + k * THREADS;
-      if (v < (uint32_t)nvec) nxt[k] = bx.ld16(v * 16u);
+      if (v < (uint32_t)nvec) nxt[k] = bx.ld16(first(k) * C::kBytes);
     }
   };
   if ((int64_t)blockIdx.x < rows) issue(blockIdx.x);
@@ -122,7 +157,7 @@ __global__ __launch_bounds__(THREADS) void fp8_token_resident(const void* __rest
     const float r = 1.0f / s;
     if (threadIdx.x == 0) scale[row] = s;
     const bool fast = fast_path_ok<FMT>(s, r, amax);
-    const RowBuf<true, kPolTokenQ> bq(q + row * cols, (uint32_t)cols);
+    const std::conditional_t<RAGGED, RowAny, RowBuf<true, kPolTokenQ>> bq(q + row * cols, (uint32_t)cols);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const uint32_t v = threadIdx.x + k * THREADS;
@@ -136,9 +171,9 @@ __global__ __launch_bounds__(THREADS) void fp8_token_resident(const void* __rest
           quant_exact<FMT, C::VEC>(f, s, w);
         }
         if constexpr (C::VEC == 8) {
-          bq.st8((u32x2){w[0], w[1]}, v * 8u);
+          bq.st8((u32x2){w[0], w[1]}, first_again(k));
         } else {
-          bq.st4(w[0], v * 4u);
+          bq.st4(w[0], first_again(k));
         }
       }
     }
@@ -146,8 +181,9 @@ __global__ __launch_bounds__(THREADS) void fp8_token_resident(const void* __rest
   }
 }
 
-// Token granularity, any alignment / row length: scalar loads, the row is
-// read twice (the second read is served by L2 for rows up to a few MB).
+// Token granularity, rows that no register-resident shape holds (under one
+// vector, or past the widest): scalar loads, the row is read twice (the second
+// read is served by L2 for rows up to a few MB).
 template <class C, int FMT>
 __global__ __launch_bounds__(256) void fp8_token_generic(const void* __restrict__ x,
                                                          uint8_t* __restrict__ q,
@@ -185,7 +221,12 @@ constexpr int kTile = 128;
 constexpr int64_t kBlockPairMinTiles = 16384;
 constexpr int64_t kBlockSplitMaxTiles = 1024;  // one round of 512-thread workgroups (4 per CU)
 
-template <class C, int FMT, int THREADS, bool RSRC, int TW, bool SPLIT = false>
+//
+// RAGGED: any n from VEC up and any element-aligned pointers, by unaligned
+// vectors from each row's own start; a row's partial last vector is loaded as
+// the row's last VEC elements and moved to the front (partial_vector: the
+// elements dropped may belong to the tile on the left).
+template <class C, int FMT, int THREADS, bool RSRC, int TW, bool SPLIT = false, bool RAGGED = false>
 __global__ __launch_bounds__(THREADS * TW) void fp8_block_resident(const void* __restrict__ x,
                                                                    uint8_t* __restrict__ q,
                                                                    float* __restrict__ scale, int64_t m,
@@ -211,6 +252,7 @@ __global__ __launch_bounds__(THREADS * TW) void fp8_block_resident(const void* _
                         (uint32_t)(left < 0x7fffffff ? left : 0x7fffffff));
   u32x4 raw[ITEMS];
   uint32_t acc = 0;
+  const int part = RAGGED && col_ok && n - col < C::VEC ? (int)(n - col) : 0;  // elements of a partial vector
   // Loads without branches: an element outside the matrix reads the
   // workgroup's first element (always inside it) and is replaced by zeros.
   // Loading under a branch instead made the compiler copy the whole of raw[]
@@ -222,7 +264,12 @@ __global__ __launch_bounds__(THREADS * TW) void fp8_block_resident(const void* _
   for (int k = 0; k < ITEMS; ++k) {
     const int64_t row = row0 + k * RPP;
     const bool ok = col_ok && row < m;
-    if constexpr (RSRC) {
+    if constexpr (RAGGED) {
+      // (The matrix's first vector stands in for the absent ones: m * n >= VEC.)
+      const int64_t e = row * n + (part ? n - C::VEC : col);
+      raw[k] = RowAny(static_cast<const char*>(x) + (ok ? e : 0) * C::kBytes, 0).ld16(0u);
+      continue;
+    } else if constexpr (RSRC) {
       const uint32_t off = (uint32_t)(((int64_t)(rr + k * RPP) * n + tile * kTile + cv * C::VEC) * C::kBytes);
       raw[k] = bx.ld16(ok ? off : 0u);
     } else {
@@ -231,6 +278,13 @@ __global__ __launch_bounds__(THREADS * TW) void fp8_block_resident(const void* _
     }
     raw[k] = ok ? raw[k] : zero;
     if constexpr (!SPLIT) acc = C::absmax_vec(raw[k], acc);
+  }
+  if constexpr (RAGGED) {
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+      if (part) raw[k] = partial_vector<C>(raw[k], part);
+      raw[k] = col_ok && row0 + k * RPP < m ? raw[k] : zero;
+    }
   }
   // SPLIT: every load is issued before the first max, instead of each max
   // waiting on its own load (see the launcher for when each pays).
@@ -257,7 +311,13 @@ __global__ __launch_bounds__(THREADS * TW) void fp8_block_resident(const void* _
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
     const int64_t row = row0 + k * RPP;
-    if (col_ok && row < m) quant_vec<C, FMT>(raw[k], s, r, fast, q, row * n + col);
+    if (col_ok && row < m) {
+      if constexpr (RAGGED) {
+        quant_vec_any<C, FMT>(raw[k], s, r, fast, q + row * n + col, part);
+      } else {
+        quant_vec<C, FMT>(raw[k], s, r, fast, q, row * n + col);
+      }
+    }
   }
 }
 
@@ -546,12 +606,22 @@ template <class C, int FMT>
 int32_t launch_token(const void* x, uint8_t* q, float* scale, int64_t m, int64_t n,
                      hipStream_t st) {
   const bool vec_ok = (n % C::VEC == 0) && host_aligned(x, 16) && host_aligned(q, C::VEC);
-  const int64_t nvec = n / C::VEC;
+  const int64_t nvec = (n + C::VEC - 1) / C::VEC;
   const unsigned g = row_grid(m);
   auto run = [&](auto shape) {
     using S = decltype(shape);
-    fp8_token_resident<C, FMT, S::kThreads, S::kItems><<<g, S::kThreads, 0, st>>>(x, q, scale, m, n);
+    if (vec_ok) {
+      fp8_token_resident<C, FMT, S::kThreads, S::kItems><<<g, S::kThreads, 0, st>>>(x, q, scale, m, n);
+    } else {
+      fp8_token_resident<C, FMT, S::kThreads, S::kItems, true><<<g, S::kThreads, 0, st>>>(x, q, scale, m, n);
+    }
   };
+  // Rows of at least one vector. The ragged ones against the scalar kernel
+  // below, which reads x twice by elements / against aligned rows of the next
+  // whole vector, bf16 on MI355X: [8184, 4100] 46.9 vs 17.8 / 18.0 us, [16384, 517]
+  // 20.8 vs 8.1 / 8.0, [6144, 5461] 48.6 vs 20.2 / 17.7, [1170, 28665] 79.5 vs 23.0 /
+  // 17.9, [1000, 40001] 126.6 vs 27.7; fp32 [3049, 11005] 82.5 vs 29.7.
+  const bool fits = n >= C::VEC;
   // 16-byte rows (f16 / bf16) from a sweep over THREADS 64..1024 x ITEMS
   // 1..4 on MI355X at 8192 bf16 rows of 2048..28672 elements (graph-replayed,
   // 2 GiB rotation): three or four vectors per thread from 2560 elements on,
@@ -562,12 +632,12 @@ int32_t launch_token(const void* x, uint8_t* q, float* scale, int64_t m, int64_t
   // against 28.8 us at [8192, 4096] for 256 x 4).
   bool done = false;
   if constexpr (C::VEC == 8) {
-    done = vec_ok && pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<128, 2>, RowShape<128, 3>,
+    done = fits && pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<128, 2>, RowShape<128, 3>,
                                     RowShape<256, 2>, RowShape<256, 3>, RowShape<256, 4>, RowShape<512, 3>,
                                     RowShape<512, 4>, RowShape<1024, 3>, RowShape<1024, 4>, RowShape<1024, 6>,
                                     RowShape<1024, 8>>(nvec, run);
   } else {
-    done = vec_ok && pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<128, 2>, RowShape<256, 2>,
+    done = fits && pick_row_shape<RowShape<64, 1>, RowShape<64, 2>, RowShape<128, 2>, RowShape<256, 2>,
                                     RowShape<512, 2>, RowShape<1024, 2>, RowShape<1024, 4>,
                                     RowShape<1024, 8>>(nvec, run);
   }
@@ -935,6 +1005,13 @@ extern "C" int32_t launch_fp8_quant_block_fwd(const void* x, uint8_t* x_fp8, flo
         fp8_block_resident<C, FMT, 512, true, 1><<<grid, 512, 0, st>>>(x, x_fp8, scale, m, n);
       } else if (vec_ok) {
         fp8_block_resident<C, FMT, 512, false, 1><<<grid, 512, 0, st>>>(x, x_fp8, scale, m, n);
+      } else if (n >= C::VEC) {
+        // Ragged rows, against the scalar kernel / aligned rows of the next whole
+        // vector, bf16 on MI355X: [8184, 4100] 88.6 vs 31.8 / 30.9 us, [6144, 5461]
+        // 102.5 vs 32.0 / 30.9, [257, 513] fp16 37.2 vs 7.4, fp32 [3049, 11005]
+        // 127.1 vs 43.9. Bound by the cache lines that neighbouring tiles share
+        // (aligned rows of 4096 take 18 us).
+        fp8_block_resident<C, FMT, 512, false, 1, true, true><<<grid, 512, 0, st>>>(x, x_fp8, scale, m, n);
       } else {
         fp8_block_generic<C, FMT><<<grid, 256, 0, st>>>(x, x_fp8, scale, m, n);
       }

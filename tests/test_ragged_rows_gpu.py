@@ -13,6 +13,7 @@ import torch
 
 from custom_cuda_kernals_amd import _native as native
 from oracle import eager, inputs
+from oracle import fp8 as ofp8
 from tests._parity import assert_codes_equal, assert_f32_bits_equal, bits_equal
 
 pytestmark = pytest.mark.gpu
@@ -121,6 +122,41 @@ def test_swiglu_fp8_token(dtype):
         s = torch.empty(rows, dtype=torch.float32, device="cuda")
         native.swiglu_fp8_fwd(_off(g, offset), _off(u, offset), q.t, s, "e5m2", None)
         codes, s_ref, _ = eager.swiglu_fp8(g, u, "e5m2", None)
+        assert_codes_equal(q.t, codes)
+        assert_f32_bits_equal(s, s_ref)
+        q.check()
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).split(".")[-1])
+def test_fp8_token(dtype):
+    vec = 16 // dtype.itemsize
+    for cols in _lengths(vec) + [256 * vec, 6144 * vec - 1, 8192 * vec - 1, 8192 * vec + 1]:
+        x = inputs.randn((5, cols), dtype, seed=cols)
+        q = Guarded(x.shape, F8["e4m3"], cols % 3)
+        s = torch.empty(5, dtype=torch.float32, device="cuda")
+        native.fp8_quant_token_fwd(_off(x, cols % 3), q.t, s, "e4m3")
+        codes, s_ref = ofp8.quant_token(x.float().numpy(), "e4m3")
+        assert_codes_equal(q.t, codes)
+        assert_f32_bits_equal(s, s_ref)
+        q.check()
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).split(".")[-1])
+def test_fp8_block(dtype):
+    """128 x 128 tiles of ragged rows: the partial vector first in its tile
+    (its loaded neighbours belong to the tile on the left), every remainder,
+    one row, and matrices of barely one vector."""
+    vec = 16 // dtype.itemsize
+    shapes = [(1, vec), (1, vec + 1), (129, vec - 1), (127, 128 + 1), (257, 513), (130, 256 - 1), (128, 128)]
+    shapes += [(131, 384 + d) for d in range(1, vec)]
+    for m, n in shapes:
+        x = inputs.randn((m, n), dtype, seed=m + n)
+        x[:, n // 2:] *= 1000.0  # neighbouring tiles of other levels
+        offset = 1 + n % 2
+        q = Guarded(x.shape, F8["e4m3"], offset)
+        s = torch.empty((m + 127) // 128, (n + 127) // 128, dtype=torch.float32, device="cuda")
+        native.fp8_quant_block_fwd(_off(x, offset), q.t, s, "e4m3")
+        codes, s_ref = ofp8.quant_block(x.float().numpy(), "e4m3")
         assert_codes_equal(q.t, codes)
         assert_f32_bits_equal(s, s_ref)
         q.check()
