@@ -15,7 +15,9 @@
 // Workgroups are 256 threads, or, for one token of more heads than 256
 // threads cover at once, a thread per (head, chunk) of the token; while the
 // grid fits one round of resident workgroups, a thread per (head, chunk)
-// with the token's cos/sin row staged in LDS.
+// with the token's cos/sin row staged in LDS. Any other number of chunks, and
+// inputs small enough to be on chip still, take rope_heads: a thread per
+// (head, chunk) for any of both counts.
 // All accesses are 16 bytes; a wave covers whole 128-byte cache lines.
 #include "launch.hpp"
 
@@ -87,7 +89,8 @@ __global__ __launch_bounds__(NT) void rope_tokens(const void* q, const void* k,
   }
 }
 
-// Any head_dim / alignment: one thread per (token, head, pair).
+// Halves that are no whole vectors, and unaligned buffers: one thread per
+// (token, head, pair).
 template <class C>
 __global__ __launch_bounds__(256) void rope_scalar(const void* q, const void* k,
                                                    const float* __restrict__ cos_t,
@@ -112,6 +115,73 @@ __global__ __launch_bounds__(256) void rope_scalar(const void* q, const void* k,
     const float x1 = C::load1(src, e0), x2 = C::load1(src, e0 + half);
     C::store1(dst, e0, x1 * c - x2 * sn);
     C::store1(dst, e0 + half, x2 * c + x1 * sn);
+  }
+}
+
+// One token per workgroup, a thread per (head, chunk) of it, for any number of
+// chunks: t = h * chunks + c is split by `magic` = ceil(2^32 / chunks), exact
+// for t < 65536 (the launcher's bound). Threads loop when the token has more
+// than 1024 of them.
+//
+// The accesses come in two more policies than the streaming ones above:
+//   ONCHIP: cached loads, for inputs that the Infinity Cache still holds from
+//     whatever wrote them (see the launcher);
+//   SPLIT:  cached loads and stores, for halves that are not whole 64-byte
+//     pieces: the two halves of a head, and neighbouring heads, share cache
+//     lines, which nontemporal loads fetch twice and write-through stores
+//     write twice.
+enum RopePolicy : int { kRopeStream, kRopeOnChip, kRopeSplit };
+
+template <class C, RopePolicy P>
+__global__ __launch_bounds__(1024) void rope_heads(const void* q, const void* k, const float* __restrict__ cos_t,
+                                                   const float* __restrict__ sin_t, void* q_out, void* k_out,
+                                                   int64_t tokens, int64_t seq_len, int hq, int hkv, int chunks,
+                                                   uint32_t magic) {
+  constexpr int VEC = C::VEC;
+  constexpr int kStore = P == kRopeSplit ? 0 : kPolSC1 | kPolNT;
+  const uint32_t half_bytes = (uint32_t)chunks * 16u;
+  const uint32_t n = (uint32_t)(hq + hkv) * (uint32_t)chunks;
+  const uint32_t q_bytes = (uint32_t)hq * 2u * half_bytes, k_bytes = (uint32_t)hkv * 2u * half_bytes;
+  for (int64_t tok = blockIdx.x; tok < tokens; tok += gridDim.x) {
+    const int64_t s = tokens <= INT32_MAX ? (int64_t)((uint32_t)tok % (uint32_t)seq_len) : tok % seq_len;
+    const float4* ct = reinterpret_cast<const float4*>(cos_t + s * chunks * VEC);
+    const float4* st = reinterpret_cast<const float4*>(sin_t + s * chunks * VEC);
+    const char* qs = static_cast<const char*>(q) + tok * q_bytes;
+    const char* ks = static_cast<const char*>(k) + tok * k_bytes;
+    const RowBuf<true, kStore> qo(static_cast<char*>(q_out) + tok * q_bytes, q_bytes);
+    const RowBuf<true, kStore> ko(static_cast<char*>(k_out) + tok * k_bytes, k_bytes);
+    for (uint32_t t = threadIdx.x; t < n; t += blockDim.x) {
+      const uint32_t h = __umulhi(t, magic), c = t - h * (uint32_t)chunks;
+      const bool isq = h < (uint32_t)hq;
+      const uint32_t off = (isq ? h : h - (uint32_t)hq) * 2u * half_bytes + c * 16u;
+      const char* src = (isq ? qs : ks) + off;
+      const u32x4* p1 = reinterpret_cast<const u32x4*>(src);
+      const u32x4* p2 = reinterpret_cast<const u32x4*>(src + half_bytes);
+      const u32x4 ra = P == kRopeStream ? ld_stream(p1) : *p1;
+      const u32x4 rb = P == kRopeStream ? ld_stream(p2) : *p2;
+      float cs[VEC], sn[VEC];
+#pragma unroll
+      for (int i = 0; i < VEC / 4; ++i) {
+        const float4 a = ct[c * (VEC / 4) + i], b = st[c * (VEC / 4) + i];
+        cs[4 * i] = a.x; cs[4 * i + 1] = a.y; cs[4 * i + 2] = a.z; cs[4 * i + 3] = a.w;
+        sn[4 * i] = b.x; sn[4 * i + 1] = b.y; sn[4 * i + 2] = b.z; sn[4 * i + 3] = b.w;
+      }
+      float x1[VEC], x2[VEC], o1[VEC], o2[VEC];
+      C::unpack(ra, x1);
+      C::unpack(rb, x2);
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        o1[i] = x1[i] * cs[i] - x2[i] * sn[i];
+        o2[i] = x2[i] * cs[i] + x1[i] * sn[i];
+      }
+      if (isq) {
+        qo.st16(C::pack(o1), off);
+        qo.st16(C::pack(o2), off + half_bytes);
+      } else {
+        ko.st16(C::pack(o1), off);
+        ko.st16(C::pack(o2), off + half_bytes);
+      }
+    }
   }
 }
 
@@ -186,11 +256,11 @@ __global__ __launch_bounds__(NT) void rope_heads_staged(const void* q, const voi
 // holds at once the tables are staged in LDS (rope_heads_staged): 3.51 vs
 // 3.95 us at 512 tokens of 32 / 8 heads of 128 bf16, 5.13 vs 5.61 at 1024;
 // with more tokens the per-token barrier lost (15.75 vs 15.29 us at 4096,
-// 105.4 vs 103.2 at config 4). With min_rounds > 0, not when the tokens fill
-// more than one but fewer than min_rounds rounds. false (nothing launched)
-// otherwise.
+// 105.4 vs 103.2 at config 4). Beyond it, not with staged_only, nor, with
+// min_rounds > 0, when the tokens fill fewer than min_rounds rounds. false
+// (nothing launched) otherwise.
 template <class C, int CHUNKS, int... WS>
-bool launch_rope_per_head(int waves, int min_rounds, std::integer_sequence<int, WS...>, const void* q,
+bool launch_rope_per_head(int waves, int min_rounds, bool staged_only, std::integer_sequence<int, WS...>, const void* q,
                           const void* k, const float* ct, const float* sn, void* q_out, void* k_out,
                           int64_t tokens, int64_t seq_len, int hq, int hkv, int d, hipStream_t st) {
   const unsigned grid = flat_grid(tokens, 1, kMaxRowGroups);
@@ -202,6 +272,7 @@ bool launch_rope_per_head(int waves, int min_rounds, std::integer_sequence<int, 
       staged<<<grid, 64 * W, 0, st>>>(q, k, ct, sn, q_out, k_out, tokens, seq_len, hq, hkv, d);
       return true;
     }
+    if (staged_only) return false;
     constexpr auto kernel = rope_tokens<C, CHUNKS, 1, 64 * W>;
     if (min_rounds > 0) {
       const int64_t resident = resident_groups<kernel>(64 * W);
@@ -284,11 +355,36 @@ extern "C" int32_t launch_rope_fwd(const void* q, const void* k, const void* cos
     // 5.16 vs 5.79 at 512) and more (103.9 vs 108.4 us at 16384) do not.
     const int heads = hq + hkv;
     const int waves = chunks > 0 ? (heads * chunks + 63) / 64 : 0;
+    // rope_heads, for the chunk counts no kernel above is built for and for
+    // inputs that fit the Infinity Cache (kRopeOnChipBytes). Measured on MI355X
+    // through the Python API, rotating over three sets of buffers (and, after the
+    // slash, over 2 GB of them, which no cache holds): halves of 96 and 80 bytes,
+    // SPLIT against the scalar kernel, fp16 32 / 32 heads of 96 at [2, 2048] 16.4
+    // vs 39.9 us (101 MB; / 22.3), bf16 32 / 8 heads of 80 at [1, 8192] 21.4, with
+    // streaming accesses instead 33.6 and 39.1. Whole 64-byte pieces, ONCHIP
+    // against the streaming kernels: bf16 32 / 8 heads of 128 at [1, 2048] 7.6 vs
+    // 8.4 (/ 9.5 vs 9.1), [1, 4096] 13.2 vs 15.3 (/ 16.4 vs 15.6); fp32 [1, 2048] 13.3
+    // vs 15.3; 16 / 16 heads of 64 at [1, 8192] 11.5 vs 16.5 (/ 16.8 vs 17.0). q and k
+    // come from the projections just before, so the first figure counts while the
+    // cache holds them; the gain fades towards its size (84 MB of input: 26.4 vs 27.9 /
+    // 29.6 vs 27.9, 16 / 4 heads of 256 28.2 vs 28.0; 151 MB loses, 50.2 vs 48.3), so
+    // the line is at a quarter of the 256 MB.
+    constexpr int64_t kRopeOnChipBytes = 64ll << 20;
+    const bool on_chip = tokens * (int64_t)heads * d * C::kBytes <= kRopeOnChipBytes;
+    auto run_heads = [&](auto policy) {
+      const int64_t n = (int64_t)heads * chunks;
+      const int nt = n < 1024 ? (int)((n + 63) / 64 * 64) : 1024;
+      const uint32_t magic = (uint32_t)(((uint64_t(1) << 32) + chunks - 1) / chunks);
+      rope_heads<C, (RopePolicy)decltype(policy)::value><<<flat_grid(tokens, 1, kMaxRowGroups), nt, 0, st>>>(
+          q, k, ct, sn, q_out, k_out, tokens, seq_len, hq, hkv, chunks, magic);
+    };
+    // (chunks == 1 has no 32-bit magic and, like 2, packs many tokens into a workgroup.)
+    const bool heads_ok = chunks > 2 && (int64_t)heads * chunks <= 65536;
     using Waves = std::integer_sequence<int, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>;
     if ((chunks == 8 || chunks == 16) && heads * chunks > 256 && waves <= 16 &&
-        (chunks == 8 ? launch_rope_per_head<C, 8>(waves, 0, Waves{}, q, k, ct, sn, q_out, k_out, tokens, seq_len,
+        (chunks == 8 ? launch_rope_per_head<C, 8>(waves, 0, on_chip, Waves{}, q, k, ct, sn, q_out, k_out, tokens, seq_len,
                                                   hq, hkv, d, st)
-                     : launch_rope_per_head<C, 16>(waves, 4, Waves{}, q, k, ct, sn, q_out, k_out, tokens, seq_len,
+                     : launch_rope_per_head<C, 16>(waves, 4, on_chip, Waves{}, q, k, ct, sn, q_out, k_out, tokens, seq_len,
                                                    hq, hkv, d, st))) {
     } else if (heads * chunks <= 256 &&
                ((chunks == 8 && launch_rope_staged_small<C, 8>(waves, std::integer_sequence<int, 1, 2, 3, 4>{}, q, k,
@@ -298,6 +394,10 @@ extern "C" int32_t launch_rope_fwd(const void* q, const void* k, const void* cos
                 (chunks == 16 && launch_rope_staged_small<C, 16>(waves, std::integer_sequence<int, 1, 2, 3, 4>{}, q,
                                                                   k, ct, sn, q_out, k_out, tokens, seq_len, hq, hkv, d,
                                                                   st)))) {
+    } else if (heads_ok && chunks % 4 != 0) {
+      run_heads(IntC<kRopeSplit>{});
+    } else if (heads_ok && on_chip) {
+      run_heads(IntC<kRopeOnChip>{});
     } else if (chunks == 8) {
       // Tokens of at most 32 heads (and more than 128): with at most 6
       // workgroups per CU (8 fit) this 256-thread shape measured 102.0 vs
@@ -317,6 +417,8 @@ extern "C" int32_t launch_rope_fwd(const void* q, const void* k, const void* cos
       CCK_ROPE(1, 32, 0);
     } else if (chunks == 32) {
       CCK_ROPE(32, 1, 0);
+    } else if (heads_ok) {
+      run_heads(IntC<kRopeStream>{});
     } else {
       const int64_t total = tokens * (int64_t)(hq + hkv) * half;
       rope_scalar<C><<<flat_grid(total, 256, 1 << 20), 256, 0, st>>>(q, k, ct, sn, q_out, k_out,
