@@ -122,7 +122,51 @@ __global__ __launch_bounds__(256) void token_gather_flat(const u32x4* __restrict
   }
 }
 
-// Any row length / alignment: element-wise (E = 1-, 2- or 4-byte element).
+// Gathers that read source rows more than once, and rows that are no whole
+// 16-byte vectors. A row is cut into `slices` column slices (a power of two,
+// at most 8) of `width` vectors, and workgroup b moves slice b % slices:
+// workgroups are dealt to the 8 XCDs round-robin, so each XCD's 4 MB L2 sees
+// one slice of the source only, and a row that k destinations name is fetched
+// from beyond the L2s once instead of once per XCD. (Where the deal is another,
+// only the speed changes.) One wave per destination row and slice; loads are
+// cached, stores nontemporal. The last vector of a row is its last 16 bytes
+// (it repeats up to 15 of its neighbour's, the same bytes); ANY: rows and
+// buffers of any alignment, at least 16 bytes a row.
+// Bound by the 8 L2s' fills and the writes: 2048 rows of 8 KB to 12288 17.3 us,
+// 117 MB at 6.8 TB/s, where the flat form read 100 MB from beyond the L2s and
+// took 31.9 (24.8 with its loads cached); two, four and eight rows in flight per
+// wave 17.4, 18.8 and 21.0.
+template <bool ANY>
+__global__ __launch_bounds__(256) void token_gather_slices(const char* __restrict__ src,
+                                                           const int64_t* __restrict__ idx, char* __restrict__ dst,
+                                                           int64_t n_dst, int64_t row_bytes, int64_t n_src,
+                                                           int slices, int64_t width) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t nvec = (row_bytes + 15) / 16, last = row_bytes - 16;
+  const int64_t c0 = (int64_t)(blockIdx.x % (unsigned)slices) * width;
+  const int64_t c1 = c0 + width < nvec ? c0 + width : nvec;
+  const int64_t groups = gridDim.x / (unsigned)slices;
+  for (int64_t row = (int64_t)(blockIdx.x / (unsigned)slices) * 4 + wave; row < n_dst; row += groups * 4) {
+    const int64_t s = idx[row];  // uniform: a scalar load
+    const bool valid = s >= 0 && s < n_src;
+    const char* from = src + (valid ? s : 0) * row_bytes;
+    char* to = dst + row * row_bytes;
+    for (int64_t v = c0 + lane; v < c1; v += 64) {
+      const int64_t at = v * 16 < last ? v * 16 : last;
+      u32x4 w = {0u, 0u, 0u, 0u};
+      if constexpr (ANY) {
+        if (valid) w = *reinterpret_cast<const u32x4_any*>(from + at);
+        __builtin_nontemporal_store(w, reinterpret_cast<u32x4_any*>(to + at));
+      } else {
+        if (valid) w = *reinterpret_cast<const u32x4*>(from + at);
+        st_stream(w, reinterpret_cast<u32x4*>(to + at));
+      }
+    }
+  }
+}
+
+// Rows under 16 bytes: element-wise (E = 1-, 2- or 4-byte element).
 template <class E>
 __global__ __launch_bounds__(256) void token_gather_elems(const E* __restrict__ src,
                                                           const int64_t* __restrict__ idx,
@@ -397,6 +441,7 @@ constexpr int64_t kGatherR8Min = 4096;
 // vs 12.1 us; 8192 -> 16384 rows of 1024, 11.8 vs 12.6; 4096 rows of 2048,
 // 6.8 vs 7.4.
 constexpr int64_t kGatherFlatMin = int64_t(1) << 22;
+constexpr int64_t kGatherSliceMin = 128;
 
 int32_t gather(const void* src, const int64_t* indices, void* dst, int64_t n_dst, int64_t h,
                int32_t dtype, int64_t n_src, hipStream_t st) {
@@ -405,7 +450,33 @@ int32_t gather(const void* src, const int64_t* indices, void* dst, int64_t n_dst
   if (es == 0) return (int32_t)hipErrorInvalidValue;
   const unsigned grid = row_grid(n_dst);
   const int64_t row_bytes = h * es;
-  if (row_bytes % 16 == 0 && host_aligned(src, 16) && host_aligned(dst, 16)) {
+  const bool whole = row_bytes % 16 == 0 && host_aligned(src, 16) && host_aligned(dst, 16);
+  // Sliced where source rows repeat often (more than two destinations a source
+  // row, whose count the checked launchers know) in rows of at least
+  // kGatherSliceMin vectors, and for every ragged row: slices of at least 64
+  // vectors, whole cache lines. Same-run A/B on MI355X, bf16, buffers on chip /
+  // from HBM: 2048 -> 12288 rows of 4096 30.9 / 31.5 vs 18.8 / 18.7 us, 4096 -> 32768
+  // of 7168 145.9 / 146.0 vs 108.1 / 108.1, 8192 -> 49152 of 2048 62.1 / 65.7 vs 48.2 /
+  // 48.1, 8192 -> 32768 of 1024 22.0 / 23.5 vs 18.5 / 23.2 (of 512, one slice: 11.1 /
+  // 11.6 vs 10.5 / 12.9, not taken); two destinations a row
+  // lose from HBM (2048 -> 4096 of 4096 10.8 / 11.7 vs 8.9 / 12.6). Ragged rows
+  // against the element-wise kernel: 1000 -> 3000 of 4100 14.1 / 21.5 vs 7.8 / 11.1,
+  // 64 of 5461 4.1 / 7.4 vs 2.7 / 2.8.
+  auto run_slices = [&](auto any) {
+    const int64_t nvec = (row_bytes + 15) / 16;
+    int slices = 1;
+    while (slices < 8 && nvec >= 64 * 2 * slices) slices *= 2;
+    const int64_t width = ((nvec + slices - 1) / slices + 7) / 8 * 8;
+    const int64_t groups = (n_dst + 3) / 4;
+    const int64_t cap = kMaxRowGroups;
+    token_gather_slices<decltype(any)::value><<<(unsigned)((groups < cap ? groups : cap) * slices), 256, 0, st>>>(
+        static_cast<const char*>(src), indices, static_cast<char*>(dst), n_dst, row_bytes, n_src, slices, width);
+  };
+  if (!whole && row_bytes >= 16) {
+    run_slices(std::true_type{});
+  } else if (whole && n_dst / 2 > n_src && row_bytes >= 16 * kGatherSliceMin) {
+    run_slices(std::false_type{});
+  } else if (whole) {
     const int64_t rv = row_bytes / 16;
     if (rv > 512 || (rv >= 64 && n_dst * rv >= kGatherFlatMin)) {
       token_gather_flat<<<flat_grid(n_dst * rv, 256, 1 << 20), 256, 0, st>>>(

@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from custom_cuda_kernals_amd import _native as native
-from oracle import eager, inputs
+from oracle import eager, inputs, moe
 from oracle import fp8 as ofp8
 from tests._parity import assert_codes_equal, assert_f32_bits_equal, bits_equal
 
@@ -160,3 +160,27 @@ def test_fp8_block(dtype):
         assert_codes_equal(q.t, codes)
         assert_f32_bits_equal(s, s_ref)
         q.check()
+
+
+@pytest.mark.parametrize("dtype", DTYPES + [F8["e4m3"]], ids=lambda d: str(d).split(".")[-1])
+def test_gather(dtype):
+    """Ragged rows and, with more than two destinations a source row, sliced whole
+    ones: one vector and less, both sides of every slice count, a last slice of
+    few vectors, indices out of range, one destination row."""
+    es = dtype.itemsize
+    nbytes = [15, 16, 17, 1000, 1023, 1024, 2047, 2048, 2064, 4096, 4080, 8191, 8192, 8208, 11008, 16384]
+    for rb in nbytes:
+        h = max(1, rb // es)
+        for n_dst in (1, 7, 4 * 19 + 1):
+            src = torch.randint(0, 256, (19, h * es), dtype=torch.uint8, generator=torch.Generator().manual_seed(rb))
+            idx = torch.randint(0, 19, (n_dst,), generator=torch.Generator().manual_seed(rb + n_dst))
+            bad = torch.zeros(n_dst, dtype=torch.bool)
+            if n_dst > 5:
+                idx[3], idx[5] = 19, -2
+                bad[3] = bad[5] = True
+            offset = rb % 2
+            dst = Guarded((n_dst, h), dtype, offset)
+            native.token_gather_fwd(_off(src.view(dtype), offset), idx.cuda(), dst.t)
+            ref = torch.where(bad[:, None], torch.zeros((), dtype=torch.uint8), src[torch.where(bad, 0, idx)])
+            assert torch.equal(dst.t.view(torch.uint8).cpu(), ref), (rb, n_dst)
+            dst.check()
