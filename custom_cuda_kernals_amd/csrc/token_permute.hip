@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256) void token_gather_slices(const char* __restric
   }
 }
 
-// Rows under 16 bytes: element-wise (E = 1-, 2- or 4-byte element).
+// Short ragged rows: element-wise (E = 1-, 2- or 4-byte element).
 template <class E>
 __global__ __launch_bounds__(256) void token_gather_elems(const E* __restrict__ src,
                                                           const int64_t* __restrict__ idx,
@@ -279,24 +279,78 @@ __device__ inline float combine_scalar_column(const void* eo, const int64_t* it,
   return h == 1 ? aten_row_sum(k, o.p_slot, o.p_row, term) : aten_scalar_sum(k, o.p_slot, term);
 }
 
+// One scalar column of one token for k <= 16: aten_scalar_sum's operations
+// (no 16-step block of a slot completes, so each slot is one running sum), with
+// every index, then every element, loaded before the first is used.
+template <class C>
+__device__ inline float combine_tail(const char* eo, const int64_t* it, const float* wt, int k, int64_t row_bytes,
+                                     int64_t c, int64_t n_rows) {
+  float x[16];
+  int64_t r[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) r[j] = it[j < k ? j : 0];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const bool ok = j < k && r[j] >= 0 && r[j] < n_rows;
+    x[j] = ok ? wt[j] * C::load1(eo + r[j] * row_bytes, c) : 0.0f;
+  }
+  const int whole = k & ~3;
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int j = 0; j < 16; ++j) s[j % 4] = j < whole ? s[j % 4] + x[j] : s[j % 4];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) s[0] = j >= whole && j < k ? s[0] + x[j] : s[0];
+  return ((s[0] + s[1]) + s[2]) + s[3];
+}
+
 // Weighted combine on 16-byte vectors: one workgroup per token, VPL vectors
 // per thread per step; JU expert rows are loaded together before they are
 // accumulated in j order (CASC: in ATen's block cascade, for k > 16). That is
-// torch's order for the main columns; the launcher then rewrites the other
-// (at most 31) columns with token_combine_elems on the same stream. Bounding
-// this kernel by the main columns instead measured 3 % slower at 4096 tokens
-// x hidden 7168 (76.0 against 73.5 us, k = 6) for the same instructions. A
+// torch's order for the main columns; the other (at most 31) columns have one
+// of their own. A
 // dropped term (index outside the source rows) adds +0.0, which changes no
 // sum that starts at +0.0.
-template <class C, int THREADS, int VPL, int JU, bool CASC>
-__global__ __launch_bounds__(THREADS) void token_combine_vec(const u32x4* __restrict__ eo,
+//
+// ANY: rows of `row_bytes` bytes and buffers at any element boundary, by
+// unaligned vectors; row_vecs covers the main columns only, and for k <= 16 the
+// workgroups from main_groups on sum the other columns (combine_tail) in the
+// same launch, beside the others instead of after them.
+template <class C, int THREADS, int VPL, int JU, bool CASC, bool ANY>
+__global__ __launch_bounds__(THREADS) void token_combine_vec(const char* __restrict__ eo,
                                                              const int64_t* __restrict__ uidx,
                                                              const float* __restrict__ w,
-                                                             u32x4* __restrict__ out, int64_t n_tokens,
-                                                             int64_t k, int64_t row_vecs, int64_t n_rows,
-                                                             int p_main) {
+                                                             char* __restrict__ out, int64_t n_tokens,
+                                                             int64_t k, int64_t row_vecs, int64_t row_bytes,
+                                                             int64_t n_rows, int p_main, unsigned main_groups) {
+  if constexpr (ANY && !CASC) {
+    if (blockIdx.x >= main_groups) {
+      const int64_t c = row_vecs * C::VEC + threadIdx.x % 32;
+      const int64_t step = (int64_t)(gridDim.x - main_groups) * (THREADS / 32);
+      for (int64_t t = (int64_t)(blockIdx.x - main_groups) * (THREADS / 32) + threadIdx.x / 32; t < n_tokens;
+           t += step) {
+        if (c * C::kBytes < row_bytes) {
+          C::store1(out + t * row_bytes, c, combine_tail<C>(eo, uidx + t * k, w + t * k, (int)k, row_bytes, c, n_rows));
+        }
+      }
+      return;
+    }
+  }
+  auto load = [&](int64_t r, int64_t c) {
+    if constexpr (ANY) {
+      return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(eo + r * row_bytes + c * 16));
+    } else {
+      return ld_stream(reinterpret_cast<const u32x4*>(eo) + r * row_vecs + c);
+    }
+  };
+  auto store = [&](const u32x4& v, int64_t t, int64_t c) {
+    if constexpr (ANY) {
+      __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any*>(out + t * row_bytes + c * 16));
+    } else {
+      st_stream(v, reinterpret_cast<u32x4*>(out) + t * row_vecs + c);
+    }
+  };
   constexpr int VEC = C::VEC;
-  for (int64_t t = blockIdx.x; t < n_tokens; t += gridDim.x) {
+  for (int64_t t = blockIdx.x; t < n_tokens; t += main_groups) {
     const int64_t* it = uidx + t * k;
     const float* wt = w + t * k;
     for (int64_t base = threadIdx.x; base < row_vecs; base += THREADS * VPL) {
@@ -319,7 +373,7 @@ __global__ __launch_bounds__(THREADS) void token_combine_vec(const u32x4* __rest
 #pragma unroll
           for (int v = 0; v < VPL; ++v) {
             const int64_t c = base + THREADS * v;
-            if (ok[u] && c < row_vecs) raw[u][v] = ld_stream(eo + r * row_vecs + c);
+            if (ok[u] && c < row_vecs) raw[u][v] = load(r, c);
           }
         }
 #pragma unroll
@@ -358,7 +412,7 @@ __global__ __launch_bounds__(THREADS) void token_combine_vec(const u32x4* __rest
 #pragma unroll
           for (int i = 0; i < VEC; ++i) acc[v][i] = cas[v][i].total();
         }
-        if (c < row_vecs) st_stream(C::pack(acc[v]), out + t * row_vecs + c);
+        if (c < row_vecs) store(C::pack(acc[v]), t, c);
       }
     }
   }
@@ -442,6 +496,8 @@ constexpr int64_t kGatherR8Min = 4096;
 // 6.8 vs 7.4.
 constexpr int64_t kGatherFlatMin = int64_t(1) << 22;
 constexpr int64_t kGatherSliceMin = 128;
+// Ragged rows of fewer bytes stay element-wise (600 rows of 200 bytes: 2.2 vs 2.4 us).
+constexpr int64_t kGatherAnyMin = 256;
 
 int32_t gather(const void* src, const int64_t* indices, void* dst, int64_t n_dst, int64_t h,
                int32_t dtype, int64_t n_src, hipStream_t st) {
@@ -472,7 +528,7 @@ int32_t gather(const void* src, const int64_t* indices, void* dst, int64_t n_dst
     token_gather_slices<decltype(any)::value><<<(unsigned)((groups < cap ? groups : cap) * slices), 256, 0, st>>>(
         static_cast<const char*>(src), indices, static_cast<char*>(dst), n_dst, row_bytes, n_src, slices, width);
   };
-  if (!whole && row_bytes >= 16) {
+  if (!whole && row_bytes >= kGatherAnyMin) {
     run_slices(std::true_type{});
   } else if (whole && n_dst / 2 > n_src && row_bytes >= 16 * kGatherSliceMin) {
     run_slices(std::false_type{});
@@ -532,17 +588,35 @@ int32_t combine(const void* eo, const int64_t* uidx, const float* w, void* out, 
   return with_codec(dtype, [&](auto codec) {
     using C = decltype(codec);
     const unsigned grid = row_grid(n_tokens);
-    if (h % C::VEC == 0 && host_aligned(eo, 16) && host_aligned(out, 16)) {
+    // Rows of main columns only by aligned vectors; other rows' main columns by
+    // unaligned ones, in the same forms, with the other columns beside them.
+    const bool whole = order.main_cols == h && host_aligned(eo, 16) && host_aligned(out, 16);
+    // (Rows of under 128 columns that are no whole vectors stay on the
+    // element-wise kernel: 2.9 vs 3.4 us at 300 tokens of 100, top 2.) On MI355X
+    // against that kernel, which took every such row, bf16: 1000 tokens of 4100, top
+    // 3, 23.7 vs 9.4 us; 16 of 5461, top 4, 19.6 vs 4.0; 8000 of 1001, top 4, 48.9 vs
+    // 20.1; fp16 2048 of 7001, top 8, 231 vs 57.6; fp32 777 of 5461, top 5, 63.4 vs
+    // 20.6. Against aligned vectors and a second launch for the other columns,
+    // 2048 of 4104, top 6, 25.7 vs 24.2 (1000 of 1000, top 6, 8.2 vs 8.4).
+    const bool vectors = host_aligned(eo, 16) && host_aligned(out, 16) && h % C::VEC == 0;
+    if (order.main_cols >= C::VEC && (vectors || h >= 128)) {
       // Two expert rows in flight per step. Top-1/2 rows: 4 vectors per thread
       // (9.4 us at T=2048, k=2, hidden 4096 bf16); deeper top-k: 2 per thread
       // (20.5 us at k=6); both measured on MI355X against 1-8 vectors and 1-8 rows.
-      const int64_t rv = h / C::VEC;
       const int64_t mv = order.main_cols / C::VEC;
-      auto wide = [&](auto vpl) {
-        constexpr int V = decltype(vpl)::value;
-        token_combine_vec<C, 512, V, 2, false><<<grid, 512, 0, st>>>(
-            static_cast<const u32x4*>(eo), uidx, w, static_cast<u32x4*>(out), n_tokens, k, rv, n_rows, order.p_main);
+      const int64_t rv = mv;
+      auto launch = [&](auto threads, auto vpl, auto casc) {
+        constexpr int TH = decltype(threads)::value, V = decltype(vpl)::value;
+        auto go = [&](auto any) {
+          constexpr bool kTail = decltype(any)::value && !decltype(casc)::value;
+          const unsigned tail = kTail && order.main_cols < h ? row_grid((n_tokens + TH / 32 - 1) / (TH / 32)) : 0u;
+          token_combine_vec<C, TH, V, 2, decltype(casc)::value, decltype(any)::value><<<grid + tail, TH, 0, st>>>(
+              static_cast<const char*>(eo), uidx, w, static_cast<char*>(out), n_tokens, k, rv, h * C::kBytes, n_rows,
+              order.p_main, grid);
+        };
+        whole ? go(std::false_type{}) : go(std::true_type{});
       };
+      auto wide = [&](auto vpl) { launch(IntC<512>{}, vpl, std::false_type{}); };
       // Many tokens, rows of 512 to 2048 vectors (4096 to 16384 bf16):
       // 512-thread workgroups holding the row in one pass, measured on MI355X
       // (graph-replayed) against the shapes below: 35.0 vs 38.1 us at T=8192,
@@ -560,15 +634,9 @@ int32_t combine(const void* eo, const int64_t* uidx, const float* w, void* out, 
       // and shorter rows lose (6.1 vs 5.3 us at 512 tokens, hidden 2048 bf16,
       // top 6).
       const bool few = n_tokens <= kCombineFewTokens && k <= 16 && mv >= 512;
-      if (mv == 0) {
-        // Rows of 8 to 31 elements: scalar columns only.
-      } else if (k > 16) {
+      if (k > 16) {
         // Deeper sums take ATen's block cascade: one vector per thread.
-        with_row_threads<1, 512>(mv, [&](auto threads) {
-          constexpr int TH = decltype(threads)::value;
-          token_combine_vec<C, TH, 1, 2, true><<<grid, TH, 0, st>>>(
-              static_cast<const u32x4*>(eo), uidx, w, static_cast<u32x4*>(out), n_tokens, k, rv, n_rows, order.p_main);
-        });
+        with_row_threads<1, 512>(mv, [&](auto threads) { launch(threads, IntC<1>{}, std::true_type{}); });
       } else if (many || few) {
         if (mv <= 512) {
           wide(IntC<1>{});
@@ -583,29 +651,14 @@ int32_t combine(const void* eo, const int64_t* uidx, const float* w, void* out, 
         // 2048 (fp32 hidden 4096, top 2); 27.9 vs 30.0 at 3072 tokens (bf16
         // hidden 8192); two passes of 128 threads for bf16 hidden 7168 stay
         // faster (14.0 vs 15.3 us at 1536 tokens).
-        with_row_threads<4, 256>(mv, [&](auto threads) {
-          constexpr int TH = decltype(threads)::value;
-          token_combine_vec<C, TH, 4, 2, false><<<grid, TH, 0, st>>>(
-              static_cast<const u32x4*>(eo), uidx, w, static_cast<u32x4*>(out), n_tokens, k, rv, n_rows, order.p_main);
-        });
+        with_row_threads<4, 256>(mv, [&](auto threads) { launch(threads, IntC<4>{}, std::false_type{}); });
       } else if (k <= 2) {
-        with_row_threads<4, 128>(mv, [&](auto threads) {
-          constexpr int TH = decltype(threads)::value;
-          token_combine_vec<C, TH, 4, 2, false><<<grid, TH, 0, st>>>(
-              static_cast<const u32x4*>(eo), uidx, w, static_cast<u32x4*>(out), n_tokens, k, rv, n_rows, order.p_main);
-        });
+        with_row_threads<4, 128>(mv, [&](auto threads) { launch(threads, IntC<4>{}, std::false_type{}); });
       } else {
-        with_row_threads<2, 256>(mv, [&](auto threads) {
-          constexpr int TH = decltype(threads)::value;
-          token_combine_vec<C, TH, 2, 2, false><<<grid, TH, 0, st>>>(
-              static_cast<const u32x4*>(eo), uidx, w, static_cast<u32x4*>(out), n_tokens, k, rv, n_rows, order.p_main);
-        });
+        with_row_threads<2, 256>(mv, [&](auto threads) { launch(threads, IntC<2>{}, std::false_type{}); });
       }
-      if (order.main_cols < h) {
-        // The h mod 32 scalar columns (at most 31) rewritten in a launch of
-        // their own, so the vector kernel keeps its registers (in the kernel,
-        // their code took 90 SGPRs instead of 64 and a second round of
-        // workgroups at 2048 tokens: 24.1 against 20.4 us, k = 6).
+      if (order.main_cols < h && k > 16) {
+        // The scalar columns of deeper sums in a launch of their own.
         token_combine_elems<C, 64><<<grid, 64, 0, st>>>(eo, uidx, w, out, n_tokens, k, h, order.main_cols, n_rows,
                                                         order);
       }

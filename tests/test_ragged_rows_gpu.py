@@ -168,7 +168,7 @@ def test_gather(dtype):
     ones: one vector and less, both sides of every slice count, a last slice of
     few vectors, indices out of range, one destination row."""
     es = dtype.itemsize
-    nbytes = [15, 16, 17, 1000, 1023, 1024, 2047, 2048, 2064, 4096, 4080, 8191, 8192, 8208, 11008, 16384]
+    nbytes = [15, 17, 250, 254, 256, 258, 262, 1000, 1023, 1024, 2047, 2048, 2064, 4096, 4080, 8191, 8192, 8208, 11008, 16384]
     for rb in nbytes:
         h = max(1, rb // es)
         for n_dst in (1, 7, 4 * 19 + 1):
@@ -184,3 +184,23 @@ def test_gather(dtype):
             ref = torch.where(bad[:, None], torch.zeros((), dtype=torch.uint8), src[torch.where(bad, 0, idx)])
             assert torch.equal(dst.t.view(torch.uint8).cpu(), ref), (rb, n_dst)
             dst.check()
+
+
+@pytest.mark.parametrize("k", [1, 3, 4, 8, 16, 17])
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).split(".")[-1])
+def test_combine(dtype, k):
+    """Main columns by unaligned vectors with the scalar columns beside them in
+    one launch (a launch of their own past top 16): row lengths around the
+    32-column boundaries, one token, terms out of range, unaligned buffers."""
+    for h in (127, 128, 129, 159, 160, 1000, 4100, 4127, 8200):
+        for t in (1, 9):
+            eo, ui, w = inputs.combine_inputs(t, k, h, dtype, seed=h + k)
+            ui_ref, w_ref = ui.clone(), w.clone()
+            if t > 1:
+                ui[2, k - 1], ui_ref[2, k - 1], w_ref[2, k - 1] = t * k, 0, 0.0
+                ui[4, 0], ui_ref[4, 0], w_ref[4, 0] = -1, 0, 0.0
+            offset = h % 2
+            out = Guarded((t, h), dtype, offset)
+            native.token_combine_fwd(_off(eo, offset), ui.cuda(), w.cuda(), out.t)
+            assert bits_equal(out.t, moe.token_combine_aten(eo, ui_ref, w_ref)).all(), (t, h)
+            out.check()
