@@ -105,7 +105,7 @@ def native_compile_args(sanitize: bool = False) -> list[str]:
              "-fno-sanitize-recover=undefined"] if sanitize else ["-O2"]
     args += [
         str(CSRC / "native.cpp"),
-        f"-L{tdir / 'lib'}", "-ltorch_python", "-ltorch", "-lc10", "-lc10_hip",
+        f"-L{tdir / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
         f"-Wl,-rpath,{tdir / 'lib'}",
         f"-L{PKG}", "-lcustom_kernels_amd",
         "-Wl,-rpath,$ORIGIN",

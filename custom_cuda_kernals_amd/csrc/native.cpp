@@ -682,6 +682,8 @@ void moe_router_fwd(py::handle logits, py::handle topk_weights, py::handle topk_
 
 }  // namespace
 
+#include "native_calls.hpp"
+
 PYBIND11_MODULE(_native, m) {
   m.doc() = "Validating binding over the libcustom_kernels_amd C ABI (gfx950).";
   m.def("rmsnorm_residual_fwd", &rmsnorm_residual_fwd, py::arg("x"), py::arg("residual"), py::arg("weight"),
@@ -711,4 +713,6 @@ PYBIND11_MODULE(_native, m) {
         "Test hook: the hipStream_t (as an int) the most recent call launched on.");
   m.def("swiglu_fp8_fwd", &swiglu_fp8_fwd, py::arg("gate"), py::arg("up"), py::arg("y_fp8"), py::arg("scale"),
         py::arg("fp8_format"), py::arg("static_scale") = py::none());
+  // The Python API in one call each (native_calls.hpp).
+  if (PyModule_AddFunctions(m.ptr(), calls::kMethods) != 0) throw py::error_already_set();
 }

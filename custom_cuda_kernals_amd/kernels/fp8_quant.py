@@ -43,6 +43,10 @@ def fp8_quant(
     scale (requires ``granularity="tensor"``); returned as a ``[1]`` tensor.
     Returns ``(x_fp8, scale)``.
     """
+    # The ordinary call in one native call; None: the long way below, which raises the errors.
+    out = native.fp8_quant_call(x, fp8_format, granularity, scale)
+    if out is not None:
+        return out
     check_fp8_format(fp8_format)
     if granularity not in ("block", "tensor", "token"):
         raise ValueError(f"granularity must be 'block', 'tensor' or 'token', got {granularity!r}")

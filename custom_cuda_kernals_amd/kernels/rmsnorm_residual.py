@@ -23,6 +23,10 @@ def rmsnorm_residual(
     x, residual: ``[..., hidden_dim]`` contiguous device tensors, same dtype
     (float32 / float16 / bfloat16). weight: ``[hidden_dim]``, same dtype.
     """
+    # The ordinary call in one native call; None: the long way below, which raises the errors.
+    out = native.rmsnorm_residual_call(x, residual, weight, eps)
+    if out is not None:
+        return out
     y = torch.empty_like(x)
     residual_out = torch.empty_like(x)
     native.rmsnorm_residual_fwd(x, residual, weight, y, residual_out, eps)
@@ -45,6 +49,10 @@ def rmsnorm_residual_fp8(
     returned with shape ``x.shape[:-1]``. ``scale=<float>``: static per-tensor
     scale, returned as a ``[1]`` tensor. Returns ``(y_fp8, scale, residual_out)``.
     """
+    # The ordinary call in one native call; None: the long way below, which raises the errors.
+    out = native.rmsnorm_residual_fp8_call(x, residual, weight, eps, fp8_format, scale)
+    if out is not None:
+        return out
     check_fp8_format(fp8_format)
     y_fp8 = torch.empty(x.shape, dtype=FP8_TORCH_DTYPES[fp8_format], device=x.device)
     residual_out = torch.empty_like(x)

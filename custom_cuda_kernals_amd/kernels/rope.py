@@ -23,6 +23,10 @@ def rope(
     tensors. cos, sin: ``[S, D/2]`` float32. With ``inplace=True`` q and k are
     overwritten and returned.
     """
+    # The ordinary call in one native call; None: the long way below, which raises the errors.
+    out = native.rope_call(q, k, cos, sin, inplace)
+    if out is not None:
+        return (q, k) if inplace else out
     if inplace:
         q_out, k_out = q, k
     else:

@@ -16,6 +16,10 @@ __all__ = ["swiglu", "swiglu_fp8"]
 
 def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """``y = SiLU(gate) * up``. gate, up: same-shape contiguous device tensors."""
+    # The ordinary call in one native call; None: the long way below, which raises the errors.
+    out = native.swiglu_call(gate, up)
+    if out is not None:
+        return out
     y = torch.empty_like(gate)
     native.swiglu_fwd(gate, up, y)
     return y
@@ -31,6 +35,10 @@ def swiglu_fp8(
     with shape ``gate.shape[:-1]``; ``scale=<float>``: static per-tensor scale,
     returned as a ``[1]`` tensor. Returns ``(y_fp8, scale)``.
     """
+    # The ordinary call in one native call; None: the long way below, which raises the errors.
+    out = native.swiglu_fp8_call(gate, up, fp8_format, scale)
+    if out is not None:
+        return out
     check_fp8_format(fp8_format)
     y_fp8 = torch.empty(gate.shape, dtype=FP8_TORCH_DTYPES[fp8_format], device=gate.device)
     if scale is None:

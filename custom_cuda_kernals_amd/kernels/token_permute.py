@@ -25,6 +25,10 @@ __all__ = ["token_gather", "token_combine", "compute_permutation"]
 def token_gather(src: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
     """``dst[i] = src[indices[i]]``. src: ``[S, H]`` contiguous device tensor,
     indices: ``[N]`` int64. Returns ``dst: [N, H]``."""
+    # The ordinary call in one native call; None: the long way below, which raises the errors.
+    out = native.token_gather_call(src, indices)
+    if out is not None:
+        return out
     n = indices.shape[0]
     h = src.shape[1]
     dst = torch.empty((n, h), dtype=src.dtype, device=src.device)
@@ -37,6 +41,10 @@ def token_combine(expert_output: torch.Tensor, unpermute_index: torch.Tensor, we
 
     expert_output: ``[N, H]`` contiguous device tensor; unpermute_index:
     ``[T, k]`` int64; weights: ``[T, k]`` float32. Returns ``[T, H]``."""
+    # The ordinary call in one native call; None: the long way below, which raises the errors.
+    out = native.token_combine_call(expert_output, unpermute_index, weights)
+    if out is not None:
+        return out
     t, _ = unpermute_index.shape
     h = expert_output.shape[1]
     combined = torch.empty((t, h), dtype=expert_output.dtype, device=expert_output.device)
@@ -54,6 +62,11 @@ def compute_permutation(topk_indices: torch.Tensor, num_experts: int | None = No
     ordered after every expert) this is one HIP kernel, a stable counting sort;
     without it, the reference's torch ops (a stable argsort and its inverse,
     baselines/token_permute.py:55-70) on the tensor's device."""
+    if num_experts is not None:
+        # The ordinary call in one native call; None: the long way below, which raises the errors.
+        out = native.compute_permutation_call(topk_indices, num_experts)
+        if out is not None:
+            return out
     t, k = topk_indices.shape
     if num_experts is not None:
         permute_index = torch.empty(t * k, dtype=torch.int64, device=topk_indices.device)

@@ -1,0 +1,150 @@
+"""The one-call form of the Python API against the long way (torch.empty and
+the validating *_fwd functions): the same outputs (shape, stride, dtype, device
+and bits) over the forms both take; what the long way refuses is refused with
+its error; tensor subclasses, torch modes and functorch transforms go the long
+way; calls on a side stream and from several threads."""
+
+from __future__ import annotations
+
+import threading
+
+import pytest
+import torch
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from custom_cuda_kernals_amd import kernels as K
+from custom_cuda_kernals_amd._lib import native
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ["rmsnorm_residual_call", "rmsnorm_residual_fp8_call", "swiglu_call", "swiglu_fp8_call", "rope_call",
+         "fp8_quant_call", "token_gather_call", "token_combine_call", "compute_permutation_call", "moe_router_call"]
+
+
+def _r(*shape, dtype=torch.bfloat16, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype).cuda()
+
+
+def _calls(dtype):
+    x, r, w = _r(3, 5, 264, dtype=dtype), _r(3, 5, 264, dtype=dtype, seed=1), _r(264, dtype=dtype, seed=2)
+    m = _r(130, 264, dtype=dtype, seed=3)
+    q, k = _r(2, 7, 4, 64, dtype=dtype), _r(2, 7, 2, 64, dtype=dtype, seed=4)
+    cos, sin = _r(7, 32, dtype=torch.float32), _r(7, 32, dtype=torch.float32, seed=5)
+    ids = torch.randint(0, 9, (6, 3), generator=torch.Generator().manual_seed(6)).cuda()
+    idx = torch.randperm(18, generator=torch.Generator().manual_seed(7)).cuda()
+    wt = torch.rand(6, 3, generator=torch.Generator().manual_seed(8)).cuda()
+    return {
+        "norm": lambda: K.rmsnorm_residual(x, r, w), "norm1d": lambda: K.rmsnorm_residual(x[0, 0], r[0, 0], w, 1e-5),
+        "norm_param": lambda: K.rmsnorm_residual(x, r, torch.nn.Parameter(w), 1e-5),
+        "norm_int_eps": lambda: K.rmsnorm_residual(x, r, w, 1),
+        "norm_fp8": lambda: K.rmsnorm_residual_fp8(x, r, w, 1e-5),
+        "norm_fp8_1d": lambda: K.rmsnorm_residual_fp8(x[0, 0], r[0, 0], w, 1e-5, "e5m2"),
+        "norm_fp8_static": lambda: K.rmsnorm_residual_fp8(x, r, w, 1e-5, "e5m2", 0.05),
+        "norm_fp8_int_scale": lambda: K.rmsnorm_residual_fp8(x, r, w, 1e-5, "e4m3", 1),
+        "swiglu": lambda: K.swiglu(x, r), "swiglu_0d": lambda: K.swiglu(x[0, 0, 0], r[0, 0, 0]),
+        "swiglu_fp8": lambda: K.swiglu_fp8(x, r), "swiglu_fp8_static": lambda: K.swiglu_fp8(x, r, "e5m2", 0.05),
+        "rope": lambda: K.rope(q, k, cos, sin),
+        "rope_inplace": lambda: K.rope(q.clone(), k.clone(), cos, sin, inplace=True),
+        "block": lambda: K.fp8_quant(m), "token": lambda: K.fp8_quant(m, "e5m2", "token"),
+        "tensor": lambda: K.fp8_quant(m, "e4m3", "tensor"),
+        "static": lambda: K.fp8_quant(m, "e4m3", "tensor", scale=0.05),
+        "gather": lambda: K.token_gather(m, idx), "combine": lambda: K.token_combine(m, ids, wt),
+        "gather_fp8": lambda: K.token_gather(m.to(torch.float8_e4m3fn), idx),
+        "permutation": lambda: K.compute_permutation(ids, 9), "router": lambda: K.moe_router(m[:, :24].contiguous(), 3),
+        "router_raw": lambda: K.moe_router(m[:, :8].contiguous(), 8, False),
+        "empty_static": lambda: K.fp8_quant(m[:0], "e4m3", "tensor", scale=0.25),
+        "empty": lambda: K.swiglu(x[:0], r[:0]),
+    }
+
+
+def _outputs(call):
+    out = call()
+    out = out if isinstance(out, tuple) else (out,)
+    torch.cuda.synchronize()
+    return [(t.shape, t.stride(), t.dtype, t.device, t.requires_grad, t.contiguous().view(-1).view(torch.uint8).tolist())
+            for t in out]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
+def test_equals_the_long_way(dtype, monkeypatch):
+    calls = _calls(dtype)
+    one = {name: _outputs(c) for name, c in calls.items()}
+    for name in NAMES:
+        monkeypatch.setattr(native, name, lambda *a: None)
+    for name, c in calls.items():
+        assert _outputs(c) == one[name], name
+
+
+def test_refused_as_before():
+    x, w = _r(4, 64), _r(64)
+    for call in (lambda: K.rmsnorm_residual(x, x[:, ::2], w), lambda: K.rmsnorm_residual(x, x.half(), w),
+                 lambda: K.rmsnorm_residual(x, x, w[:32]), lambda: K.swiglu(x.t(), x.t()),
+                 lambda: K.swiglu(x, x[:2]), lambda: K.fp8_quant(x[0]), lambda: K.fp8_quant(x, "e3m4"),
+                 lambda: K.fp8_quant(x, "e4m3", "token", 0.5), lambda: K.swiglu_fp8(x, x.cpu()),
+                 lambda: K.fp8_quant(x.double()), lambda: K.token_gather(x, torch.zeros(3, dtype=torch.int32).cuda()),
+                 lambda: K.moe_router(x, 65), lambda: K.compute_permutation(torch.zeros(3, 2).cuda(), 4),
+                 lambda: K.compute_permutation(torch.zeros(3, 2, dtype=torch.int64).cuda(), 257),
+                 lambda: K.rope(x.view(1, 4, 1, 64), x.view(1, 4, 1, 64), w.float(), w.float())):
+        with pytest.raises((ValueError, RuntimeError, TypeError)):
+            call()
+
+
+def test_modes_and_subclasses_go_the_long_way():
+    x = _r(4, 64)
+
+    class Fn(TorchFunctionMode):
+        seen = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            Fn.seen += func is torch.empty_like
+            return func(*args, **(kwargs or {}))
+
+    class Disp(TorchDispatchMode):
+        seen = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Disp.seen += "empty" in str(func)
+            return func(*args, **(kwargs or {}))
+
+    ref = K.swiglu(x, x)
+    with Fn():
+        assert native.swiglu_call(x, x) is None and torch.equal(K.swiglu(x, x), ref)
+    with Disp():
+        assert native.swiglu_call(x, x) is None
+        out = K.swiglu(x, x)
+    assert torch.equal(out, ref) and Fn.seen and Disp.seen
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert native.swiglu_call(x.as_subclass(Sub), x) is None
+
+    def inner(t):
+        assert native.swiglu_call(t, t) is None
+        return t
+
+    torch.func.vmap(inner)(x)
+
+
+def test_streams_and_threads():
+    x, r = _r(64, 4096), _r(64, 4096, seed=1)
+    ref = K.swiglu(x, r)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        y = K.swiglu(x, r)
+        assert native._last_launch_stream() == side.cuda_stream
+    side.synchronize()
+    assert torch.equal(y, ref)
+    bad = []
+
+    def work():
+        for _ in range(50):
+            if not torch.equal(K.swiglu(x, r), ref):
+                bad.append(1)
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not bad
