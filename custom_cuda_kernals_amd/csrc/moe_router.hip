@@ -21,10 +21,11 @@
 // Three forms, by expert count E (and token count T), the same steps and
 // results in each:
 //   * E <= 8: one lane per token (moe_router_lanes);
-//   * 9 <= E <= 32, and E <= 64 from T = 4096 on: four lanes per token, each
-//     holding its quarter of every 16-expert stripe (moe_router_groups);
-//     65 <= E <= 256 from T = 8192 (E <= 128) or 12288 on: eight lanes;
-//   * otherwise one wave per token (moe_router_waves), below.
+//   * E >= 9: a group of lanes per token, each holding its part of every
+//     16-expert stripe (moe_router_groups): four lanes up to 16 experts, 16 lanes
+//     above, eight for up to 64 experts of many tokens;
+//   * 16-bit rows of E > 192 and few tokens: one wave per token
+//     (moe_router_waves), below.
 // One wave64 per token holds up to 256 experts (4 per lane, expert
 // e = lane + 64 * slot). The max is a wave all-reduction (DPP). The
 // exponentials go to a per-wave LDS row; every lane then runs its lane
@@ -278,7 +279,7 @@ __global__ __launch_bounds__(kLaneThreads) void moe_router_lanes(const void* __r
   for (int i = 0; i < k; ++i) topk_w[t * k + i] = renormalize ? sel[i][tid] / wsum : sel[i][tid];
 }
 
-// G lanes per token (G = 2, 4 or 8), for n <= 16 * NS experts. The row is
+// G lanes per token (G = 2, 4, 8 or 16), for n <= 16 * NS experts. The row is
 // cut into stripes of 16 experts (the AVX-512 vector), and lane r of a group
 // holds the CW = 16 / G experts [16 s + r CW, 16 s + (r + 1) CW) of every
 // stripe s, so each of the 16 lane classes of the softmax sum lives in one
@@ -290,33 +291,38 @@ __global__ __launch_bounds__(kLaneThreads) void moe_router_lanes(const void* __r
 // with class 0's total. Below 16 experts (one stripe) the sum is a running
 // sum handed from lane to lane instead (G = 2 or 4). The max and each top-k
 // round's arg-max are group all-reductions (xor 1 and xor 2 quad
-// permutations, then for G = 8 the half-row mirror, which pairs each lane
-// with one of the other quad). Lane r of a group writes the outputs of the
+// permutations, then for G = 8 and 16 the half-row mirror, which pairs each lane
+// with one of the other quad, and for G = 16 the row mirror). Lane r of a group writes the outputs of the
 // rounds i = r mod G.
 constexpr int kDppRowShr1 = 0x111;     // lane i reads lane i - 1 of its row
 constexpr int kDppQuadBcast3 = 0xFF;  // quad_perm:[3,3,3,3]
 constexpr int kDppQuadBcast1 = 0xF5;  // quad_perm:[1,1,3,3]
+constexpr int kDppRowRor8 = 0x128;  // lane i reads lane i ^ 8 of its row
 constexpr int kDppRowShr4 = 0x114;  // lane i reads lane i - 4 of its row
 
 template <int G, class Op>
 __device__ inline uint32_t group_allreduce(uint32_t v, Op op) {
-  static_assert(G == 2 || G == 4 || G == 8, "group size");
+  static_assert(G == 2 || G == 4 || G == 8 || G == 16, "group size");
   v = op(v, dpp<kDppQuadXor1>(v));
   if constexpr (G >= 4) v = op(v, dpp<kDppQuadXor2>(v));
   // For an idempotent op, lane i combined with lane 7 - i (the other quad of
   // its 8) completes the group.
-  if constexpr (G == 8) v = op(v, dpp<kDppRowHalfMirror>(v));
+  if constexpr (G >= 8) v = op(v, dpp<kDppRowHalfMirror>(v));
+  // ... and with lane 15 - i, in the other 8 of its 16.
+  if constexpr (G == 16) v = op(v, dpp<kDppRowMirror>(v));
   return v;
 }
 
-// The value of lane r ^ D of this lane's group (D = 1, 2 or 4; groups of 8
-// lanes are aligned within the 16-lane DPP rows).
+// The value of lane r ^ D of this lane's group (D = 1, 2, 4 or 8; groups are
+// aligned within the 16-lane DPP rows).
 template <int D>
 __device__ inline uint32_t lane_xor(uint32_t v, int r) {
   if constexpr (D == 1) {
     return dpp<kDppQuadXor1>(v);
   } else if constexpr (D == 2) {
     return dpp<kDppQuadXor2>(v);
+  } else if constexpr (D == 8) {
+    return dpp<kDppRowRor8>(v);
   } else {
     static_assert(D == 4, "lane distance");
     const uint32_t up = dpp<kDppRowShl4>(v), down = dpp<kDppRowShr4>(v);
@@ -335,7 +341,7 @@ __global__ __launch_bounds__(kLaneThreads) void moe_router_groups(const void* __
   constexpr int PER = NS * CW;           // experts per lane
   constexpr int TPB = kLaneThreads / G;  // tokens per workgroup
   static_assert(PER <= 32 && (VB != 16 || CW % C::VEC == 0) && (VB != 8 || CW * C::kBytes == 8) &&
-                    (VB != 4 || CW * C::kBytes == 4) && (G != 8 || NS >= 2),
+                    (VB != 4 || CW * C::kBytes == 4) && (G < 8 || NS >= 2),
                 "group router shape");
   __shared__ float sel[NS * kSoftmaxLanes][TPB];
   const int tid = threadIdx.x, r = tid % G, slot = tid / G;
@@ -436,7 +442,10 @@ __global__ __launch_bounds__(kLaneThreads) void moe_router_groups(const void* __
 #pragma unroll
       for (int j = 0; j < CW; ++j) {
         const uint32_t a = f32_bits(acc[j]);
-        const uint32_t o = step / CW == 1 ? lane_xor<1>(a, r) : step / CW == 2 ? lane_xor<2>(a, r) : lane_xor<4>(a, r);
+        const uint32_t o = step / CW == 1   ? lane_xor<1>(a, r)
+                           : step / CW == 2 ? lane_xor<2>(a, r)
+                           : step / CW == 4 ? lane_xor<4>(a, r)
+                                            : lane_xor<8>(a, r);
         acc[j] = acc[j] + bits_f32(o);
       }
     }
@@ -451,34 +460,39 @@ __global__ __launch_bounds__(kLaneThreads) void moe_router_groups(const void* __
 #pragma unroll
   for (int i = 0; i < PER; ++i) p[i] = p[i] * inv;
 
-  uint32_t live = 0u;
+  // The remaining experts' probabilities as integer bits (they are >= +0), -1
+  // once selected or absent. A round takes the largest of the group, then the
+  // smallest expert that holds it: two ops per two experts for the maximum,
+  // two each to find it and to strike it out, instead of a running (value,
+  // index) pair over a mask of the live ones.
+  int32_t key[PER];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
 #pragma unroll
     for (int j = 0; j < CW; ++j) {
-      if (kSoftmaxLanes * s + r * CW + j < n) live |= 1u << (s * CW + j);
+      key[s * CW + j] = kSoftmaxLanes * s + r * CW + j < n ? (int32_t)f32_bits(p[s * CW + j]) : -1;
     }
   }
   for (int i = 0; i < k; ++i) {
-    int32_t key = -1;
+    int32_t top = -1;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) top = max(top, key[q]);
+    const int32_t best = (int32_t)group_allreduce<G>((uint32_t)top, MaxI32{});
     uint32_t mine = 0xffffffffu;
-    int bit = -1;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-#pragma unroll
-      for (int j = 0; j < CW; ++j) {
-        const int32_t b = (int32_t)f32_bits(p[s * CW + j]);
-        if (((live >> (s * CW + j)) & 1u) && b > key) {
-          key = b;
-          mine = (uint32_t)(kSoftmaxLanes * s + r * CW + j);
-          bit = s * CW + j;
-        }
-      }
+    for (int q = PER - 1; q >= 0; --q) {
+      if (key[q] == best) mine = (uint32_t)(kSoftmaxLanes * (q / CW) + q % CW);
     }
-    const uint32_t best = group_allreduce<G>((uint32_t)key, MaxI32{});
-    const uint32_t pick = group_allreduce<G>((int32_t)best == key ? mine : 0xffffffffu, MinU32{});
-    if (pick == mine && bit >= 0) live &= ~(1u << bit);
-    sel[i][slot] = bits_f32(best);
+    // (No expert is left where only NaNs of negative sign remain.)
+    if (best >= 0 && mine != 0xffffffffu) mine += (uint32_t)(r * CW);
+    if (best < 0) mine = 0xffffffffu;
+    const uint32_t pick = group_allreduce<G>(mine, MinU32{});
+    const uint32_t own = pick - (uint32_t)(r * CW);
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      if (own == (uint32_t)(kSoftmaxLanes * (q / CW) + q % CW)) key[q] = -1;
+    }
+    sel[i][slot] = bits_f32((uint32_t)best);
     if (i % G == r) topk_i[t * k + i] = (int64_t)pick;
   }
   const float wsum = renormalize ? aten_small_row_sum<TPB>(&sel[0][slot], k) : 1.0f;
@@ -529,19 +543,19 @@ void launch_router_groups(const void* logits, float* w, int64_t* idx, int64_t t,
   moe_router_groups<C, G, NS, 0><<<grid, kLaneThreads, 0, st>>>(logits, w, idx, t, n, k, renorm);
 }
 
-// Group kernels serve up to 64 experts; from 33 on only with enough tokens,
-// where the wave kernel's one wave per token no longer fits the GPU at once.
-constexpr int kGroupMaxExperts = 64;
-constexpr int64_t kGroupWideMinTokens = 4096;
-// Eight lanes per token (32 experts each at most) for 65 to 256 experts, from
-// enough tokens that the wave kernel's one wave per token takes several
-// rounds of the GPU: same-run A/B against it, fp32 / bf16, top-8 of 96 at
-// 8192 tokens 7.4 / 9.2 vs 13.5 / 13.6 us, top-6 of 160 at 12288 8.6 / 11.8
-// vs 14.6 / 15.7, at 16384 9.1 / 12.1 vs 18.3 / 19.6; top-8 of 256 at 16384
-// 14.7 / 18.5 vs 24.0 / 26.1. Below those counts the wave kernel's shorter
-// chain wins (top-6 of 160 at 2048 tokens: 5.4 vs 6.8 us fp32).
-constexpr int kGroup8MaxExperts = 256;
-inline int64_t group8_min_tokens(int n) { return n <= 128 ? 8192 : 12288; }
+// From 17 experts up a token takes 16 lanes, one per lane class of the softmax
+// sum. Graph-replayed on MI355X against the forms that served these sizes, fp32:
+// top-6 of 32 at 4096 tokens 2.9 vs 4.3 us (four lanes), top-8 of 64 at 2048 4.0 vs 6.4
+// (a wave per token) and at 8192 4.9 vs 7.7 (four lanes), top-6 of 160 at 512 / 2048 /
+// 4096 4.1 / 4.3 / 4.8 vs 4.9 / 5.2 / 6.8 (waves) and at 16384 7.5 vs 9.1 (eight lanes),
+// top-8 of 256 at 4096 / 16384 7.1 / 11.9 vs 8.8 (waves) / 14.7. They are bound by the
+// chain of one wave up to about one wave per SIMD (4096 tokens), by instructions
+// after that, where eight lanes hold fewer idle slots of few experts: top-6 of 32
+// at 16384 tokens 4.0 vs 4.2, at 32768 5.2 vs 6.1; top-8 of 64 at 32768 8.1 vs 9.2.
+constexpr int64_t kNarrowMany = 8192;  // twice that from 33 experts up
+// 16-bit rows of more than 192 experts keep a wave per token below this count
+// (top-8 of 256 bf16 at 512 tokens 6.6 vs 7.0 us; at 2048 7.0 vs 7.1, at 4096 8.9 vs 7.4).
+constexpr int64_t kWideFew = 2048;
 
 }  // namespace
 
@@ -553,34 +567,39 @@ extern "C" int32_t launch_moe_router_fwd(const void* logits, float* topk_weights
   if (k == 0) return (int32_t)hipSuccess;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int n = (int)num_experts, kk = (int)k, rn = renormalize != 0;
-  // One workgroup per 64 / G tokens: every grid below fits for any token count this guard lets through.
-  const bool small_grid = num_tokens <= (int64_t)kLaneThreads * (INT32_MAX / 4);
-  const bool groups = n <= 2 * kSoftmaxLanes || (n <= kGroupMaxExperts && num_tokens >= kGroupWideMinTokens);
+  // One workgroup per 64 / G >= 4 tokens: every grid below fits for any token count this guard lets through.
+  const bool small_grid = num_tokens <= 4 * (int64_t)INT32_MAX;
   return with_codec(dtype, [&](auto codec) {
     using C = decltype(codec);
     if (small_grid && n <= kLaneMaxExperts) {
       launch_router_lanes<C, kLaneMaxExperts>(logits, topk_weights, topk_indices, num_tokens, n, kk, rn, st);
       return launch_status();
     }
-    if (small_grid && n > kGroupMaxExperts && n <= kGroup8MaxExperts && num_tokens >= group8_min_tokens(n)) {
-      if (n <= 8 * kSoftmaxLanes) {
-        launch_router_groups<C, 8, 8>(logits, topk_weights, topk_indices, num_tokens, n, kk, rn, st);
-      } else if (n <= 10 * kSoftmaxLanes) {
-        launch_router_groups<C, 8, 10>(logits, topk_weights, topk_indices, num_tokens, n, kk, rn, st);
-      } else {
-        launch_router_groups<C, 8, 16>(logits, topk_weights, topk_indices, num_tokens, n, kk, rn, st);
-      }
+    auto groups = [&](auto lanes, auto stripes) {
+      launch_router_groups<C, decltype(lanes)::value, decltype(stripes)::value>(logits, topk_weights, topk_indices,
+                                                                               num_tokens, n, kk, rn, st);
       return launch_status();
+    };
+    if (small_grid && n <= kSoftmaxLanes) return groups(IntC<4>{}, IntC<1>{});
+    if (small_grid && n <= 4 * kSoftmaxLanes && num_tokens >= (n <= 2 * kSoftmaxLanes ? kNarrowMany : 2 * kNarrowMany)) {
+      return n <= 2 * kSoftmaxLanes ? groups(IntC<8>{}, IntC<2>{}) : groups(IntC<8>{}, IntC<4>{});
     }
-    if (small_grid && groups) {
-      if (n <= kSoftmaxLanes) {
-        launch_router_groups<C, 4, 1>(logits, topk_weights, topk_indices, num_tokens, n, kk, rn, st);
-      } else if (n <= 2 * kSoftmaxLanes) {
-        launch_router_groups<C, 4, 2>(logits, topk_weights, topk_indices, num_tokens, n, kk, rn, st);
-      } else {
-        launch_router_groups<C, 4, 4>(logits, topk_weights, topk_indices, num_tokens, n, kk, rn, st);
+    const bool waves = C::VEC == 8 && n > 12 * kSoftmaxLanes && num_tokens < kWideFew;
+    if (small_grid && !waves) {
+      switch ((n + kSoftmaxLanes - 1) / kSoftmaxLanes) {
+        case 2: return groups(IntC<16>{}, IntC<2>{});
+        case 3: return groups(IntC<16>{}, IntC<3>{});
+        case 4: return groups(IntC<16>{}, IntC<4>{});
+        case 5:
+        case 6: return groups(IntC<16>{}, IntC<6>{});
+        case 7:
+        case 8: return groups(IntC<16>{}, IntC<8>{});
+        case 9:
+        case 10: return groups(IntC<16>{}, IntC<10>{});
+        case 11:
+        case 12: return groups(IntC<16>{}, IntC<12>{});
+        default: return groups(IntC<16>{}, IntC<16>{});
       }
-      return launch_status();
     }
     moe_router_waves<C><<<flat_grid(num_tokens, kWavesPerGroup, kMaxRowGroups), 256, 0, st>>>(
         logits, topk_weights, topk_indices, num_tokens, n, kk, rn);
