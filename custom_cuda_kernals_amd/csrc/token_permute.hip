@@ -692,7 +692,8 @@ __device__ inline uint32_t lanes_below(uint64_t m) {
 }
 
 __device__ inline int perm_bucket(int64_t id, int n_experts) {
-  return (id >= 0 && id < n_experts) ? (int)id : n_experts;
+  const uint32_t lo = (uint32_t)id, hi = (uint32_t)((uint64_t)id >> 32);
+  return hi == 0u ? (int)min(lo, (uint32_t)n_experts) : n_experts;
 }
 
 // hist[key] += 1 for every active lane, in one LDS atomic per wave. The lanes
@@ -718,12 +719,15 @@ __device__ inline void perm_bases(const uint32_t* after, const uint32_t* before,
     loc[i] = b < nb ? before[b] + after[b] : 0u;
     sum += loc[i];
   }
+  // Inclusive scan over the wave: within each row of 16 lanes, then row 0's
+  // total into row 1 and row 2's into row 3, then rows 0-1's into rows 2 and 3.
   uint32_t incl = sum;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t o = __shfl_up(incl, d);
-    if (lane >= d) incl += o;
-  }
+  incl += dpp<0x111>(incl);  // row_shr:1, 2, 4, 8 (0 past the row's start)
+  incl += dpp<0x112>(incl);
+  incl += dpp<0x114>(incl);
+  incl += dpp<0x118>(incl);
+  incl += dpp_rows<kDppRowBcast15, 0xA>(0u, incl);
+  incl += dpp_rows<kDppRowBcast31, 0xC>(0u, incl);
   uint32_t run = incl - sum;
 #pragma unroll
   for (int i = 0; i < kPermPerLane; ++i) {
@@ -733,15 +737,36 @@ __device__ inline void perm_bases(const uint32_t* after, const uint32_t* before,
   }
 }
 
-// Stable ranking of the entries [c0, c1) from base[]: per tile, every lane
-// ORs its lane bit into its wave's mask of its bucket; the bits below a lane
-// in its own mask rank it among the wave's lanes of the same bucket, the
-// popcounts of the lower waves' masks offset it, so ties keep index order; a
-// running count per bucket carries the order from tile to tile.
-// lane_mask must be zero on entry and is zero on return.
+// Stable ranking of the entries [c0, c1) from base[]: per tile, every lane ORs
+// its lane bit into its wave's mask of its bucket and reads the mask back (LDS
+// accesses of one wave complete in order); the bits below a lane rank it among
+// the wave's lanes of that bucket, and the first of them stores their count and
+// clears the mask. One thread per bucket then turns the 16 waves' counts into
+// positions, in wave order, so ties keep index order, and carries base[] to the
+// next tile. masks and counts must be zero on entry. `id` is this thread's
+// entry of the first tile (ids[c0 + tid], loaded by the caller ahead of its
+// other work). Against every lane summing the lower waves' mask popcounts for
+// itself, graph-replayed on MI355X: 4096 tokens x 6 of 160 7.8 vs 7.6 us, 512 x 2 of 8
+// 4.6 vs 4.2, 8000 x 8 of 256 12.9 vs 12.5, three launches 16384 x 8 14.4 vs 13.5. What
+// is left of the one-launch form is the count of all n ids by every workgroup
+// (id loads at 64 bytes a clock and one LDS atomic each); counting by 16-byte pairs
+// of ids, or with the next ids loaded before the atomics, measured 9.1 and 8.1.
+struct PermTile {
+  unsigned long long mask[kPermWaves][kPermBuckets];
+  uint32_t count[kPermWaves][kPermBuckets];
+  // Cleared by the whole workgroup; a barrier must follow.
+  __device__ void clear_counts() {
+    for (int i = threadIdx.x; i < kPermWaves * kPermBuckets; i += kPermThreads) (&count[0][0])[i] = 0u;
+  }
+  __device__ void clear() {
+    for (int i = threadIdx.x; i < kPermWaves * kPermBuckets; i += kPermThreads) (&mask[0][0])[i] = 0ull;
+    clear_counts();
+  }
+};
+
 template <bool kWritePermute>
-__device__ inline void perm_rank_chunk(const int64_t* __restrict__ ids, int64_t k, int n_experts, int64_t c0,
-                                       int64_t c1, uint32_t* base, unsigned long long (*lane_mask)[kPermBuckets],
+__device__ inline void perm_rank_chunk(const int64_t* __restrict__ ids, int64_t id, int64_t k, int n_experts,
+                                       int64_t c0, int64_t c1, uint32_t* base, PermTile& tile,
                                        int64_t* __restrict__ permute_index, int64_t* __restrict__ unpermute_index) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -749,27 +774,43 @@ __device__ inline void perm_rank_chunk(const int64_t* __restrict__ ids, int64_t 
   for (int64_t t0 = c0; t0 < c1; t0 += kPermThreads) {
     const int64_t j = t0 + tid;
     const bool valid = j < c1;
-    const int b = valid ? perm_bucket(ids[j], n_experts) : 0;
-    if (valid) atomicOr(&lane_mask[wave][b], 1ull << lane);
-    __syncthreads();
-    if (valid) {
-      uint32_t pos = base[b] + lanes_below(lane_mask[wave][b]);
-      for (int w = 0; w < wave; ++w) pos += (uint32_t)__popcll(lane_mask[w][b]);
-      if constexpr (kWritePermute) permute_index[pos] = j / k;
-      unpermute_index[j] = pos;
+    if (t0 != c0) {
+      __syncthreads();  // the previous tile's positions have been read
+      tile.clear_counts();
+      if (valid) id = ids[j];
+      __syncthreads();
     }
+    const int b = valid ? perm_bucket(id, n_experts) : 0;
+    uint32_t below = 0u;
+    if (valid) atomicOr(&tile.mask[wave][b], 1ull << lane);
+    __builtin_amdgcn_wave_barrier();
+    if (valid) {
+      const unsigned long long m = __hip_atomic_load(&tile.mask[wave][b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      below = lanes_below(m);
+      if (below == 0u) tile.count[wave][b] = (uint32_t)__popcll(m);
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (valid && below == 0u) tile.mask[wave][b] = 0ull;
     __syncthreads();
-    // Carry this tile's counts into base and clear the masks for the next tile.
-    for (int i = tid; i < nb; i += kPermThreads) {
-      uint32_t c = 0u;
+    if (tid < nb) {
+      uint32_t c[kPermWaves];
+#pragma unroll
+      for (int w = 0; w < kPermWaves; ++w) c[w] = tile.count[w][tid];
+      uint32_t run = base[tid];
 #pragma unroll
       for (int w = 0; w < kPermWaves; ++w) {
-        c += (uint32_t)__popcll(lane_mask[w][i]);
-        lane_mask[w][i] = 0ull;
+        tile.count[w][tid] = run;
+        run += c[w];
       }
-      base[i] += c;
+      base[tid] = run;
     }
     __syncthreads();
+    if (valid) {
+      const uint32_t pos = tile.count[wave][b] + below;
+      // Entries are below 2^31 (the launcher's bound), so the token is a 32-bit quotient.
+      if constexpr (kWritePermute) permute_index[pos] = (int64_t)((uint32_t)j / (uint32_t)k);
+      unpermute_index[j] = pos;
+    }
   }
 }
 
@@ -789,30 +830,32 @@ __global__ __launch_bounds__(kPermThreads) void moe_permutation(const int64_t* _
                                                                 int64_t* __restrict__ unpermute_index) {
   // before = sides[0], after = sides[1]
   __shared__ uint32_t sides[2 * kPermBuckets], base[kPermBuckets];
-  __shared__ unsigned long long lane_mask[kPermWaves][kPermBuckets];
+  __shared__ PermTile tile;
   uint32_t* before = sides;
   uint32_t* after = sides + kPermBuckets;
   const int tid = threadIdx.x;
   const int nb = n_experts + 1;
-  for (int i = tid; i < 2 * kPermBuckets; i += kPermThreads) sides[i] = 0u;
-  for (int i = tid; i < kPermWaves * kPermBuckets; i += kPermThreads) (&lane_mask[0][0])[i] = 0ull;
-  __syncthreads();
   const int64_t c0 = (int64_t)blockIdx.x * chunk;
   const int64_t c1 = c0 + chunk < n ? c0 + chunk : n;
+  const int64_t own = c0 + tid < c1 ? ids[c0 + tid] : 0;  // the first ranked tile's entry
+  for (int i = tid; i < 2 * kPermBuckets; i += kPermThreads) sides[i] = 0u;
+  tile.clear();
+  __syncthreads();
   // kPermUnroll ids per thread in flight before their LDS atomics (one DRAM
   // round trip per kPermUnroll ids instead of per id).
-  for (int64_t j0 = tid; j0 < n; j0 += (int64_t)kPermThreads * kPermUnroll) {
+  const int total = (int)n;
+  for (int j0 = tid; j0 < total; j0 += kPermThreads * kPermUnroll) {
     int64_t v[kPermUnroll];
 #pragma unroll
     for (int u = 0; u < kPermUnroll; ++u) {
-      const int64_t j = j0 + (int64_t)u * kPermThreads;
-      v[u] = j < n ? ids[j] : 0;
+      const int j = j0 + u * kPermThreads;
+      v[u] = j < total ? ids[j] : 0;
     }
 #pragma unroll
     for (int u = 0; u < kPermUnroll; ++u) {
-      const int64_t j = j0 + (int64_t)u * kPermThreads;
-      if (j < n) {
-        const int key = perm_bucket(v[u], n_experts) + (j < c0 ? 0 : kPermBuckets);
+      const int j = j0 + u * kPermThreads;
+      if (j < total) {
+        const int key = perm_bucket(v[u], n_experts) + (j < (int)c0 ? 0 : kPermBuckets);
         if constexpr (kCombine) {
           perm_count(sides, key);
         } else {
@@ -824,7 +867,7 @@ __global__ __launch_bounds__(kPermThreads) void moe_permutation(const int64_t* _
   __syncthreads();
   if (tid < 64) perm_bases(after, before, base, nb, tid);
   __syncthreads();
-  perm_rank_chunk<true>(ids, k, n_experts, c0, c1, base, lane_mask, permute_index, unpermute_index);
+  perm_rank_chunk<true>(ids, own, k, n_experts, c0, c1, base, tile, permute_index, unpermute_index);
 }
 
 // Three launches from kPermSplitMin entries on, so that each id is counted
@@ -876,14 +919,17 @@ __global__ __launch_bounds__(kPermThreads) void moe_permutation_rank(const int64
                                                                      const uint32_t* __restrict__ counts,
                                                                      int64_t* __restrict__ unpermute_index) {
   __shared__ uint32_t after[kPermBuckets], before[kPermBuckets], base[kPermBuckets];
-  __shared__ unsigned long long lane_mask[kPermWaves][kPermBuckets];
+  __shared__ PermTile tile;
   const int tid = threadIdx.x;
   const int nb = n_experts + 1;
+  const int64_t c0 = (int64_t)blockIdx.x * chunk;
+  const int64_t c1 = c0 + chunk < n ? c0 + chunk : n;
+  const int64_t own = c0 + tid < c1 ? ids[c0 + tid] : 0;  // the first tile's entry
   for (int i = tid; i < nb; i += kPermThreads) {
     after[i] = 0u;
     before[i] = 0u;
   }
-  for (int i = tid; i < kPermWaves * kPermBuckets; i += kPermThreads) (&lane_mask[0][0])[i] = 0ull;
+  tile.clear();
   __syncthreads();
   // counts[g][b] for every chunk g: flat index i = g * nb + b, coalesced
   // (at most kPermSplitMaxGroups x kPermBuckets of them, so 32-bit).
@@ -904,9 +950,7 @@ __global__ __launch_bounds__(kPermThreads) void moe_permutation_rank(const int64
   __syncthreads();
   if (tid < 64) perm_bases(after, before, base, nb, tid);
   __syncthreads();
-  const int64_t c0 = (int64_t)blockIdx.x * chunk;
-  const int64_t c1 = c0 + chunk < n ? c0 + chunk : n;
-  perm_rank_chunk<false>(ids, k, n_experts, c0, c1, base, lane_mask, nullptr, unpermute_index);
+  perm_rank_chunk<false>(ids, own, k, n_experts, c0, c1, base, tile, nullptr, unpermute_index);
 }
 
 __global__ __launch_bounds__(256) void moe_permutation_invert(const int64_t* __restrict__ unpermute_index, int64_t n,
