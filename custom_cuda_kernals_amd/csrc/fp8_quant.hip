@@ -875,7 +875,14 @@ int onepass_groups() {
 // 9.58 against 11.67 / 9.92; [4096, 4096] 14.83 / 12.92 against 18.52 /
 // 16.67; [8192, 4096] 24.04 / 22.12 against 29.66 / 27.76.
 constexpr int64_t kOnePassMinVecs = int64_t(1) << 20;
-constexpr int64_t kOnePassSoloVecs = (int64_t)kOnePassThreads * 2;  // one workgroup: no exchange
+// One workgroup, no exchange and no second launch, up to this many vectors: where
+// its one CU's time reaches that of the two launches' grids. Graph-replayed on
+// MI355X, one workgroup vs two launches, bf16 3072 vectors 3.5 vs 4.4 us, 4096 3.9 vs
+// 4.7, 6144 5.2 vs 4.8, 8192 6.4 vs 4.7; fp32 4096 3.1 vs 4.5, 6144 4.0 vs 4.5, 8192 5.0 vs
+// 4.6. Called one by one through the Python API the second launch costs 3.5 us
+// of host time more.
+template <class C>
+constexpr int64_t kOnePassSoloVecs = (int64_t)kOnePassThreads * (C::VEC == 8 ? 4 : 6);
 
 // Launches the one-pass form where it pays: inputs one workgroup holds
 // (no exchange and no init launch: the fewest vectors per thread that
@@ -887,13 +894,13 @@ constexpr int64_t kOnePassSoloVecs = (int64_t)kOnePassThreads * 2;  // one workg
 template <class C, int FMT>
 bool launch_onepass(const void* x, uint8_t* q, float* scale, int32_t* amax_scratch, int64_t nvec,
                     hipStream_t st) {
-  if (nvec > kOnePassSoloVecs && nvec < kOnePassMinVecs) return false;
+  if (nvec > kOnePassSoloVecs<C> && nvec < kOnePassMinVecs) return false;
   const int polls = poll_limit.load(std::memory_order_relaxed);
   auto attempt = [&](auto u, auto wpe) {
     constexpr int U = decltype(u)::value, WPE = decltype(wpe)::value;
     constexpr int64_t per_group = (int64_t)kOnePassThreads * U;
     const int64_t g = (nvec + per_group - 1) / per_group;
-    if (nvec <= kOnePassSoloVecs ? g > 1 : (g > onepass_groups<C, FMT, U, WPE>() || 4 * g > per_group * C::VEC)) {
+    if (nvec <= kOnePassSoloVecs<C> ? g > 1 : (g > onepass_groups<C, FMT, U, WPE>() || 4 * g > per_group * C::VEC)) {
       return false;
     }
     if (g > 1) {
@@ -907,7 +914,7 @@ bool launch_onepass(const void* x, uint8_t* q, float* scale, int32_t* amax_scrat
       attempt(IntC<16>{}, IntC<4>{})) {
     return true;
   }
-  if (nvec <= kOnePassSoloVecs) return false;
+  if (nvec <= kOnePassSoloVecs<C>) return false;
   // Beyond what the grid holds: every resident workgroup takes an equal
   // chunk, 16 vectors per thread of it in registers and the rest streamed.
   constexpr int U = 16, WPE = 4;
