@@ -21,15 +21,23 @@
 namespace cck {
 namespace {
 
+template <class C>
+__device__ inline float swiglu1(float g, float u) {
+  return C::round(silu_one<C>(g)) * u;
+}
+
 // The plain op: a grid-stride stream of 16-byte vectors, UNROLL per thread
 // per step, the next step's loads issued before this step's math. It uses the
 // arithmetic SiLU for every dtype: with the LDS table (and its per-workgroup
 // fill) the bf16 stream measured slower on MI355X (111.4 vs 109.9 us at
-// 8192 x 14336, 233.8 vs 218.8 us at 16384 x 14336).
+// 8192 x 14336, 233.8 vs 218.8 us at 16384 x 14336). The last workgroup also takes
+// the `tail` elements past the last vector: in a launch of their own they cost 1.6
+// us more (graph-replayed on MI355X, bf16 [301, 11007] 6.8 vs 5.5 us, [33, 101] 3.7 vs
+// 2.0, static-scale FP8 [301, 5461] 6.4 vs 4.9) and 3.5 us of a call's host time.
 template <class C, int THREADS, int UNROLL>
 __global__ __launch_bounds__(THREADS) void swiglu_flat(const u32x4* __restrict__ gate,
                                                        const u32x4* __restrict__ up,
-                                                       u32x4* __restrict__ y, int64_t nvec) {
+                                                       u32x4* __restrict__ y, int64_t nvec, int tail) {
   const int64_t stride = (int64_t)gridDim.x * THREADS * UNROLL;
   int64_t base = (int64_t)blockIdx.x * THREADS * UNROLL + threadIdx.x;
   u32x4 g[UNROLL], u[UNROLL];
@@ -59,11 +67,10 @@ __global__ __launch_bounds__(THREADS) void swiglu_flat(const u32x4* __restrict__
     }
     load(base + stride);
   }
-}
-
-template <class C>
-__device__ inline float swiglu1(float g, float u) {
-  return C::round(silu_one<C>(g)) * u;
+  if (blockIdx.x == gridDim.x - 1 && (int)threadIdx.x < tail) {
+    const int64_t i = nvec * C::VEC + threadIdx.x;
+    C::store1(y, i, swiglu1<C>(C::load1(gate, i), C::load1(up, i)));
+  }
 }
 
 template <class C>
@@ -76,6 +83,15 @@ __global__ __launch_bounds__(256) void swiglu_scalar(const void* __restrict__ ga
   }
 }
 
+// One element of the static-scale FP8 variant.
+template <class C, int FMT>
+__device__ inline void swiglu_fp8_static1(const void* gate, const void* up, uint8_t* yq, float s, float r, int64_t i) {
+  const float yv = C::round(swiglu1<C>(C::load1(gate, i), C::load1(up, i)));
+  const bool fast = fast_path_ok<FMT>(s, r, __builtin_fabsf(yv));
+  const float qv = fast ? div_by_scale(yv, s, r) : div_x86(yv, s);
+  yq[i] = (uint8_t)(fast ? (Fp8<FMT>::cvt4(qv, 0.0f, 0.0f, 0.0f) & 0xffu) : Fp8<FMT>::encode(qv));
+}
+
 // Static-scale FP8 variant: no row reduction is needed, so it streams like
 // swiglu_flat; each 16-byte vector takes the fast conversion when its own
 // max |y| * (1/s) is inside the fast range, the exact path otherwise. The
@@ -85,7 +101,8 @@ template <class C, int FMT, int THREADS, int UNROLL, bool TAB>
 __global__ __launch_bounds__(THREADS) void swiglu_fp8_static_flat(const u32x4* __restrict__ gate,
                                                                  const u32x4* __restrict__ up,
                                                                  uint8_t* __restrict__ yq, float s,
-                                                                 int64_t nvec, float* __restrict__ scale_out) {
+                                                                 int64_t nvec, int tail,
+                                                                 float* __restrict__ scale_out) {
   constexpr int VEC = C::VEC;
   if (scale_out != nullptr && blockIdx.x == 0 && threadIdx.x == 0) scale_out[0] = s;
   __shared__ __attribute__((aligned(16))) float tab[TAB ? SiluTableBF16::kEntries : 1];
@@ -140,6 +157,10 @@ __global__ __launch_bounds__(THREADS) void swiglu_fp8_static_flat(const u32x4* _
     }
     load(base + stride);
   }
+  // The elements past the last vector, as in swiglu_flat.
+  if (blockIdx.x == gridDim.x - 1 && (int)threadIdx.x < tail) {
+    swiglu_fp8_static1<C, FMT>(gate, up, yq, s, r, nvec * VEC + threadIdx.x);
+  }
 }
 
 template <class C, int FMT>
@@ -152,10 +173,7 @@ __global__ __launch_bounds__(256) void swiglu_fp8_static_scalar(const void* __re
   const float r = 1.0f / s;
   const int64_t stride = (int64_t)gridDim.x * 256;
   for (int64_t i = begin + (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
-    const float yv = C::round(swiglu1<C>(C::load1(gate, i), C::load1(up, i)));
-    const bool fast = fast_path_ok<FMT>(s, r, __builtin_fabsf(yv));
-    const float qv = fast ? div_by_scale(yv, s, r) : div_x86(yv, s);
-    yq[i] = (uint8_t)(fast ? (Fp8<FMT>::cvt4(qv, 0.0f, 0.0f, 0.0f) & 0xffu) : Fp8<FMT>::encode(qv));
+    swiglu_fp8_static1<C, FMT>(gate, up, yq, s, r, i);
   }
 }
 
@@ -485,9 +503,9 @@ extern "C" int32_t launch_swiglu_fwd(const void* gate, const void* up, void* y, 
         constexpr int THREADS = 512, UNROLL = 2;
         swiglu_flat<C, THREADS, UNROLL>
             <<<flat_grid((nvec + UNROLL - 1) / UNROLL, THREADS, 1 << 20), THREADS, kLdsForGroupsPerCu<3>, st>>>(
-                g4, u4, y4, nvec);
+                g4, u4, y4, nvec, (int)(n % C::VEC));
+        done = n;
       }
-      done = nvec * C::VEC;
     }
     if (done < n) {
       swiglu_scalar<C><<<flat_grid(n - done, 256, 4096), 256, 0, st>>>(gate, up, y, done, n);
@@ -523,18 +541,18 @@ extern "C" int32_t launch_swiglu_fp8_fwd(const void* gate, const void* up, uint8
           if (nvec >= kTabMinVec) {
             constexpr int kPer = kTabThreads * kTabUnroll;
             swiglu_fp8_static_flat<C, FMT, kTabThreads, kTabUnroll, true>
-                <<<flat_grid((nvec + kPer - 1) / kPer, 1, 1 << 20), kTabThreads, 0, st>>>(g4, u4, y_fp8,
-                                                                                          static_scale, nvec, scale);
+                <<<flat_grid((nvec + kPer - 1) / kPer, 1, 1 << 20), kTabThreads, 0, st>>>(
+                    g4, u4, y_fp8, static_scale, nvec, (int)(n % C::VEC), scale);
             tab = true;
           }
         }
         if (!tab && nvec > 0) {
           constexpr int UNROLL = 4;
           swiglu_fp8_static_flat<C, FMT, 256, UNROLL, false>
-              <<<flat_grid((nvec + UNROLL - 1) / UNROLL, 256, 1 << 20), 256, 0, st>>>(g4, u4, y_fp8, static_scale,
-                                                                                      nvec, scale);
+              <<<flat_grid((nvec + UNROLL - 1) / UNROLL, 256, 1 << 20), 256, 0, st>>>(
+                  g4, u4, y_fp8, static_scale, nvec, (int)(n % C::VEC), scale);
         }
-        done = nvec * C::VEC;
+        if (nvec > 0) done = n;
       }
       if (done < n) {
         swiglu_fp8_static_scalar<C, FMT><<<flat_grid(n - done, 256, 4096), 256, 0, st>>>(gate, up, y_fp8, static_scale,

@@ -204,3 +204,37 @@ def test_combine(dtype, k):
             native.token_combine_fwd(_off(eo, offset), ui.cuda(), w.cuda(), out.t)
             assert bits_equal(out.t, moe.token_combine_aten(eo, ui_ref, w_ref)).all(), (t, h)
             out.check()
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).split(".")[-1])
+def test_flat_swiglu_tails(dtype):
+    """The elements past the last vector, plain and static-scale FP8: every
+    remainder after one vector, after one workgroup's vectors and in the
+    SiLU-table stream."""
+    vec = 16 // dtype.itemsize
+    for n in [vec + d for d in range(vec)] + [1024 * vec + d for d in (1, vec - 1)] + [(1 << 17) * vec + 3]:
+        g, u = inputs.swiglu_inputs(1, n, dtype, seed=n)
+        y, q = Guarded(g.shape, dtype, 0), Guarded(g.shape, F8["e4m3"], 0)
+        s = torch.empty(1, dtype=torch.float32, device="cuda")
+        native.swiglu_fwd(g.cuda(), u.cuda(), y.t)
+        native.swiglu_fp8_fwd(g.cuda(), u.cuda(), q.t, s, "e4m3", 0.05)
+        y_ref = eager.swiglu(g, u)
+        assert bits_equal(y.t, y_ref).all(), n
+        assert_codes_equal(q.t, ofp8.quant_static(y_ref.float().numpy(), 0.05, "e4m3"))
+        y.check()
+        q.check()
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).split(".")[-1])
+def test_fp8_tensor_one_workgroup_edge(dtype):
+    """Per-tensor FP8 either side of what one workgroup takes whole."""
+    vec = 16 // dtype.itemsize
+    for nvec in (2048, 2049, 4096, 4097, 6144, 6145):
+        x = inputs.randn((nvec, vec), dtype, seed=nvec)
+        q = Guarded(x.shape, F8["e5m2"], 0)
+        s = torch.empty(1, dtype=torch.float32, device="cuda")
+        native.fp8_quant_tensor_fwd(x.cuda(), q.t, s, None, "e5m2")
+        codes, s_ref = ofp8.quant_tensor(x.float().numpy(), "e5m2")
+        assert_codes_equal(q.t, codes)
+        assert_f32_bits_equal(s, np.asarray(s_ref).reshape(1))
+        q.check()
