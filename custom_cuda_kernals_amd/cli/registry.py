@@ -331,9 +331,9 @@ REGISTRY: dict[str, OpSpec] = {
             dtypes=("float32", "float16", "bfloat16"),
             memory_profile="latency-bound (1.3 MB at 2048 x 160).",
             design=("E <= 8: one lane per token, every step serial in its registers",
-                    "9..32 experts (up to 64 from 4096 tokens): four lanes per token over 16-expert stripes",
-                    "65..256 experts from 8192 / 12288 tokens: eight lanes per token",
-                    "otherwise one wave per token, 4 experts per lane; wave arg-max per selection"),
+                    "9..16 experts: four lanes per token over 16-expert stripes",
+                    "17 experts up: 16 lanes per token (eight for up to 64 experts of many tokens)",
+                    "16-bit rows of over 192 experts below 2048 tokens: one wave per token"),
             target="weights bit-exact against torch-CPU; indices equal the oracle's (exact ties aside)",
             reference=("baselines/moe_router.py:117-128", "csrc/kernels/moe_router.cu",
                        "csrc/includes/moe_router.h:20-29"),
