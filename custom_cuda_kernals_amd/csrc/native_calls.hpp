@@ -85,8 +85,12 @@ inline int64_t int_arg(PyObject* o, int64_t most) {
   return overflow == 0 && v >= 1 && v <= most ? (int64_t)v : -1;
 }
 
+// Without the interpreter lock, as torch.empty: an allocation may have to wait
+// for the GPU, whose work may wait for another Python thread.
 inline at::Tensor empty(c10::IntArrayRef sizes, c10::ScalarType type, const at::Tensor& like) {
-  return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
+  const auto options = at::TensorOptions().dtype(type).device(like.device());
+  const py::gil_scoped_release unlocked;
+  return at::empty(sizes, options);
 }
 
 inline bool same(const at::Tensor& a, const at::Tensor& b) {
