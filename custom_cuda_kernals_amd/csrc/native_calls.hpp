@@ -21,6 +21,7 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/util/DimVector.h>
 #include <torch/csrc/Exceptions.h>
 
 namespace {
@@ -51,9 +52,49 @@ inline const at::Tensor* plain(PyObject* o) {
   return t.is_contiguous() && t.numel() > 0 ? &t : nullptr;
 }
 
+// A plain input as the checks saw it: what they compare and the outputs are
+// sized by is this copy, since another Python thread may set the tensor's data
+// whenever the interpreter lock is not held. (Operators that change a tensor
+// without the lock, as set_ and resize_, race with any reader of it.)
+class Input {
+ public:
+  explicit Input(PyObject* o) : object_(o), t_(plain(o)) {
+    if (t_ == nullptr) return;
+    sizes_ = t_->sizes();
+    type_ = t_->scalar_type();
+    device_ = t_->device();
+  }
+  explicit operator bool() const { return t_ != nullptr; }
+  // The tensor still is what the checks saw.
+  bool unchanged() const {
+    return plain(object_) == t_ && t_->sizes() == sizes() && t_->scalar_type() == type_ && t_->device() == device_;
+  }
+  const at::Tensor& tensor() const { return *t_; }
+  // For the launch, in the hold of the lock of the last look at the tensor.
+  void* data() const { return t_->data_ptr(); }
+  c10::IntArrayRef sizes() const { return sizes_; }
+  int64_t dim() const { return (int64_t)sizes_.size(); }
+  int64_t size(int64_t i) const { return sizes_[i < 0 ? i + sizes_.size() : i]; }
+  int64_t numel() const { return c10::multiply_integers(sizes_); }
+  c10::ScalarType type() const { return type_; }
+  c10::Device device() const { return device_; }
+
+ private:
+  PyObject* object_;
+  const at::Tensor* t_;
+  c10::DimVector sizes_;
+  c10::ScalarType type_ = c10::ScalarType::Undefined;
+  c10::Device device_ = c10::kCPU;
+};
+
+template <class... In>
+inline bool unchanged(const In&... in) {
+  return (in.unchanged() && ...);
+}
+
 // The tag of a float32 / float16 / bfloat16 tensor, -1 otherwise.
-inline int32_t float_tag(const at::Tensor& t) {
-  const int32_t tag = tag_of(t.scalar_type());
+inline int32_t float_tag(const Input& t) {
+  const int32_t tag = tag_of(t.type());
   return tag == F32 || tag == F16 || tag == BF16 ? tag : -1;
 }
 
@@ -85,16 +126,25 @@ inline int64_t int_arg(PyObject* o, int64_t most) {
   return overflow == 0 && v >= 1 && v <= most ? (int64_t)v : -1;
 }
 
+struct Output {
+  c10::IntArrayRef sizes;
+  c10::ScalarType type;
+};
+inline Output like(const Input& t) { return {t.sizes(), t.type()}; }
+
 // Without the interpreter lock, as torch.empty: an allocation may have to wait
-// for the GPU, whose work may wait for another Python thread.
-inline at::Tensor empty(c10::IntArrayRef sizes, c10::ScalarType type, const at::Tensor& like) {
-  const auto options = at::TensorOptions().dtype(type).device(like.device());
+// for the GPU, whose work may wait for another Python thread. Sizes are the
+// caller's copies. The inputs must be looked at again afterwards.
+template <size_t N>
+inline void allocate(c10::Device device, const Output (&wanted)[N], at::Tensor (&out)[N]) {
   const py::gil_scoped_release unlocked;
-  return at::empty(sizes, options);
+  for (size_t i = 0; i < N; ++i) {
+    out[i] = at::empty(wanted[i].sizes, at::TensorOptions().dtype(wanted[i].type).device(device));
+  }
 }
 
-inline bool same(const at::Tensor& a, const at::Tensor& b) {
-  return a.scalar_type() == b.scalar_type() && a.device() == b.device() && a.sizes() == b.sizes();
+inline bool same(const Input& a, const Input& b) {
+  return a.type() == b.type() && a.device() == b.device() && a.sizes() == b.sizes();
 }
 
 template <class... T>
@@ -113,20 +163,26 @@ inline PyObject* result(T... t) {
 inline PyObject* rmsnorm_residual(PyObject*, PyArgs a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 4 || !PyFloat_CheckExact(a[3]) || !ordinary_state()) Py_RETURN_NONE;
-  const at::Tensor *x = plain(a[0]), *r = plain(a[1]), *w = plain(a[2]);
-  if (!x || !r || !w || float_tag(*x) < 0 || !same(*x, *r) || x->dim() < 1) Py_RETURN_NONE;
-  const int64_t cols = x->size(-1);
-  if (w->dim() != 1 || w->size(0) != cols || w->scalar_type() != x->scalar_type() || w->device() != x->device()) {
-    Py_RETURN_NONE;
-  }
-  const Launch launch(x->device().index());
-  at::Tensor y = empty(x->sizes(), x->scalar_type(), *x), ro = empty(x->sizes(), x->scalar_type(), *x);
+  const Input x(a[0]), r(a[1]), w(a[2]);
+  if (!x || !r || !w || float_tag(x) < 0 || !same(x, r) || x.dim() < 1) Py_RETURN_NONE;
+  const int64_t cols = x.size(-1);
+  if (w.dim() != 1 || w.size(0) != cols || w.type() != x.type() || w.device() != x.device()) Py_RETURN_NONE;
+  const Launch launch(x.device().index());
+  at::Tensor out[2];
+  allocate(x.device(), {like(x), like(x)}, out);
+  if (!unchanged(x, r, w)) Py_RETURN_NONE;
   check_launch("launch_rmsnorm_residual_fwd",
-               launch_rmsnorm_residual_fwd(x->data_ptr(), r->data_ptr(), w->data_ptr(), y.data_ptr(), ro.data_ptr(),
-                                           x->numel() / cols, cols, (float)PyFloat_AS_DOUBLE(a[3]), float_tag(*x),
+               launch_rmsnorm_residual_fwd(x.data(), r.data(), w.data(), out[0].data_ptr(), out[1].data_ptr(),
+                                           x.numel() / cols, cols, (float)PyFloat_AS_DOUBLE(a[3]), float_tag(x),
                                            launch.st));
-  return result(std::move(y), std::move(ro));
+  return result(std::move(out[0]), std::move(out[1]));
   END_HANDLE_TH_ERRORS
+}
+
+// The scale tensor of the fused FP8 calls: one scale a row of x, or one.
+constexpr int64_t kOne[1] = {1};
+inline Output scales_of(const Input& x, bool is_static) {
+  return {is_static ? c10::IntArrayRef(kOne) : x.sizes().slice(0, x.dim() - 1), c10::ScalarType::Float};
 }
 
 // (x, residual, weight, eps, fp8_format, scale)
@@ -138,23 +194,21 @@ inline PyObject* rmsnorm_residual_fp8(PyObject*, PyArgs a, Py_ssize_t n) {
     Py_RETURN_NONE;
   }
   const int32_t fmt = fmt_tag(a[4]);
-  const at::Tensor *x = plain(a[0]), *r = plain(a[1]), *w = plain(a[2]);
-  if (fmt < 0 || !x || !r || !w || float_tag(*x) < 0 || !same(*x, *r) || x->dim() < 1) Py_RETURN_NONE;
-  const int64_t cols = x->size(-1), rows = x->numel() / cols;
-  if (w->dim() != 1 || w->size(0) != cols || w->scalar_type() != x->scalar_type() || w->device() != x->device()) {
-    Py_RETURN_NONE;
-  }
-  const Launch launch(x->device().index());
-  at::Tensor q = empty(x->sizes(), fp8_type(fmt), *x), ro = empty(x->sizes(), x->scalar_type(), *x);
-  at::Tensor s = is_static ? empty({1}, c10::ScalarType::Float, *x)
-                           : empty(x->sizes().slice(0, x->dim() - 1), c10::ScalarType::Float, *x);
+  const Input x(a[0]), r(a[1]), w(a[2]);
+  if (fmt < 0 || !x || !r || !w || float_tag(x) < 0 || !same(x, r) || x.dim() < 1) Py_RETURN_NONE;
+  const int64_t cols = x.size(-1);
+  if (w.dim() != 1 || w.size(0) != cols || w.type() != x.type() || w.device() != x.device()) Py_RETURN_NONE;
+  const Launch launch(x.device().index());
+  at::Tensor out[3];
+  allocate(x.device(), {{x.sizes(), fp8_type(fmt)}, scales_of(x, is_static), like(x)}, out);
+  if (!unchanged(x, r, w)) Py_RETURN_NONE;
   check_launch("launch_rmsnorm_residual_fp8_fwd",
-               launch_rmsnorm_residual_fp8_fwd(x->data_ptr(), r->data_ptr(), w->data_ptr(), (uint8_t*)q.data_ptr(),
-                                               (float*)s.data_ptr(), ro.data_ptr(), rows, cols,
+               launch_rmsnorm_residual_fp8_fwd(x.data(), r.data(), w.data(), (uint8_t*)out[0].data_ptr(),
+                                               (float*)out[1].data_ptr(), out[2].data_ptr(), x.numel() / cols, cols,
                                                (float)PyFloat_AS_DOUBLE(a[3]), value,
-                                               is_static ? CCK_SCALE_STATIC : CCK_SCALE_TOKEN, float_tag(*x), fmt,
+                                               is_static ? CCK_SCALE_STATIC : CCK_SCALE_TOKEN, float_tag(x), fmt,
                                                launch.st));
-  return result(std::move(q), std::move(s), std::move(ro));
+  return result(std::move(out[0]), std::move(out[1]), std::move(out[2]));
   END_HANDLE_TH_ERRORS
 }
 
@@ -162,13 +216,15 @@ inline PyObject* rmsnorm_residual_fp8(PyObject*, PyArgs a, Py_ssize_t n) {
 inline PyObject* swiglu(PyObject*, PyArgs a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 2 || !ordinary_state()) Py_RETURN_NONE;
-  const at::Tensor *g = plain(a[0]), *u = plain(a[1]);
-  if (!g || !u || float_tag(*g) < 0 || !same(*g, *u)) Py_RETURN_NONE;
-  const Launch launch(g->device().index());
-  at::Tensor y = empty(g->sizes(), g->scalar_type(), *g);
-  check_launch("launch_swiglu_fwd", launch_swiglu_fwd(g->data_ptr(), u->data_ptr(), y.data_ptr(), g->numel(),
-                                                      float_tag(*g), launch.st));
-  return result(std::move(y));
+  const Input g(a[0]), u(a[1]);
+  if (!g || !u || float_tag(g) < 0 || !same(g, u)) Py_RETURN_NONE;
+  const Launch launch(g.device().index());
+  at::Tensor out[1];
+  allocate(g.device(), {like(g)}, out);
+  if (!unchanged(g, u)) Py_RETURN_NONE;
+  check_launch("launch_swiglu_fwd",
+               launch_swiglu_fwd(g.data(), u.data(), out[0].data_ptr(), g.numel(), float_tag(g), launch.st));
+  return result(std::move(out[0]));
   END_HANDLE_TH_ERRORS
 }
 
@@ -179,18 +235,18 @@ inline PyObject* swiglu_fp8(PyObject*, PyArgs a, Py_ssize_t n) {
   float value = 0.0f;
   if (n != 4 || !scale_arg(a[3], &is_static, &value) || !ordinary_state()) Py_RETURN_NONE;
   const int32_t fmt = fmt_tag(a[2]);
-  const at::Tensor *g = plain(a[0]), *u = plain(a[1]);
-  if (fmt < 0 || !g || !u || float_tag(*g) < 0 || !same(*g, *u) || g->dim() < 1) Py_RETURN_NONE;
-  const int64_t cols = g->size(-1);
-  const Launch launch(g->device().index());
-  at::Tensor q = empty(g->sizes(), fp8_type(fmt), *g);
-  at::Tensor s = is_static ? empty({1}, c10::ScalarType::Float, *g)
-                           : empty(g->sizes().slice(0, g->dim() - 1), c10::ScalarType::Float, *g);
+  const Input g(a[0]), u(a[1]);
+  if (fmt < 0 || !g || !u || float_tag(g) < 0 || !same(g, u) || g.dim() < 1) Py_RETURN_NONE;
+  const int64_t cols = g.size(-1);
+  const Launch launch(g.device().index());
+  at::Tensor out[2];
+  allocate(g.device(), {{g.sizes(), fp8_type(fmt)}, scales_of(g, is_static)}, out);
+  if (!unchanged(g, u)) Py_RETURN_NONE;
   check_launch("launch_swiglu_fp8_fwd",
-               launch_swiglu_fp8_fwd(g->data_ptr(), u->data_ptr(), (uint8_t*)q.data_ptr(), (float*)s.data_ptr(),
-                                     g->numel() / cols, cols, value, is_static ? CCK_SCALE_STATIC : CCK_SCALE_TOKEN,
-                                     float_tag(*g), fmt, launch.st));
-  return result(std::move(q), std::move(s));
+               launch_swiglu_fp8_fwd(g.data(), u.data(), (uint8_t*)out[0].data_ptr(), (float*)out[1].data_ptr(),
+                                     g.numel() / cols, cols, value, is_static ? CCK_SCALE_STATIC : CCK_SCALE_TOKEN,
+                                     float_tag(g), fmt, launch.st));
+  return result(std::move(out[0]), std::move(out[1]));
   END_HANDLE_TH_ERRORS
 }
 
@@ -198,22 +254,27 @@ inline PyObject* swiglu_fp8(PyObject*, PyArgs a, Py_ssize_t n) {
 inline PyObject* rope(PyObject*, PyArgs a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 5 || (a[4] != Py_True && a[4] != Py_False) || !ordinary_state()) Py_RETURN_NONE;
-  const at::Tensor *q = plain(a[0]), *k = plain(a[1]), *c = plain(a[2]), *s = plain(a[3]);
-  if (!q || !k || !c || !s || float_tag(*q) < 0 || q->dim() != 4 || k->dim() != 4) Py_RETURN_NONE;
-  const int64_t b = q->size(0), len = q->size(1), d = q->size(3);
-  if (k->scalar_type() != q->scalar_type() || k->device() != q->device() || k->size(0) != b || k->size(1) != len ||
-      k->size(3) != d || d % 2 != 0 || c->scalar_type() != c10::ScalarType::Float || !same(*c, *s) ||
-      c->device() != q->device() || c->dim() != 2 || c->size(0) != len || c->size(1) != d / 2) {
+  const Input q(a[0]), k(a[1]), c(a[2]), s(a[3]);
+  if (!q || !k || !c || !s || float_tag(q) < 0 || q.dim() != 4 || k.dim() != 4) Py_RETURN_NONE;
+  const int64_t b = q.size(0), len = q.size(1), d = q.size(3);
+  if (k.type() != q.type() || k.device() != q.device() || k.size(0) != b || k.size(1) != len || k.size(3) != d ||
+      d % 2 != 0 || c.type() != c10::ScalarType::Float || !same(c, s) || c.device() != q.device() || c.dim() != 2 ||
+      c.size(0) != len || c.size(1) != d / 2) {
     Py_RETURN_NONE;
   }
-  const Launch launch(q->device().index());
-  const bool inplace = a[4] == Py_True;
-  at::Tensor qo = inplace ? *q : empty(q->sizes(), q->scalar_type(), *q);
-  at::Tensor ko = inplace ? *k : empty(k->sizes(), k->scalar_type(), *k);
+  const Launch launch(q.device().index());
+  at::Tensor out[2];
+  if (a[4] == Py_True) {
+    out[0] = q.tensor();
+    out[1] = k.tensor();
+  } else {
+    allocate(q.device(), {like(q), like(k)}, out);
+    if (!unchanged(q, k, c, s)) Py_RETURN_NONE;
+  }
   check_launch("launch_rope_fwd",
-               launch_rope_fwd(q->data_ptr(), k->data_ptr(), c->data_ptr(), s->data_ptr(), qo.data_ptr(),
-                               ko.data_ptr(), b, len, q->size(2), k->size(2), d, float_tag(*q), launch.st));
-  return result(std::move(qo), std::move(ko));
+               launch_rope_fwd(q.data(), k.data(), c.data(), s.data(), out[0].data_ptr(), out[1].data_ptr(), b, len,
+                               q.size(2), k.size(2), d, float_tag(q), launch.st));
+  return result(std::move(out[0]), std::move(out[1]));
   END_HANDLE_TH_ERRORS
 }
 
@@ -226,23 +287,24 @@ inline PyObject* fp8_quant(PyObject*, PyArgs a, Py_ssize_t n) {
     Py_RETURN_NONE;
   }
   const int32_t fmt = fmt_tag(a[1]);
-  const at::Tensor* x = plain(a[0]);
+  const Input x(a[0]);
   const bool block = PyUnicode_CompareWithASCIIString(a[2], "block") == 0;
   const bool token = !block && PyUnicode_CompareWithASCIIString(a[2], "token") == 0;
   const bool tensor = !block && !token && PyUnicode_CompareWithASCIIString(a[2], "tensor") == 0;
-  if (fmt < 0 || !x || float_tag(*x) < 0 || x->dim() != 2 || !(block || token || tensor) || (is_static && !tensor)) {
+  if (fmt < 0 || !x || float_tag(x) < 0 || x.dim() != 2 || !(block || token || tensor) || (is_static && !tensor)) {
     Py_RETURN_NONE;
   }
-  const int64_t m = x->size(0), cols = x->size(1);
-  const int32_t dt = float_tag(*x);
-  const Launch launch(x->device().index());
-  at::Tensor q = empty({m, cols}, fp8_type(fmt), *x);
-  at::Tensor s = block   ? empty({(m + 127) / 128, (cols + 127) / 128}, c10::ScalarType::Float, *x)
-                 : token ? empty({m}, c10::ScalarType::Float, *x)
-                         : empty({1}, c10::ScalarType::Float, *x);
-  const void* xp = x->data_ptr();
-  uint8_t* qp = (uint8_t*)q.data_ptr();
-  float* sp = (float*)s.data_ptr();
+  const int64_t m = x.size(0), cols = x.size(1);
+  const int32_t dt = float_tag(x);
+  const int64_t tiles[2] = {(m + 127) / 128, (cols + 127) / 128};
+  const c10::IntArrayRef scales = block ? c10::IntArrayRef(tiles) : token ? x.sizes().slice(0, 1) : c10::IntArrayRef(kOne);
+  const Launch launch(x.device().index());
+  at::Tensor out[2];
+  allocate(x.device(), {{x.sizes(), fp8_type(fmt)}, {scales, c10::ScalarType::Float}}, out);
+  if (!unchanged(x)) Py_RETURN_NONE;
+  const void* xp = x.data();
+  uint8_t* qp = (uint8_t*)out[0].data_ptr();
+  float* sp = (float*)out[1].data_ptr();
   if (is_static) {
     check_launch("launch_fp8_quant_static_fwd",
                  launch_fp8_quant_static_fwd(xp, qp, value, sp, m, cols, dt, fmt, launch.st));
@@ -254,7 +316,7 @@ inline PyObject* fp8_quant(PyObject*, PyArgs a, Py_ssize_t n) {
     check_launch("launch_fp8_quant_tensor_fwd",
                  launch_fp8_quant_tensor_fwd(xp, qp, sp, nullptr, m, cols, dt, fmt, launch.st));
   }
-  return result(std::move(q), std::move(s));
+  return result(std::move(out[0]), std::move(out[1]));
   END_HANDLE_TH_ERRORS
 }
 
@@ -262,18 +324,20 @@ inline PyObject* fp8_quant(PyObject*, PyArgs a, Py_ssize_t n) {
 inline PyObject* token_gather(PyObject*, PyArgs a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 2 || !ordinary_state()) Py_RETURN_NONE;
-  const at::Tensor *src = plain(a[0]), *idx = plain(a[1]);
-  if (!src || !idx || tag_of(src->scalar_type()) < 0 || src->dim() != 2 || idx->dim() != 1 ||
-      idx->scalar_type() != c10::ScalarType::Long || idx->device() != src->device()) {
+  const Input src(a[0]), idx(a[1]);
+  if (!src || !idx || tag_of(src.type()) < 0 || src.dim() != 2 || idx.dim() != 1 ||
+      idx.type() != c10::ScalarType::Long || idx.device() != src.device()) {
     Py_RETURN_NONE;
   }
-  const Launch launch(src->device().index());
-  at::Tensor dst = empty({idx->size(0), src->size(1)}, src->scalar_type(), *src);
+  const int64_t sizes[2] = {idx.size(0), src.size(1)};
+  const Launch launch(src.device().index());
+  at::Tensor out[1];
+  allocate(src.device(), {{sizes, src.type()}}, out);
+  if (!unchanged(src, idx)) Py_RETURN_NONE;
   check_launch("launch_token_gather_fwd",
-               launch_token_gather_checked_fwd(src->data_ptr(), (const int64_t*)idx->data_ptr(), dst.data_ptr(),
-                                               src->size(0), idx->size(0), src->size(1), tag_of(src->scalar_type()),
-                                               launch.st));
-  return result(std::move(dst));
+               launch_token_gather_checked_fwd(src.data(), (const int64_t*)idx.data(), out[0].data_ptr(), src.size(0),
+                                               sizes[0], sizes[1], tag_of(src.type()), launch.st));
+  return result(std::move(out[0]));
   END_HANDLE_TH_ERRORS
 }
 
@@ -281,19 +345,22 @@ inline PyObject* token_gather(PyObject*, PyArgs a, Py_ssize_t n) {
 inline PyObject* token_combine(PyObject*, PyArgs a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 3 || !ordinary_state()) Py_RETURN_NONE;
-  const at::Tensor *eo = plain(a[0]), *idx = plain(a[1]), *w = plain(a[2]);
-  if (!eo || !idx || !w || float_tag(*eo) < 0 || eo->dim() != 2 || idx->dim() != 2 ||
-      idx->scalar_type() != c10::ScalarType::Long || w->scalar_type() != c10::ScalarType::Float ||
-      w->sizes() != idx->sizes() || idx->device() != eo->device() || w->device() != eo->device()) {
+  const Input eo(a[0]), idx(a[1]), w(a[2]);
+  if (!eo || !idx || !w || float_tag(eo) < 0 || eo.dim() != 2 || idx.dim() != 2 ||
+      idx.type() != c10::ScalarType::Long || w.type() != c10::ScalarType::Float || w.sizes() != idx.sizes() ||
+      idx.device() != eo.device() || w.device() != eo.device()) {
     Py_RETURN_NONE;
   }
-  const Launch launch(eo->device().index());
-  at::Tensor out = empty({idx->size(0), eo->size(1)}, eo->scalar_type(), *eo);
+  const int64_t sizes[2] = {idx.size(0), eo.size(1)};
+  const Launch launch(eo.device().index());
+  at::Tensor out[1];
+  allocate(eo.device(), {{sizes, eo.type()}}, out);
+  if (!unchanged(eo, idx, w)) Py_RETURN_NONE;
   check_launch("launch_token_combine_fwd",
-               launch_token_combine_checked_fwd(eo->data_ptr(), (const int64_t*)idx->data_ptr(),
-                                                (const float*)w->data_ptr(), out.data_ptr(), eo->size(0),
-                                                idx->size(0), idx->size(1), eo->size(1), float_tag(*eo), launch.st));
-  return result(std::move(out));
+               launch_token_combine_checked_fwd(eo.data(), (const int64_t*)idx.data(), (const float*)w.data(),
+                                                out[0].data_ptr(), eo.size(0), sizes[0], idx.size(1), sizes[1],
+                                                float_tag(eo), launch.st));
+  return result(std::move(out[0]));
   END_HANDLE_TH_ERRORS
 }
 
@@ -301,17 +368,18 @@ inline PyObject* token_combine(PyObject*, PyArgs a, Py_ssize_t n) {
 inline PyObject* compute_permutation(PyObject*, PyArgs a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 2 || !ordinary_state()) Py_RETURN_NONE;
-  const at::Tensor* ids = plain(a[0]);
+  const Input ids(a[0]);
   const int64_t experts = int_arg(a[1], 256);
-  if (!ids || experts < 0 || ids->dim() != 2 || ids->scalar_type() != c10::ScalarType::Long) Py_RETURN_NONE;
-  const int64_t t = ids->size(0), k = ids->size(1);
-  const Launch launch(ids->device().index());
-  at::Tensor permute = empty({t * k}, c10::ScalarType::Long, *ids);
-  at::Tensor unpermute = empty({t, k}, c10::ScalarType::Long, *ids);
+  if (!ids || experts < 0 || ids.dim() != 2 || ids.type() != c10::ScalarType::Long) Py_RETURN_NONE;
+  const int64_t flat[1] = {ids.numel()};
+  const Launch launch(ids.device().index());
+  at::Tensor out[2];
+  allocate(ids.device(), {{flat, c10::ScalarType::Long}, {ids.sizes(), c10::ScalarType::Long}}, out);
+  if (!unchanged(ids)) Py_RETURN_NONE;
   check_launch("launch_moe_permutation_fwd",
-               launch_moe_permutation_fwd((const int64_t*)ids->data_ptr(), (int64_t*)permute.data_ptr(),
-                                          (int64_t*)unpermute.data_ptr(), t, k, experts, launch.st));
-  return result(std::move(permute), std::move(unpermute));
+               launch_moe_permutation_fwd((const int64_t*)ids.data(), (int64_t*)out[0].data_ptr(),
+                                          (int64_t*)out[1].data_ptr(), ids.size(0), ids.size(1), experts, launch.st));
+  return result(std::move(out[0]), std::move(out[1]));
   END_HANDLE_TH_ERRORS
 }
 
@@ -319,16 +387,19 @@ inline PyObject* compute_permutation(PyObject*, PyArgs a, Py_ssize_t n) {
 inline PyObject* moe_router(PyObject*, PyArgs a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 3 || (a[2] != Py_True && a[2] != Py_False) || !ordinary_state()) Py_RETURN_NONE;
-  const at::Tensor* logits = plain(a[0]);
-  if (!logits || float_tag(*logits) < 0 || logits->dim() != 2 || logits->size(1) > 256) Py_RETURN_NONE;
-  const int64_t t = logits->size(0), experts = logits->size(1), k = int_arg(a[1], experts);
+  const Input logits(a[0]);
+  if (!logits || float_tag(logits) < 0 || logits.dim() != 2 || logits.size(1) > 256) Py_RETURN_NONE;
+  const int64_t experts = logits.size(1), k = int_arg(a[1], experts);
   if (k < 0) Py_RETURN_NONE;
-  const Launch launch(logits->device().index());
-  at::Tensor w = empty({t, k}, c10::ScalarType::Float, *logits), ids = empty({t, k}, c10::ScalarType::Long, *logits);
+  const int64_t sizes[2] = {logits.size(0), k};
+  const Launch launch(logits.device().index());
+  at::Tensor out[2];
+  allocate(logits.device(), {{sizes, c10::ScalarType::Float}, {sizes, c10::ScalarType::Long}}, out);
+  if (!unchanged(logits)) Py_RETURN_NONE;
   check_launch("launch_moe_router_fwd",
-               launch_moe_router_fwd(logits->data_ptr(), (float*)w.data_ptr(), (int64_t*)ids.data_ptr(), t, experts,
-                                     k, float_tag(*logits), a[2] == Py_True ? 1 : 0, launch.st));
-  return result(std::move(w), std::move(ids));
+               launch_moe_router_fwd(logits.data(), (float*)out[0].data_ptr(), (int64_t*)out[1].data_ptr(), sizes[0],
+                                     experts, k, float_tag(logits), a[2] == Py_True ? 1 : 0, launch.st));
+  return result(std::move(out[0]), std::move(out[1]));
   END_HANDLE_TH_ERRORS
 }
 

@@ -148,3 +148,38 @@ def test_streams_and_threads():
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not bad
+
+
+def test_inputs_that_another_thread_changes():
+    """An argument whose .data another thread sets to other memory of another size
+    during the calls (under the interpreter lock): each call quantises the one or
+    the other, whole, or is refused; never the one's memory with the other's size.
+    (The memory holds the larger size either way.)"""
+    a, b = _r(128, 4096), _r(128, 4096, seed=1)
+    views = [a, b[:64]]
+    ref = {v.shape[0]: [t.view(torch.uint8).clone() for t in K.fp8_quant(v, "e4m3", "token")] for v in views}
+    x = a.detach()
+    done = threading.Event()
+
+    def flip():
+        i = 0
+        while not done.is_set():
+            i += 1
+            x.data = views[i % 2]
+
+    thread = threading.Thread(target=flip)
+    thread.start()
+    seen, wrong = set(), 0
+    try:
+        for _ in range(200):
+            try:
+                out = K.fp8_quant(x, "e4m3", "token")
+            except ValueError:
+                continue
+            rows = out[0].shape[0]
+            seen.add(rows)
+            wrong += not all(torch.equal(t.view(torch.uint8), r) for t, r in zip(out, ref[rows]))
+    finally:
+        done.set()
+        thread.join()
+    assert wrong == 0 and seen == {64, 128}
