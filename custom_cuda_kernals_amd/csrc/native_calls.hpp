@@ -39,7 +39,7 @@ inline bool ordinary_state() {
          !c10::impl::tls_local_dispatch_key_set().included_.has_any(kWrappers);
 }
 
-// A plain (exactly torch.Tensor or Parameter), contiguous, non-empty GPU tensor, or nullptr.
+// A plain (exactly torch.Tensor or Parameter), contiguous, non-empty, unnamed GPU tensor, or nullptr.
 inline const at::Tensor* plain(PyObject* o) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
@@ -49,7 +49,7 @@ inline const at::Tensor* plain(PyObject* o) {
                                                c10::DispatchKey::FuncTorchGradWrapper}))) {
     return nullptr;
   }
-  return t.is_contiguous() && t.numel() > 0 ? &t : nullptr;
+  return t.is_contiguous() && t.numel() > 0 && !t.has_names() ? &t : nullptr;
 }
 
 // A plain input as the checks saw it: what they compare and the outputs are
@@ -61,18 +61,21 @@ class Input {
   explicit Input(PyObject* o) : object_(o), t_(plain(o)) {
     if (t_ == nullptr) return;
     sizes_ = t_->sizes();
+    strides_ = t_->strides();
     type_ = t_->scalar_type();
     device_ = t_->device();
   }
   explicit operator bool() const { return t_ != nullptr; }
   // The tensor still is what the checks saw.
   bool unchanged() const {
-    return plain(object_) == t_ && t_->sizes() == sizes() && t_->scalar_type() == type_ && t_->device() == device_;
+    return plain(object_) == t_ && t_->sizes() == sizes() && t_->strides() == strides() &&
+           t_->scalar_type() == type_ && t_->device() == device_;
   }
   const at::Tensor& tensor() const { return *t_; }
   // For the launch, in the hold of the lock of the last look at the tensor.
   void* data() const { return t_->data_ptr(); }
   c10::IntArrayRef sizes() const { return sizes_; }
+  c10::IntArrayRef strides() const { return strides_; }
   int64_t dim() const { return (int64_t)sizes_.size(); }
   int64_t size(int64_t i) const { return sizes_[i < 0 ? i + sizes_.size() : i]; }
   int64_t numel() const { return c10::multiply_integers(sizes_); }
@@ -82,7 +85,7 @@ class Input {
  private:
   PyObject* object_;
   const at::Tensor* t_;
-  c10::DimVector sizes_;
+  c10::DimVector sizes_, strides_;
   c10::ScalarType type_ = c10::ScalarType::Undefined;
   c10::Device device_ = c10::kCPU;
 };
@@ -126,20 +129,26 @@ inline int64_t int_arg(PyObject* o, int64_t most) {
   return overflow == 0 && v >= 1 && v <= most ? (int64_t)v : -1;
 }
 
+// An output: dense in row-major order or, as empty_like, with the strides of
+// an input (they differ from those in dimensions of size 1 only).
 struct Output {
   c10::IntArrayRef sizes;
   c10::ScalarType type;
+  c10::IntArrayRef strides = {};
 };
-inline Output like(const Input& t) { return {t.sizes(), t.type()}; }
+inline Output like(const Input& t) { return {t.sizes(), t.type(), t.strides()}; }
 
 // Without the interpreter lock, as torch.empty: an allocation may have to wait
-// for the GPU, whose work may wait for another Python thread. Sizes are the
-// caller's copies. The inputs must be looked at again afterwards.
+// for the GPU, whose work may wait for another Python thread. Sizes and strides
+// are the caller's copies. The inputs must be looked at again afterwards.
 template <size_t N>
 inline void allocate(c10::Device device, const Output (&wanted)[N], at::Tensor (&out)[N]) {
   const py::gil_scoped_release unlocked;
   for (size_t i = 0; i < N; ++i) {
-    out[i] = at::empty(wanted[i].sizes, at::TensorOptions().dtype(wanted[i].type).device(device));
+    const auto options = at::TensorOptions().dtype(wanted[i].type).device(device);
+    out[i] = wanted[i].strides.size() != wanted[i].sizes.size()
+                 ? at::empty(wanted[i].sizes, options)
+                 : at::empty_strided(wanted[i].sizes, wanted[i].strides, options);
   }
 }
 

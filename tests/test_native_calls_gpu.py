@@ -183,3 +183,28 @@ def test_inputs_that_another_thread_changes():
         done.set()
         thread.join()
     assert wrong == 0 and seen == {64, 128}
+
+
+def _forms(call):
+    out = call()
+    return [(t.shape, t.stride(), t.names) for t in (out if isinstance(out, tuple) else (out,))]
+
+
+def test_strides_and_names_as_the_long_way(monkeypatch):
+    """Inputs that are contiguous with other strides in dimensions of size 1 (one
+    token cut out of a batch), and inputs with dimension names: the outputs made
+    like an input keep both."""
+    base, w = _r(1, 6, 4, 64), _r(64)
+    q = base[:, 2:3]
+    x = base.view(1, 24, 64)[:, 5:6]
+    assert x.is_contiguous() and x.stride() != torch.empty(x.shape).stride()
+    named = x.clone().rename("b", "s", "h")
+    cos = _r(1, 32, dtype=torch.float32)
+    calls = [lambda: K.rmsnorm_residual(x, x, w), lambda: K.rmsnorm_residual_fp8(x, x, w), lambda: K.swiglu(x, x),
+             lambda: K.swiglu_fp8(x, x), lambda: K.rope(q, q.clone(), cos, cos), lambda: K.swiglu(named, named),
+             lambda: K.rmsnorm_residual(named, x, w), lambda: K.fp8_quant(x[0])]
+    one = [_forms(c) for c in calls]
+    for name in NAMES:
+        monkeypatch.setattr(native, name, lambda *a: None)
+    assert [_forms(c) for c in calls] == one
+    assert one[0][0][1] == x.stride() and one[5][0][2] == ("b", "s", "h")
