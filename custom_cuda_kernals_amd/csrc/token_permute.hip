@@ -280,26 +280,41 @@ __device__ inline float combine_scalar_column(const void* eo, const int64_t* it,
 }
 
 // One scalar column of one token for k <= 16: aten_scalar_sum's operations
-// (no 16-step block of a slot completes, so each slot is one running sum), with
-// every index, then every element, loaded before the first is used.
+// (no 16-step block of a slot completes, so each slot is one running sum). Eight
+// terms at a time: their indices, then their elements, all in flight before the
+// first is used. So no load may depend on a branch: a term out of range, or past
+// k, loads from the weights, which are always there, and is then left out.
 template <class C>
 __device__ inline float combine_tail(const char* eo, const int64_t* it, const float* wt, int k, int64_t row_bytes,
                                      int64_t c, int64_t n_rows) {
-  float x[16];
-  int64_t r[16];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) r[j] = it[j < k ? j : 0];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const bool ok = j < k && r[j] >= 0 && r[j] < n_rows;
-    x[j] = ok ? wt[j] * C::load1(eo + r[j] * row_bytes, c) : 0.0f;
-  }
   const int whole = k & ~3;
   float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int j0 = 0; j0 < k; j0 += 8) {
+    int64_t r[8];
+    float x[8], f[8];
+    uint32_t keep[8];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) s[j % 4] = j < whole ? s[j % 4] + x[j] : s[j % 4];
+    for (int j = 0; j < 8; ++j) r[j] = it[j0 + j < k ? j0 + j : 0];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) s[0] = j >= whole && j < k ? s[0] + x[j] : s[0];
+    for (int j = 0; j < 8; ++j) f[j] = wt[j0 + j < k ? j0 + j : 0];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const bool ok = j0 + j < k && r[j] >= 0 && r[j] < n_rows;
+      x[j] = C::load1(ok ? eo + r[j] * row_bytes + c * C::kBytes : reinterpret_cast<const char*>(wt), 0);
+      // Left out by a mask that is opaque to the optimiser, which moves the load
+      // into a branch on ok otherwise.
+      keep[j] = ok ? 0xffffffffu : 0u;
+      asm("" : "+v"(keep[j]));
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = bits_f32(f32_bits(f[j] * x[j]) & keep[j]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int i = j0 + j;
+      s[j % 4] = i < whole ? s[j % 4] + f[j] : s[j % 4];
+      s[0] = i >= whole && i < k ? s[0] + f[j] : s[0];
+    }
+  }
   return ((s[0] + s[1]) + s[2]) + s[3];
 }
 
@@ -364,6 +379,10 @@ __global__ __launch_bounds__(THREADS) void token_combine_vec(const char* __restr
         u32x4 raw[JU][VPL];
         float wj[JU];
         bool ok[JU];
+        // The last step's loads have all been used by now (vmcnt 0), but the
+        // compiler does not see it, since they stand under branches: it would wait
+        // before each load that reuses a register, so for the load before it.
+        if constexpr (ANY) __builtin_amdgcn_s_waitcnt(0x0f70);
 #pragma unroll
         for (int u = 0; u < JU; ++u) {
           const int64_t j = j0 + u;
@@ -590,21 +609,32 @@ int32_t combine(const void* eo, const int64_t* uidx, const float* w, void* out, 
     const unsigned grid = row_grid(n_tokens);
     // Rows of main columns only by aligned vectors; other rows' main columns by
     // unaligned ones, in the same forms, with the other columns beside them.
-    const bool whole = order.main_cols == h && host_aligned(eo, 16) && host_aligned(out, 16);
-    // (Rows of under 128 columns that are no whole vectors stay on the
-    // element-wise kernel: 2.9 vs 3.4 us at 300 tokens of 100, top 2.) On MI355X
-    // against that kernel, which took every such row, bf16: 1000 tokens of 4100, top
-    // 3, 23.7 vs 9.4 us; 16 of 5461, top 4, 19.6 vs 4.0; 8000 of 1001, top 4, 48.9 vs
-    // 20.1; fp16 2048 of 7001, top 8, 231 vs 57.6; fp32 777 of 5461, top 5, 63.4 vs
-    // 20.6. Against aligned vectors and a second launch for the other columns,
-    // 2048 of 4104, top 6, 25.7 vs 24.2 (1000 of 1000, top 6, 8.2 vs 8.4).
+    // Deeper sums, whose other columns have a launch of their own anyway, write
+    // whole vectors, the last columns to be rewritten, where those need no further
+    // wave: 1000 tokens of 72, top 17, 15.8 us against 17.1; 128 of 4104, a 513th
+    // vector, 22.3 against 16.7.
     const bool vectors = host_aligned(eo, 16) && host_aligned(out, 16) && h % C::VEC == 0;
-    if (order.main_cols >= C::VEC && (vectors || h >= 128)) {
+    const int64_t mv = order.main_cols / C::VEC;
+    const bool whole = vectors && (order.main_cols == h || (k > 16 && (h / C::VEC - 1) / 64 == (mv - 1) / 64));
+    // Against the element-wise kernel, which would take every other row, on
+    // MI355X, bf16, graph-replayed, buffers on chip / from HBM: 1000 tokens of 4100, top
+    // 4, 30.1 vs 8.6 us; 16 of 4100, top 4, 15.5 vs 3.1; 4096 of 1001, top 4, 26.5 vs 9.8 /
+    // 34.2 vs 10.9; 4096 of 700, top 16, 87.3 vs 19.7. Against aligned vectors and a second
+    // launch, 1000 tokens of 1000, top 8, 9.9 vs 6.7 / 13.0 vs 6.9; of 776, top 16, 15.3
+    // vs 10.5; of 4104, top 8, 18.3 vs 13.6. Few columns leave the vectors' workgroups
+    // idle, and few tokens do not pay for the other columns' workgroups: 128
+    // tokens of 129, top 1, 2.36 vs 2.74 us, top 8 3.42 vs 3.88, 1000 of 129, top 1, 2.97
+    // vs 3.15 (1500: 3.46 vs 3.40; 128 of 190, top 2, 2.75 vs 2.62). Deeper sums step
+    // through their rows two at a time and take two launches: top 17, 128 tokens
+    // of 513 10.7 vs 12.3 us (fp32, top 32, 22.7 vs 18.9), of 700 13.6 vs 12.3; 1000 of 387 16.0 vs 16.6 / 20.5 vs 22.1,
+    // of 513 19.1 vs 17.0; 3000 of 150 17.6 vs 22.9 / 21.9 vs 24.5, of 259 26.5 vs 22.9.
+    const int64_t few_deep = n_tokens <= 256 ? (C::VEC == 8 ? 600 : 500) : n_tokens <= 1536 ? 400 : n_tokens <= 3072 ? 160 : 128;
+    const int64_t few_columns = k > 16 ? few_deep : n_tokens <= 1024 ? (k == 1 ? 288 : 160) : 128;
+    if (order.main_cols >= C::VEC && (vectors || h >= few_columns)) {
       // Two expert rows in flight per step. Top-1/2 rows: 4 vectors per thread
       // (9.4 us at T=2048, k=2, hidden 4096 bf16); deeper top-k: 2 per thread
       // (20.5 us at k=6); both measured on MI355X against 1-8 vectors and 1-8 rows.
-      const int64_t mv = order.main_cols / C::VEC;
-      const int64_t rv = mv;
+      const int64_t rv = whole ? h / C::VEC : mv;
       auto launch = [&](auto threads, auto vpl, auto casc) {
         constexpr int TH = decltype(threads)::value, V = decltype(vpl)::value;
         auto go = [&](auto any) {
@@ -636,7 +666,7 @@ int32_t combine(const void* eo, const int64_t* uidx, const float* w, void* out, 
       const bool few = n_tokens <= kCombineFewTokens && k <= 16 && mv >= 512;
       if (k > 16) {
         // Deeper sums take ATen's block cascade: one vector per thread.
-        with_row_threads<1, 512>(mv, [&](auto threads) { launch(threads, IntC<1>{}, std::true_type{}); });
+        with_row_threads<1, 512>(rv, [&](auto threads) { launch(threads, IntC<1>{}, std::true_type{}); });
       } else if (many || few) {
         if (mv <= 512) {
           wide(IntC<1>{});
@@ -662,6 +692,10 @@ int32_t combine(const void* eo, const int64_t* uidx, const float* w, void* out, 
         token_combine_elems<C, 64><<<grid, 64, 0, st>>>(eo, uidx, w, out, n_tokens, k, h, order.main_cols, n_rows,
                                                         order);
       }
+    } else if (vectors) {
+      // At most 31 columns, so one wave: 4096 tokens of 16, top 2, 3.5 us against 5.6
+      // for four.
+      token_combine_elems<C, 64><<<grid, 64, 0, st>>>(eo, uidx, w, out, n_tokens, k, h, 0, n_rows, order);
     } else {
       token_combine_elems<C, 256><<<grid, 256, 0, st>>>(eo, uidx, w, out, n_tokens, k, h, 0, n_rows, order);
     }

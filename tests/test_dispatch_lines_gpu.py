@@ -1,0 +1,65 @@
+"""Either side of the lines that a measurement drew between two kernels of one
+op: the call takes the kernel that was the faster one there, and its results are
+the oracle's bits."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from custom_cuda_kernals_amd import _native as native
+from oracle import inputs, moe
+from tests._parity import bits_equal
+from tests._routes import kernels_of
+
+pytestmark = pytest.mark.gpu
+
+BF16 = torch.bfloat16
+
+
+def _takes(call, kernel: str, threads: int | None = None) -> None:
+    name, block = kernels_of(call)[0]
+    assert kernel in name and threads in (None, block), (name, block)
+
+
+# (tokens, top k, columns, kernel, threads)
+COMBINES = [(1024, 1, 287, "token_combine_elems", 256), (1024, 1, 289, "token_combine_vec", None),
+            (1025, 1, 287, "token_combine_vec", None), (1024, 2, 159, "token_combine_elems", 256),
+            (1024, 2, 161, "token_combine_vec", None), (1025, 4, 129, "token_combine_vec", None),
+            (256, 17, 599, "token_combine_elems", 256), (256, 17, 601, "token_combine_vec", None),
+            (257, 17, 399, "token_combine_elems", 256), (257, 17, 401, "token_combine_vec", None),
+            (1537, 17, 159, "token_combine_elems", 256), (1537, 17, 161, "token_combine_vec", None),
+            (3073, 17, 129, "token_combine_vec", None),
+            (5, 2, 8, "token_combine_elems", 64), (5, 17, 24, "token_combine_elems", 64),
+            (7, 17, 72, "token_combine_vecINS_9CodecBF16ELi64ELi1ELi2ELb1ELb0E", 64),
+            (7, 17, 4104, "token_combine_vecINS_9CodecBF16ELi512ELi1ELi2ELb1ELb1E", 512),
+            (7, 16, 72, "token_combine_vecINS_9CodecBF16ELi64ELi2ELi2ELb0ELb1E", 64)]
+
+
+@pytest.mark.parametrize("t,k,h,kernel,threads", COMBINES)
+def test_combine(t, k, h, kernel, threads):
+    eo, ui, w = inputs.combine_inputs(t, k, h, BF16, seed=h + k)
+    ui_ref, w_ref = ui.clone(), w.clone()
+    for row, j, bad in ((0, 0, -1), (t // 2, k - 1, t * k)):
+        ui[row, j], ui_ref[row, j], w_ref[row, j] = bad, 0, 0.0
+    d = [v.cuda() for v in (eo, ui, w)]
+    out = torch.empty(t, h, dtype=BF16, device="cuda")
+    _takes(lambda: native.token_combine_fwd(*d, out), kernel, threads)
+    assert bits_equal(out, moe.token_combine_aten(eo, ui_ref, w_ref)).all()
+
+
+@pytest.mark.parametrize("k", [1, 7, 8, 9, 15, 16])
+@pytest.mark.parametrize("h", [1003, 1000])
+def test_combine_of_no_rows_and_of_infinite_weights(h, k):
+    """The other columns' loads stand under no branch: with no expert rows, and
+    with weights that would make NaNs of a dropped term, dropped terms add nothing."""
+    eo, ui, w = inputs.combine_inputs(6, k, h, BF16, seed=k)
+    out = torch.empty(6, h, dtype=BF16, device="cuda")
+    native.token_combine_fwd(eo[:0].cuda(), ui.cuda(), torch.full_like(w, float("inf")).cuda(), out)
+    assert bits_equal(out, torch.zeros(6, h, dtype=BF16)).all()
+    bad = ui.clone()
+    bad[::2, k // 2] = 6 * k
+    w_bad, ui_ref, w_ref = w.clone(), ui.clone(), w.clone()
+    w_bad[::2, k // 2], ui_ref[::2, k // 2], w_ref[::2, k // 2] = float("nan"), 0, 0.0
+    native.token_combine_fwd(eo.cuda(), bad.cuda(), w_bad.cuda(), out)
+    assert bits_equal(out, moe.token_combine_aten(eo, ui_ref, w_ref)).all()
