@@ -122,45 +122,62 @@ __global__ __launch_bounds__(256) void token_gather_flat(const u32x4* __restrict
   }
 }
 
-// Gathers that read source rows more than once, and rows that are no whole
-// 16-byte vectors. A row is cut into `slices` column slices (a power of two,
-// at most 8) of `width` vectors, and workgroup b moves slice b % slices:
-// workgroups are dealt to the 8 XCDs round-robin, so each XCD's 4 MB L2 sees
-// one slice of the source only, and a row that k destinations name is fetched
-// from beyond the L2s once instead of once per XCD. (Where the deal is another,
-// only the speed changes.) One wave per destination row and slice; loads are
-// cached, stores nontemporal. The last vector of a row is its last 16 bytes
-// (it repeats up to 15 of its neighbour's, the same bytes); ANY: rows and
-// buffers of any alignment, at least 16 bytes a row.
+// Gathers that read source rows several times over, and rows that are no whole
+// 16-byte vectors. A row is cut into 1 << slice_bits column slices (at most 8) of
+// `width` vectors, and workgroup b moves slice b mod that: workgroups are dealt
+// to the 8 XCDs round-robin, so each XCD's 4 MB L2 sees one slice of the source
+// only, and a row that k destinations name is fetched from beyond the L2s once
+// instead of once per XCD. (Where the deal is another, only the speed changes.)
+// One wave per destination row and slice; loads are cached, stores nontemporal.
+// ANY: rows and buffers of any alignment, at least 16 bytes a row, two vectors in
+// flight a lane; the last vector of a row is its last 16 bytes (it repeats up to
+// 15 of its neighbour's, the same bytes). CACHED: plain stores, see the launcher.
 // Bound by the 8 L2s' fills and the writes: 2048 rows of 8 KB to 12288 17.3 us,
 // 117 MB at 6.8 TB/s, where the flat form read 100 MB from beyond the L2s and
 // took 31.9 (24.8 with its loads cached); two, four and eight rows in flight per
-// wave 17.4, 18.8 and 21.0.
-template <bool ANY>
+// wave 17.4, 18.8 and 21.0, two vectors of one row 16.1 against 15.4 to 10240 rows.
+// (The slice split by division instead of shifts took 16.6 there, and 0.1 to 0.2
+// us of the 2.1 us of the smallest gathers.)
+template <bool ANY, bool CACHED = false>
 __global__ __launch_bounds__(256) void token_gather_slices(const char* __restrict__ src,
                                                            const int64_t* __restrict__ idx, char* __restrict__ dst,
                                                            int64_t n_dst, int64_t row_bytes, int64_t n_src,
-                                                           int slices, int64_t width) {
+                                                           int slice_bits, int64_t width) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t nvec = (row_bytes + 15) / 16, last = row_bytes - 16;
-  const int64_t c0 = (int64_t)(blockIdx.x % (unsigned)slices) * width;
+  const int64_t c0 = (int64_t)(blockIdx.x & ((1u << slice_bits) - 1u)) * width;
   const int64_t c1 = c0 + width < nvec ? c0 + width : nvec;
-  const int64_t groups = gridDim.x / (unsigned)slices;
-  for (int64_t row = (int64_t)(blockIdx.x / (unsigned)slices) * 4 + wave; row < n_dst; row += groups * 4) {
+  const int64_t groups = gridDim.x >> slice_bits;
+  for (int64_t row = (int64_t)(blockIdx.x >> slice_bits) * 4 + wave; row < n_dst; row += groups * 4) {
     const int64_t s = idx[row];  // uniform: a scalar load
     const bool valid = s >= 0 && s < n_src;
     const char* from = src + (valid ? s : 0) * row_bytes;
     char* to = dst + row * row_bytes;
-    for (int64_t v = c0 + lane; v < c1; v += 64) {
-      const int64_t at = v * 16 < last ? v * 16 : last;
-      u32x4 w = {0u, 0u, 0u, 0u};
-      if constexpr (ANY) {
-        if (valid) w = *reinterpret_cast<const u32x4_any*>(from + at);
-        __builtin_nontemporal_store(w, reinterpret_cast<u32x4_any*>(to + at));
-      } else {
-        if (valid) w = *reinterpret_cast<const u32x4*>(from + at);
-        st_stream(w, reinterpret_cast<u32x4*>(to + at));
+    if constexpr (ANY) {
+      auto store = [&](const u32x4& w, int64_t at) {
+        if constexpr (CACHED) {
+          *reinterpret_cast<u32x4_any*>(to + at) = w;
+        } else {
+          __builtin_nontemporal_store(w, reinterpret_cast<u32x4_any*>(to + at));
+        }
+      };
+      for (int64_t v = c0 + lane; v < c1; v += 128) {
+        const bool more = v + 64 < c1;
+        const int64_t at = v * 16 < last ? v * 16 : last, next = (v + 64) * 16 < last ? (v + 64) * 16 : last;
+        u32x4 w = {0u, 0u, 0u, 0u}, x = {0u, 0u, 0u, 0u};
+        if (valid) {
+          w = *reinterpret_cast<const u32x4_any*>(from + at);
+          x = *reinterpret_cast<const u32x4_any*>(from + (more ? next : at));
+        }
+        store(w, at);
+        if (more) store(x, next);
+      }
+    } else {
+      for (int64_t v = c0 + lane; v < c1; v += 64) {
+        u32x4 w = {0u, 0u, 0u, 0u};
+        if (valid) w = reinterpret_cast<const u32x4*>(from)[v];
+        st_stream(w, reinterpret_cast<u32x4*>(to) + v);
       }
     }
   }
@@ -514,9 +531,50 @@ constexpr int64_t kGatherR8Min = 4096;
 // vs 12.1 us; 8192 -> 16384 rows of 1024, 11.8 vs 12.6; 4096 rows of 2048,
 // 6.8 vs 7.4.
 constexpr int64_t kGatherFlatMin = int64_t(1) << 22;
-constexpr int64_t kGatherSliceMin = 128;
+// Column slices of a row of `nvec` vectors: 1 << bits of them (at most 8, of at
+// least 64 vectors), `width` vectors each, whole cache lines.
+struct GatherSlices {
+  int bits = 0;
+  int64_t width;
+  explicit GatherSlices(int64_t nvec) {
+    while (bits < 3 && nvec >= 128 << bits) ++bits;
+    width = (((nvec - 1) >> bits) + 8) / 8 * 8;
+  }
+};
+
+// Whether a gather of whole rows moves by slices: where source rows repeat (the
+// checked launchers know their count) in rows of at least 128 vectors. Same-run
+// A/B on MI355X, bf16, buffers on chip / from HBM, the other forms vs sliced:
+//   * more than four destinations a source row: 2048 -> 10240 rows of 1024 7.5 / 7.6 vs
+//     6.3 / 6.6 us, of 4096 26.6 / 26.9 vs 15.4 / 15.2, of 7168 46.0 / 46.8 vs 27.9 / 28.2;
+//     256 -> 2048 of 4096 6.5 / 6.8 vs 5.0 / 4.5;
+//   * more than three, in rows of 352 vectors or whose slices fill their waves to
+//     four fifths: 2048 -> 8192 of 4096 21.5 / 22.0 vs 12.5 / 19.6, of 5120 27.0 / 27.6 vs
+//     16.2 / 27.9 (not of 1280: 7.7 / 7.9 vs 6.5 / 8.6);
+//   * more than two, in rows of 512 vectors whose slices fill their waves so: 2048 ->
+//     6144 of 4096 16.8 / 17.2 vs 10.4 / 16.4, of 7168 28.6 / 29.0 vs 18.8 / 27.5 (not of
+//     5120: 20.9 / 21.3 vs 13.3 / 22.8; of 1536 6.9 / 7.1 vs 6.3 / 8.5, of 1024 5.3 / 5.1 vs
+//     4.3 / 5.7);
+//   * past 512 vectors not where there is little to move: 16 -> 80 fp32 rows of 7168
+//     2.5 vs 2.6 us (32 -> 256 bf16 2.8 / 3.5 vs 2.7 / 2.8); up to four destinations a row
+//     64 -> 256 fp32 of 7168 4.5 / 4.5 vs 2.8 / 5.2 (256 -> 1024 10.6 / 10.8 vs 6.6 / 10.2).
+inline bool gather_by_slices(int64_t n_dst, int64_t n_src, int64_t nvec) {
+  if (nvec < 128 || (n_dst - 1) / 2 < n_src) return false;
+  const int64_t total = n_dst * nvec;
+  if ((n_dst - 1) / 4 >= n_src) return nvec <= 512 || total >= 3 << 16;
+  if (nvec > 512 && total <= 1 << 19) return false;
+  const int64_t width = GatherSlices(nvec).width, lanes = (width + 63) / 64 * 64;
+  const bool filled = 5 * width >= 4 * lanes;
+  return (n_dst - 1) / 3 >= n_src ? filled || nvec >= 352 : filled && nvec >= 512;
+}
+
 // Ragged rows of fewer bytes stay element-wise (600 rows of 200 bytes: 2.2 vs 2.4 us).
 constexpr int64_t kGatherAnyMin = 256;
+// Ragged destinations up to this size are stored plainly, and their partial lines
+// meet in the L2s: bf16, buffers on chip / from HBM, 64 rows of 1001 2.44 us
+// nontemporal, 2.26 plain; 2000 of 1001 3.21 / 3.95 vs 2.95 / 4.02; 4000 of 1001 4.04 /
+// 5.47 vs 4.17 / 5.65; 2000 of 4099 7.8 / 9.8 vs 8.0 / 10.8.
+constexpr int64_t kGatherCachedMax = 4 << 20;
 
 int32_t gather(const void* src, const int64_t* indices, void* dst, int64_t n_dst, int64_t h,
                int32_t dtype, int64_t n_src, hipStream_t st) {
@@ -526,31 +584,27 @@ int32_t gather(const void* src, const int64_t* indices, void* dst, int64_t n_dst
   const unsigned grid = row_grid(n_dst);
   const int64_t row_bytes = h * es;
   const bool whole = row_bytes % 16 == 0 && host_aligned(src, 16) && host_aligned(dst, 16);
-  // Sliced where source rows repeat often (more than two destinations a source
-  // row, whose count the checked launchers know) in rows of at least
-  // kGatherSliceMin vectors, and for every ragged row: slices of at least 64
-  // vectors, whole cache lines. Same-run A/B on MI355X, bf16, buffers on chip /
-  // from HBM: 2048 -> 12288 rows of 4096 30.9 / 31.5 vs 18.8 / 18.7 us, 4096 -> 32768
-  // of 7168 145.9 / 146.0 vs 108.1 / 108.1, 8192 -> 49152 of 2048 62.1 / 65.7 vs 48.2 /
-  // 48.1, 8192 -> 32768 of 1024 22.0 / 23.5 vs 18.5 / 23.2 (of 512, one slice: 11.1 /
-  // 11.6 vs 10.5 / 12.9, not taken); two destinations a row
-  // lose from HBM (2048 -> 4096 of 4096 10.8 / 11.7 vs 8.9 / 12.6). Ragged rows
-  // against the element-wise kernel: 1000 -> 3000 of 4100 14.1 / 21.5 vs 7.8 / 11.1,
-  // 64 of 5461 4.1 / 7.4 vs 2.7 / 2.8.
-  auto run_slices = [&](auto any) {
-    const int64_t nvec = (row_bytes + 15) / 16;
-    int slices = 1;
-    while (slices < 8 && nvec >= 64 * 2 * slices) slices *= 2;
-    const int64_t width = ((nvec + slices - 1) / slices + 7) / 8 * 8;
+  // Ragged rows move by slices too. Against the element-wise kernel, as above: 64 of
+  // 1001 2.24 vs 2.26 us; 1000 of 1001 2.66 / 4.11 vs 2.45 / 3.27; 4000 of 2050 9.4 / 14.6
+  // vs 7.4 / 9.4; 10000 of 4099 62.9 / 63.3 vs 32.3 / 39.1; fp32 4000 of 2881 22.3 / 24.2 vs
+  // 17.4 / 21.6, but 4000 of 2050 12.1 / 17.9 vs 13.2 / 16.2 and 2000 of 4099 11.6 / 16.8 vs
+  // 13.1 / 16.9 (destinations of about the L2s' size).
+  auto run_slices = [&](auto any, auto cached) {
+    const GatherSlices slices((row_bytes + 15) / 16);
     const int64_t groups = (n_dst + 3) / 4;
     const int64_t cap = kMaxRowGroups;
-    token_gather_slices<decltype(any)::value><<<(unsigned)((groups < cap ? groups : cap) * slices), 256, 0, st>>>(
-        static_cast<const char*>(src), indices, static_cast<char*>(dst), n_dst, row_bytes, n_src, slices, width);
+    token_gather_slices<decltype(any)::value, decltype(cached)::value><<<(unsigned)((groups < cap ? groups : cap) << slices.bits), 256, 0, st>>>(
+        static_cast<const char*>(src), indices, static_cast<char*>(dst), n_dst, row_bytes, n_src,
+        slices.bits, slices.width);
   };
   if (!whole && row_bytes >= kGatherAnyMin) {
-    run_slices(std::true_type{});
-  } else if (whole && n_dst / 2 > n_src && row_bytes >= 16 * kGatherSliceMin) {
-    run_slices(std::false_type{});
+    if (n_dst * row_bytes <= kGatherCachedMax) {
+      run_slices(std::true_type{}, std::true_type{});
+    } else {
+      run_slices(std::true_type{}, std::false_type{});
+    }
+  } else if (whole && gather_by_slices(n_dst, n_src, row_bytes / 16)) {
+    run_slices(std::false_type{}, std::false_type{});
   } else if (whole) {
     const int64_t rv = row_bytes / 16;
     if (rv > 512 || (rv >= 64 && n_dst * rv >= kGatherFlatMin)) {

@@ -63,3 +63,26 @@ def test_combine_of_no_rows_and_of_infinite_weights(h, k):
     w_bad[::2, k // 2], ui_ref[::2, k // 2], w_ref[::2, k // 2] = float("nan"), 0, 0.0
     native.token_combine_fwd(eo.cuda(), bad.cuda(), w_bad.cuda(), out)
     assert bits_equal(out, moe.token_combine_aten(eo, ui_ref, w_ref)).all()
+
+
+PLAIN, RAGGED, CACHED = (f"token_gather_slicesILb{a}ELb{c}E" for a, c in ((0, 0), (1, 0), (1, 1)))
+# (source rows, destination rows, columns, kernel)
+GATHERS = [(8, 33, 1016, "token_gather_rows"), (8, 33, 1280, PLAIN), (8, 32, 1280, "token_gather_rows"),
+           (8, 25, 1024, PLAIN), (8, 24, 1024, "token_gather_rows"), (8, 17, 4096, PLAIN),
+           (8, 16, 4096, "token_gather_rows"),
+           (300, 901, 5120, PLAIN), (300, 900, 5120, "token_gather_flat"), (8, 25, 2880, PLAIN), (40, 189, 8320, "token_gather_flat"), (40, 190, 8320, PLAIN),
+           (200, 585, 7168, "token_gather_flat"), (200, 586, 7168, PLAIN), (0, 3, 1024, PLAIN),
+           (7, 9, 127, "token_gather_elems"), (7, 9, 129, CACHED), (0, 9, 1001, CACHED), (500, 2095, 1001, CACHED),
+           (500, 2096, 1001, RAGGED), (40, 300, 8321, RAGGED)]
+
+
+@pytest.mark.parametrize("ns,nd,h,kernel", GATHERS)
+def test_gather(ns, nd, h, kernel):
+    """(A source of no rows: every index is out of range, and nothing is read.)"""
+    src = inputs.randn((max(ns, 1), h), BF16, seed=h)
+    idx = torch.randint(-1, ns + 1, (nd,), generator=torch.Generator().manual_seed(nd))
+    dst = torch.empty(nd, h, dtype=BF16, device="cuda")
+    d = src[:ns].cuda(), idx.cuda()
+    _takes(lambda: native.token_gather_fwd(*d, dst), kernel)
+    ok = (idx >= 0) & (idx < ns)
+    assert bits_equal(dst, torch.where(ok[:, None], src[torch.where(ok, idx, 0)], 0.0)).all()
