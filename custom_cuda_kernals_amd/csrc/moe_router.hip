@@ -23,9 +23,9 @@
 //   * E <= 8: one lane per token (moe_router_lanes);
 //   * E >= 9: a group of lanes per token, each holding its part of every
 //     16-expert stripe (moe_router_groups): four lanes up to 16 experts, 16 lanes
-//     above, eight for up to 64 experts of many tokens;
-//   * 16-bit rows of E > 192 and few tokens: one wave per token
-//     (moe_router_waves), below.
+//     above, eight and four for up to 64 and 32 experts of many tokens;
+//   * more than 128 experts of few tokens and picks (keeps_waves): one wave per
+//     token (moe_router_waves), below.
 // One wave64 per token holds up to 256 experts (4 per lane, expert
 // e = lane + 64 * slot). The max is a wave all-reduction (DPP). The
 // exponentials go to a per-wave LDS row; every lane then runs its lane
@@ -544,18 +544,41 @@ void launch_router_groups(const void* logits, float* w, int64_t* idx, int64_t t,
 }
 
 // From 17 experts up a token takes 16 lanes, one per lane class of the softmax
-// sum. Graph-replayed on MI355X against the forms that served these sizes, fp32:
-// top-6 of 32 at 4096 tokens 2.9 vs 4.3 us (four lanes), top-8 of 64 at 2048 4.0 vs 6.4
-// (a wave per token) and at 8192 4.9 vs 7.7 (four lanes), top-6 of 160 at 512 / 2048 /
-// 4096 4.1 / 4.3 / 4.8 vs 4.9 / 5.2 / 6.8 (waves) and at 16384 7.5 vs 9.1 (eight lanes),
-// top-8 of 256 at 4096 / 16384 7.1 / 11.9 vs 8.8 (waves) / 14.7. They are bound by the
-// chain of one wave up to about one wave per SIMD (4096 tokens), by instructions
-// after that, where eight lanes hold fewer idle slots of few experts: top-6 of 32
-// at 16384 tokens 4.0 vs 4.2, at 32768 5.2 vs 6.1; top-8 of 64 at 32768 8.1 vs 9.2.
+// sum. Graph-replayed on MI355X against the forms that served these sizes, fp32 /
+// bf16: top-8 of 64 at 2048 tokens 4.0 / 4.1 vs 6.4 (a wave per token) and at 8192 4.9 /
+// 4.8 vs 7.3 / 7.6 us (four lanes), top-6 of 160 at 512 / 2048 / 4096 4.2 / 4.3 / 4.4 vs 5.0 /
+// 5.3 / 6.9 (waves; bf16 4.7 / 4.7 / 4.9 vs 5.1 / 5.5 / 7.1), top-8 of 256 at 4096 / 16384
+// 6.5 / 12.1 vs 8.8 (waves) / 14.8 (eight lanes). They are bound by the chain of one
+// wave up to about one wave per SIMD (4096 tokens), by instructions after that, where
+// fewer lanes hold fewer idle slots of few experts: up to 32 experts, top-8, eight
+// lanes against 16 at 16384 tokens 4.6 vs 4.8, at 32768 6.1 vs 6.9 (four 5.9; 65536 tokens 8.2
+// by four, 9.1 by eight; 24576 5.7 by four, 5.4 by eight); top-8 of 64 at 32768 8.1 by
+// eight vs 9.2.
 constexpr int64_t kNarrowMany = 8192;  // twice that from 33 experts up
-// 16-bit rows of more than 192 experts keep a wave per token below this count
-// (top-8 of 256 bf16 at 512 tokens 6.6 vs 7.0 us; at 2048 7.0 vs 7.1, at 4096 8.9 vs 7.4).
-constexpr int64_t kWideFew = 2048;
+constexpr int64_t kNarrowMost = 24576;
+
+// Where a wave per token stays the faster form: its chain holds four experts a
+// lane instead of up to 16, so rows of many experts start sooner, while a round of
+// its arg-max costs 0.15 us more. So it keeps one or two tokens of more than 128
+// experts, and, while all tokens' waves run at once, few picks of them: fp32 / bf16,
+// wave against 16 lanes, one token, top-2 of 160 2.9 / 3.1 vs 3.1 / 3.5, top-8 of 256 5.5 vs
+// 6.6 (bf16 keeps waves); 512 tokens, top-2 of 256 3.81 vs 3.88, top-6 5.25 vs 5.24; bf16 512
+// tokens, top-2 of 144 3.66 vs 3.68, of 192 3.76 vs 3.91, top-6 of 176 5.11 vs 5.18, of
+// 192 5.20 vs 5.01; 2047 tokens, top-2 of 160 3.98 vs 3.75,
+// top-1 of 176 3.58 vs 3.92; 2048, top-6 of 256 5.97 vs
+// 6.10, top-1 3.92 vs 4.40; 3000, top-4 5.4 vs 5.5, top-6 6.64 vs 6.26. (16-bit rows are moved an expert a lane by 16 lanes, so they gain less.)
+template <class C>
+bool keeps_waves(int64_t tokens, int n, int k) {
+  const int stripes = (n + kSoftmaxLanes - 1) / kSoftmaxLanes;
+  if (stripes <= 8) return false;
+  if (tokens <= 2) return true;
+  if constexpr (C::VEC == 8) {
+    if (stripes > 12) return tokens <= 2048 || (tokens <= 3072 && k <= 4);
+    return tokens <= (k == 1 && stripes > 10 ? 3072 : 1024) && k <= (stripes <= 10 ? 2 : stripes == 11 ? 6 : 4);
+  } else {
+    return stripes > 12 && tokens <= 1024 && (tokens <= 4 || k <= (tokens <= 64 ? 6 : 5));
+  }
+}
 
 }  // namespace
 
@@ -581,11 +604,11 @@ extern "C" int32_t launch_moe_router_fwd(const void* logits, float* topk_weights
       return launch_status();
     };
     if (small_grid && n <= kSoftmaxLanes) return groups(IntC<4>{}, IntC<1>{});
+    if (small_grid && n <= 2 * kSoftmaxLanes && num_tokens > kNarrowMost) return groups(IntC<4>{}, IntC<2>{});
     if (small_grid && n <= 4 * kSoftmaxLanes && num_tokens >= (n <= 2 * kSoftmaxLanes ? kNarrowMany : 2 * kNarrowMany)) {
       return n <= 2 * kSoftmaxLanes ? groups(IntC<8>{}, IntC<2>{}) : groups(IntC<8>{}, IntC<4>{});
     }
-    const bool waves = C::VEC == 8 && n > 12 * kSoftmaxLanes && num_tokens < kWideFew;
-    if (small_grid && !waves) {
+    if (small_grid && !keeps_waves<C>(num_tokens, n, kk)) {
       switch ((n + kSoftmaxLanes - 1) / kSoftmaxLanes) {
         case 2: return groups(IntC<16>{}, IntC<2>{});
         case 3: return groups(IntC<16>{}, IntC<3>{});

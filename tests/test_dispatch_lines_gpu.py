@@ -11,6 +11,7 @@ from custom_cuda_kernals_amd import _native as native
 from oracle import inputs, moe
 from tests._parity import bits_equal
 from tests._routes import kernels_of
+from tests.test_moe_router_gpu import _check as check_router
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +87,29 @@ def test_gather(ns, nd, h, kernel):
     _takes(lambda: native.token_gather_fwd(*d, dst), kernel)
     ok = (idx >= 0) & (idx < ns)
     assert bits_equal(dst, torch.where(ok[:, None], src[torch.where(ok, idx, 0)], 0.0)).all()
+
+
+WAVES = "moe_router_waves"
+F32 = torch.float32
+# (dtype, tokens, experts, top k, kernel)
+ROUTERS = [(BF16, 2, 129, 8, WAVES), (BF16, 3, 129, 3, "ELi16ELi10E"), (BF16, 3, 129, 2, WAVES),
+           (BF16, 1024, 160, 2, WAVES), (BF16, 1025, 160, 2, "ELi16ELi10E"), (BF16, 2, 128, 2, "ELi16ELi8E"),
+           (BF16, 3072, 161, 1, WAVES), (BF16, 3073, 161, 1, "ELi16ELi12E"), (BF16, 5, 176, 6, WAVES), (BF16, 5, 176, 7, "ELi16ELi12E"), (BF16, 5, 177, 4, WAVES),
+           (BF16, 5, 177, 5, "ELi16ELi12E"), (BF16, 2048, 193, 8, WAVES), (BF16, 2049, 193, 8, "ELi16ELi16E"),
+           (BF16, 2049, 193, 4, WAVES), (BF16, 3073, 193, 4, "ELi16ELi16E"),
+           (F32, 2, 160, 8, WAVES), (F32, 3, 160, 1, "ELi16ELi10E"), (F32, 4, 256, 8, WAVES),
+           (F32, 5, 256, 8, "ELi16ELi16E"), (F32, 64, 256, 6, WAVES), (F32, 65, 256, 6, "ELi16ELi16E"),
+           (F32, 1024, 200, 5, WAVES), (F32, 1025, 200, 5, "ELi16ELi16E"),
+           (BF16, 24576, 32, 2, "ELi8ELi2E"), (F32, 24577, 32, 2, "ELi4ELi2E"), (BF16, 24577, 17, 9, "ELi4ELi2E"),
+           (BF16, 24577, 33, 2, "ELi8ELi4E")]
+
+
+@pytest.mark.parametrize("dtype,t,e,k,kernel", ROUTERS)
+def test_router(dtype, t, e, k, kernel):
+    logits = inputs.router_inputs(t, e, dtype, seed=t + e)
+    logits[::3] = torch.round(logits[::3])  # many exact ties
+    logits[1::5, : e // 2] = float("-inf")
+    d = logits.cuda()
+    w, i = torch.empty(t, k, device="cuda"), torch.empty(t, k, dtype=torch.int64, device="cuda")
+    _takes(lambda: native.moe_router_fwd(d, w, i, True), kernel)
+    check_router(logits, k, True)
