@@ -95,9 +95,9 @@ constexpr int kPolTokenQ = kBufStorePolicy;
 // aligned x, VEC-aligned q, or RAGGED: any row length from VEC elements up and
 // any element-aligned pointers, by vectors from the row's own start (RowAny),
 // the last one overlapping its neighbour (overlap_first; the max and the codes
-// are per element).
+// are per element), stored as RowAnyT<CACHED> says.
 // ---------------------------------------------------------------------------
-template <class C, int FMT, int THREADS, int ITEMS, bool RAGGED = false>
+template <class C, int FMT, int THREADS, int ITEMS, bool RAGGED = false, bool CACHED = false>
 __global__ __launch_bounds__(THREADS) void fp8_token_resident(const void* __restrict__ x,
                                                               uint8_t* __restrict__ q,
                                                               float* __restrict__ scale,
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(THREADS) void fp8_token_resident(const void* __rest
     const float r = 1.0f / s;
     if (threadIdx.x == 0) scale[row] = s;
     const bool fast = fast_path_ok<FMT>(s, r, amax);
-    const std::conditional_t<RAGGED, RowAny, RowBuf<true, kPolTokenQ>> bq(q + row * cols, (uint32_t)cols);
+    const std::conditional_t<RAGGED, RowAnyT<CACHED>, RowBuf<true, kPolTokenQ>> bq(q + row * cols, (uint32_t)cols);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const uint32_t v = threadIdx.x + k * THREADS;
@@ -612,6 +612,14 @@ int32_t launch_token(const void* x, uint8_t* q, float* scale, int64_t m, int64_t
     using S = decltype(shape);
     if (vec_ok) {
       fp8_token_resident<C, FMT, S::kThreads, S::kItems><<<g, S::kThreads, 0, st>>>(x, q, scale, m, n);
+      return;
+    }
+    if constexpr (S::kThreads * S::kItems == 64) {
+      if (m * n <= kPlainCodesMax) {
+        fp8_token_resident<C, FMT, 64, 1, true, true><<<g, 64, 0, st>>>(x, q, scale, m, n);
+      } else {
+        fp8_token_resident<C, FMT, 64, 1, true><<<g, 64, 0, st>>>(x, q, scale, m, n);
+      }
     } else {
       fp8_token_resident<C, FMT, S::kThreads, S::kItems, true><<<g, S::kThreads, 0, st>>>(x, q, scale, m, n);
     }

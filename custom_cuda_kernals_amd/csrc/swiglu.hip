@@ -197,13 +197,15 @@ constexpr int kPolQ = kPolSC1 | kPolNT;
 // RAGGED: any row length from VEC elements up and any element-aligned
 // pointers, by vectors from the row's own start (RowAny), the last one
 // overlapping its neighbour (overlap_first): y, the amax and the codes are per
-// element, so the repeated elements change nothing. Bound by HBM like the
+// element, so the repeated elements change nothing; stored as RowAnyT<CACHED>
+// says. Bound by HBM like the
 // aligned rows, plus the cache lines that neighbouring rows share: bf16,
 // against the two-pass scalar kernel / aligned rows of the next whole vector,
 // [2048, 5461] 24.3 vs 12.8 us, [12291, 1365] 37.7 vs 19.2 / 17.7, [3072, 5461]
 // 40.5 vs 18.1 / 17.9, [1228, 13653] 50.2 vs 18.9 / 18.0, [585, 28665] 94.5 vs
 // 25.4 / 20.1, [256, 40001] 119.7 vs 14.4; fp32 [3072, 5461] 60.8 vs 26.8.
-template <class C, int THREADS, int ITEMS, int FMT, bool TAB, bool STATIC, bool LDSY = false, bool RAGGED = false>
+template <class C, int THREADS, int ITEMS, int FMT, bool TAB, bool STATIC, bool LDSY = false, bool RAGGED = false,
+          bool CACHED = false>
 __global__ __launch_bounds__(THREADS) void swiglu_fp8_resident(
     const void* __restrict__ gate, const void* __restrict__ up, uint8_t* __restrict__ yq,
     float* __restrict__ scale, float static_scale, int64_t rows, int64_t cols) {
@@ -310,7 +312,7 @@ __global__ __launch_bounds__(THREADS) void swiglu_fp8_resident(
     }
     const float r = 1.0f / s;
     const bool fast = fast_path_ok<FMT>(s, r, amax);
-    const std::conditional_t<RAGGED, RowAny, RowBuf<kRsrcQ, kPolQ>> bq(yq + row * cols, (uint32_t)cols);
+    const std::conditional_t<RAGGED, RowAnyT<CACHED>, RowBuf<kRsrcQ, kPolQ>> bq(yq + row * cols, (uint32_t)cols);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const uint32_t v = threadIdx.x + k * THREADS;
@@ -384,9 +386,10 @@ bool launch_swiglu_fp8_rows(const void* gate, const void* up, uint8_t* yq, float
     // The table pays for its per-workgroup fill only on long rows. Static
     // scales use these rows only from 768 threads (the flat stream otherwise).
     constexpr bool kTab = std::is_same_v<C, CodecBF16> && S::kThreads * S::kItems >= 1152;
-    auto go = [&](auto ldsy) {
+    auto go = [&](auto ldsy, auto cached) {
       constexpr bool kLdsY = decltype(ldsy)::value;
-      constexpr auto kernel = swiglu_fp8_resident<C, S::kThreads, S::kItems, FMT, kTab, STATIC, kLdsY, RAGGED>;
+      constexpr auto kernel =
+          swiglu_fp8_resident<C, S::kThreads, S::kItems, FMT, kTab, STATIC, kLdsY, RAGGED, decltype(cached)::value>;
       // bf16 rows with y in LDS run on a grid of the workgroups the device
       // holds at once, each looping over rows: one SiLU table fill per
       // workgroup instead of per row, no idle CU between rows, and the next
@@ -400,9 +403,11 @@ bool launch_swiglu_fp8_rows(const void* gate, const void* up, uint8_t* yq, float
       kernel<<<grid, S::kThreads, 0, st>>>(gate, up, yq, scale, static_scale, rows, cols);
       launched = true;
     };
-    if constexpr (S::kItems > 4) {
+    if constexpr (RAGGED && S::kThreads * S::kItems == 64) {
+      rows * cols <= kPlainCodesMax ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+    } else if constexpr (S::kItems > 4) {
       // (Ragged rows of 1024 x 8 would spill registers.)
-      if constexpr (!STATIC && !(RAGGED && S::kItems > 6)) go(std::true_type{});
+      if constexpr (!STATIC && !(RAGGED && S::kItems > 6)) go(std::true_type{}, std::false_type{});
     } else if constexpr (kTab && !STATIC && S::kThreads == 1024 && S::kItems >= 3) {
       // bf16 per-token rows of three and four vectors per thread park y in
       // LDS (48 / 64 KB) on the looping grid too, where the grid loops (more
@@ -419,12 +424,12 @@ bool launch_swiglu_fp8_rows(const void* gate, const void* up, uint8_t* yq, float
       const int64_t last = nvec - (int64_t)(S::kItems - 1) * S::kThreads;  // threads holding a last vector
       const int64_t resident = resident_groups<kParked>(S::kThreads);
       if (4 * last <= 3 * S::kThreads && resident > 0 && resident < rows) {
-        go(std::true_type{});
+        go(std::true_type{}, std::false_type{});
       } else {
-        go(std::false_type{});
+        go(std::false_type{}, std::false_type{});
       }
     } else if constexpr (!STATIC || (kTab && S::kThreads >= 768)) {
-      go(std::false_type{});
+      go(std::false_type{}, std::false_type{});
     }
   };
   // bf16 rows from a sweep over THREADS 256..1024 (step 128) x ITEMS 1..4,

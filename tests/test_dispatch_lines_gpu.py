@@ -8,8 +8,9 @@ import pytest
 import torch
 
 from custom_cuda_kernals_amd import _native as native
-from oracle import inputs, moe
-from tests._parity import bits_equal
+from oracle import eager, inputs, moe
+from oracle import fp8 as ofp8
+from tests._parity import assert_codes_equal, assert_f32_bits_equal, bits_equal
 from tests._routes import kernels_of
 from tests.test_moe_router_gpu import _check as check_router
 
@@ -113,3 +114,38 @@ def test_router(dtype, t, e, k, kernel):
     w, i = torch.empty(t, k, device="cuda"), torch.empty(t, k, dtype=torch.int64, device="cuda")
     _takes(lambda: native.moe_router_fwd(d, w, i, True), kernel)
     check_router(logits, k, True)
+
+
+def _ragged(rows: int, cols: int, seed: int, dtype=BF16) -> torch.Tensor:
+    return inputs.randn((rows, cols), dtype, seed=seed)
+
+
+# (rows, columns, kernel): the last template arguments are RAGGED, CACHED.
+TOKENS = [(300, 9, "ELi64ELi1ELb1ELb1E"), (4056, 259, "ELi64ELi1ELb1ELb0E"), (4000, 259, "ELi64ELi1ELb1ELb1E"),
+          (5, 511, "ELi64ELi1ELb1ELb1E"), (5, 513, "ELi64ELi2ELb1ELb0E"), (5, 8, "ELi64ELi1ELb0ELb0E")]
+
+
+@pytest.mark.parametrize("m,n,kernel", TOKENS)
+def test_fp8_token(m, n, kernel):
+    x = _ragged(m, n, m + n)
+    xd, q, s = x.cuda(), torch.empty(m, n, dtype=torch.float8_e4m3fn, device="cuda"), torch.empty(m, device="cuda")
+    _takes(lambda: native.fp8_quant_token_fwd(xd, q, s, "e4m3"), kernel)
+    codes, s_ref = ofp8.quant_token(x.float().numpy(), "e4m3")
+    assert_codes_equal(q, codes)
+    assert_f32_bits_equal(s, s_ref)
+
+
+# (rows, columns, kernel): RAGGED, CACHED as above, after TAB, STATIC and LDSY.
+GATED = [(300, 9, "ELb0ELb0ELb0ELb1ELb1E"), (4056, 259, "ELb0ELb0ELb0ELb1ELb0E"), (4000, 259, "ELb0ELb0ELb0ELb1ELb1E"),
+         (5, 513, "ELi64ELi2ELi4ELb0ELb0ELb0ELb1ELb0E")]
+
+
+@pytest.mark.parametrize("m,n,kernel", GATED)
+def test_swiglu_fp8_token(m, n, kernel):
+    g, u = inputs.swiglu_inputs(m, n, BF16, seed=n)
+    gd, ud = g.cuda(), u.cuda()
+    q, s = torch.empty(m, n, dtype=torch.float8_e5m2, device="cuda"), torch.empty(m, device="cuda")
+    _takes(lambda: native.swiglu_fp8_fwd(gd, ud, q, s, "e5m2", None), kernel)
+    codes, s_ref, _ = eager.swiglu_fp8(g, u, "e5m2", None)
+    assert_codes_equal(q, codes)
+    assert_f32_bits_equal(s, s_ref)
