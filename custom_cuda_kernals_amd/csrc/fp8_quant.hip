@@ -208,6 +208,17 @@ __global__ __launch_bounds__(256) void fp8_token_generic(const void* __restrict_
   }
 }
 
+constexpr int kTile = 128;
+constexpr int64_t kBlockPairMinTiles = 16384;
+constexpr int64_t kBlockSplitMaxTiles = 1024;  // one round of 512-thread workgroups (4 per CU)
+// Elements a ragged tile up to which the scalar kernel keeps it: one a thread of
+// its 256 (fp32 two), where a load a thread beats a quarter of a tile of them.
+// Graph-replayed on MI355X, scalar vs vectors: bf16 [1, 4100] 2.49 vs 2.61 us, [2, 517]
+// 2.41 vs 2.65, [4, 517] 2.88 vs 2.72, [16, 9] 2.18 vs 2.41, [16, 17] 2.57 vs 2.42; fp32
+// [1, 4097] 2.46 vs 2.83, [2, 517] 2.39 vs 2.85, [4, 517] 2.87 vs 2.92, [8, 517] 3.84 vs 2.94.
+template <class C>
+constexpr int64_t kBlockFewElements = C::VEC == 8 ? 256 : 512;
+
 // ---------------------------------------------------------------------------
 // Block granularity: one workgroup of THREADS per 128x128 tile, tile kept in
 // registers. Vector path needs n % VEC == 0 and aligned pointers. RSRC loads
@@ -216,16 +227,12 @@ __global__ __launch_bounds__(256) void fp8_token_generic(const void* __restrict_
 // stored as streaming stores; measured on MI355X against 256 threads with
 // global-pointer loads and cached stores: 6.55 vs 9.8 us at [2048, 4096]
 // bf16, 35.0 vs 38.0 us at [16384, 4096].
-// ---------------------------------------------------------------------------
-constexpr int kTile = 128;
-constexpr int64_t kBlockPairMinTiles = 16384;
-constexpr int64_t kBlockSplitMaxTiles = 1024;  // one round of 512-thread workgroups (4 per CU)
-
 //
 // RAGGED: any n from VEC up and any element-aligned pointers, by unaligned
 // vectors from each row's own start; a row's partial last vector is loaded as
 // the row's last VEC elements and moved to the front (partial_vector: the
 // elements dropped may belong to the tile on the left).
+// ---------------------------------------------------------------------------
 template <class C, int FMT, int THREADS, bool RSRC, int TW, bool SPLIT = false, bool RAGGED = false>
 __global__ __launch_bounds__(THREADS * TW) void fp8_block_resident(const void* __restrict__ x,
                                                                    uint8_t* __restrict__ q,
@@ -1020,7 +1027,7 @@ extern "C" int32_t launch_fp8_quant_block_fwd(const void* x, uint8_t* x_fp8, flo
         fp8_block_resident<C, FMT, 512, true, 1><<<grid, 512, 0, st>>>(x, x_fp8, scale, m, n);
       } else if (vec_ok) {
         fp8_block_resident<C, FMT, 512, false, 1><<<grid, 512, 0, st>>>(x, x_fp8, scale, m, n);
-      } else if (n >= C::VEC) {
+      } else if (n >= C::VEC && (m < kTile ? m : kTile) * (n < kTile ? n : kTile) > kBlockFewElements<C>) {
         // Ragged rows, against the scalar kernel / aligned rows of the next whole
         // vector, bf16 on MI355X: [8184, 4100] 88.6 vs 31.8 / 30.9 us, [6144, 5461]
         // 102.5 vs 32.0 / 30.9, [257, 513] fp16 37.2 vs 7.4, fp32 [3049, 11005]

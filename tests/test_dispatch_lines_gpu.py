@@ -149,3 +149,21 @@ def test_swiglu_fp8_token(m, n, kernel):
     codes, s_ref, _ = eager.swiglu_fp8(g, u, "e5m2", None)
     assert_codes_equal(q, codes)
     assert_f32_bits_equal(s, s_ref)
+
+
+BLOCK, SCALAR = "fp8_block_resident", "fp8_block_generic"
+# (dtype, rows, columns, kernel)
+BLOCKS = [(BF16, 1, 4101, SCALAR), (BF16, 2, 129, SCALAR), (BF16, 3, 129, BLOCK), (BF16, 28, 9, SCALAR),
+          (BF16, 29, 9, BLOCK), (BF16, 500, 7, SCALAR), (F32, 4, 129, SCALAR), (F32, 5, 129, BLOCK),
+          (F32, 102, 5, SCALAR), (F32, 103, 5, BLOCK), (BF16, 1, 4096, BLOCK)]
+
+
+@pytest.mark.parametrize("dtype,m,n,kernel", BLOCKS)
+def test_fp8_block(dtype, m, n, kernel):
+    x = _ragged(m, n, m + n, dtype)
+    xd, q = x.cuda(), torch.empty(m, n, dtype=torch.float8_e4m3fn, device="cuda")
+    s = torch.empty((m + 127) // 128, (n + 127) // 128, device="cuda")
+    _takes(lambda: native.fp8_quant_block_fwd(xd, q, s, "e4m3"), kernel)
+    codes, s_ref = ofp8.quant_block(x.float().numpy(), "e4m3")
+    assert_codes_equal(q, codes)
+    assert_f32_bits_equal(s, s_ref)
