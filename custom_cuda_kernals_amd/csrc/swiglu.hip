@@ -30,11 +30,14 @@ __device__ inline float swiglu1(float g, float u) {
 // per step, the next step's loads issued before this step's math. It uses the
 // arithmetic SiLU for every dtype: with the LDS table (and its per-workgroup
 // fill) the bf16 stream measured slower on MI355X (111.4 vs 109.9 us at
-// 8192 x 14336, 233.8 vs 218.8 us at 16384 x 14336). The last workgroup also takes
-// the `tail` elements past the last vector: in a launch of their own they cost 1.6
-// us more (graph-replayed on MI355X, bf16 [301, 11007] 6.8 vs 5.5 us, [33, 101] 3.7 vs
-// 2.0, static-scale FP8 [301, 5461] 6.4 vs 4.9) and 3.5 us of a call's host time.
-template <class C, int THREADS, int UNROLL>
+// 8192 x 14336, 233.8 vs 218.8 us at 16384 x 14336). TAIL: the last workgroup also
+// takes the `tail` elements past the last vector: in a launch of their own they
+// cost 1.6 us more (graph-replayed on MI355X, bf16 [301, 11007] 6.8 vs 5.5 us, [33, 101]
+// 3.7 vs 2.0, static-scale FP8 [301, 5461] 6.4 vs 4.9) and 3.5 us of a call's host
+// time. Whole vectors take the kernel without that code, whose registers and
+// instructions cost the small static-scale streams up to 0.2 us (fp32 [16, 517] 3.0 vs
+// 3.2, [1, 4100] 2.9 vs 3.1).
+template <class C, int THREADS, int UNROLL, bool TAIL>
 __global__ __launch_bounds__(THREADS) void swiglu_flat(const u32x4* __restrict__ gate,
                                                        const u32x4* __restrict__ up,
                                                        u32x4* __restrict__ y, int64_t nvec, int tail) {
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(THREADS) void swiglu_flat(const u32x4* __restrict__
     }
     load(base + stride);
   }
-  if (blockIdx.x == gridDim.x - 1 && (int)threadIdx.x < tail) {
+  if (TAIL && blockIdx.x == gridDim.x - 1 && (int)threadIdx.x < tail) {
     const int64_t i = nvec * C::VEC + threadIdx.x;
     C::store1(y, i, swiglu1<C>(C::load1(gate, i), C::load1(up, i)));
   }
@@ -97,7 +100,7 @@ __device__ inline void swiglu_fp8_static1(const void* gate, const void* up, uint
 // max |y| * (1/s) is inside the fast range, the exact path otherwise. The
 // static kernels also store s into scale_out[0] when given one (the scale
 // tensor the Python API returns), so a static call is one launch.
-template <class C, int FMT, int THREADS, int UNROLL, bool TAB>
+template <class C, int FMT, int THREADS, int UNROLL, bool TAB, bool TAIL>
 __global__ __launch_bounds__(THREADS) void swiglu_fp8_static_flat(const u32x4* __restrict__ gate,
                                                                  const u32x4* __restrict__ up,
                                                                  uint8_t* __restrict__ yq, float s,
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(THREADS) void swiglu_fp8_static_flat(const u32x4* _
     load(base + stride);
   }
   // The elements past the last vector, as in swiglu_flat.
-  if (blockIdx.x == gridDim.x - 1 && (int)threadIdx.x < tail) {
+  if (TAIL && blockIdx.x == gridDim.x - 1 && (int)threadIdx.x < tail) {
     swiglu_fp8_static1<C, FMT>(gate, up, yq, s, r, nvec * VEC + threadIdx.x);
   }
 }
@@ -506,9 +509,10 @@ extern "C" int32_t launch_swiglu_fwd(const void* gate, const void* up, void* y, 
         // at most 3 workgroups per CU (4 fit): 107.3-107.9 vs 108.0-108.5 us
         // (fp16 107.4 vs 108.4, fp32 216.1 vs 218.4).
         constexpr int THREADS = 512, UNROLL = 2;
-        swiglu_flat<C, THREADS, UNROLL>
-            <<<flat_grid((nvec + UNROLL - 1) / UNROLL, THREADS, 1 << 20), THREADS, kLdsForGroupsPerCu<3>, st>>>(
-                g4, u4, y4, nvec, (int)(n % C::VEC));
+        const int tail = (int)(n % C::VEC);
+        auto kernel = tail == 0 ? swiglu_flat<C, THREADS, UNROLL, false> : swiglu_flat<C, THREADS, UNROLL, true>;
+        kernel<<<flat_grid((nvec + UNROLL - 1) / UNROLL, THREADS, 1 << 20), THREADS, kLdsForGroupsPerCu<3>, st>>>(
+            g4, u4, y4, nvec, tail);
         done = n;
       }
     }
@@ -541,21 +545,24 @@ extern "C" int32_t launch_swiglu_fp8_fwd(const void* gate, const void* up, uint8
         const int64_t nvec = n / C::VEC;
         const u32x4* g4 = static_cast<const u32x4*>(gate);
         const u32x4* u4 = static_cast<const u32x4*>(up);
+        const int tail = (int)(n % C::VEC);
         bool tab = false;
         if constexpr (std::is_same_v<C, CodecBF16>) {
           if (nvec >= kTabMinVec) {
             constexpr int kPer = kTabThreads * kTabUnroll;
-            swiglu_fp8_static_flat<C, FMT, kTabThreads, kTabUnroll, true>
-                <<<flat_grid((nvec + kPer - 1) / kPer, 1, 1 << 20), kTabThreads, 0, st>>>(
-                    g4, u4, y_fp8, static_scale, nvec, (int)(n % C::VEC), scale);
+            auto kernel = tail == 0 ? swiglu_fp8_static_flat<C, FMT, kTabThreads, kTabUnroll, true, false>
+                                    : swiglu_fp8_static_flat<C, FMT, kTabThreads, kTabUnroll, true, true>;
+            kernel<<<flat_grid((nvec + kPer - 1) / kPer, 1, 1 << 20), kTabThreads, 0, st>>>(
+                g4, u4, y_fp8, static_scale, nvec, tail, scale);
             tab = true;
           }
         }
         if (!tab && nvec > 0) {
           constexpr int UNROLL = 4;
-          swiglu_fp8_static_flat<C, FMT, 256, UNROLL, false>
-              <<<flat_grid((nvec + UNROLL - 1) / UNROLL, 256, 1 << 20), 256, 0, st>>>(
-                  g4, u4, y_fp8, static_scale, nvec, (int)(n % C::VEC), scale);
+          auto kernel = tail == 0 ? swiglu_fp8_static_flat<C, FMT, 256, UNROLL, false, false>
+                                  : swiglu_fp8_static_flat<C, FMT, 256, UNROLL, false, true>;
+          kernel<<<flat_grid((nvec + UNROLL - 1) / UNROLL, 256, 1 << 20), 256, 0, st>>>(
+              g4, u4, y_fp8, static_scale, nvec, tail, scale);
         }
         if (nvec > 0) done = n;
       }

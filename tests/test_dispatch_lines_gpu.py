@@ -167,3 +167,18 @@ def test_fp8_block(dtype, m, n, kernel):
     codes, s_ref = ofp8.quant_block(x.float().numpy(), "e4m3")
     assert_codes_equal(q, codes)
     assert_f32_bits_equal(s, s_ref)
+
+
+@pytest.mark.parametrize("dtype", [BF16, torch.float16, F32], ids=lambda d: str(d).split(".")[-1])
+def test_swiglu_streams_of_whole_vectors_have_no_tail(dtype):
+    vec = 16 // dtype.itemsize
+    for n, tail in ((64 * vec, "Lb0EE"), (64 * vec + 1, "Lb1EE"), ((1 << 17) * vec, "Lb0EE"), ((1 << 17) * vec + 1, "Lb1EE")):
+        g, u = inputs.swiglu_inputs(1, n, dtype, seed=n)
+        gd, ud, y = g.cuda(), u.cuda(), torch.empty(1, n, dtype=dtype, device="cuda")
+        q, s = torch.empty(1, n, dtype=torch.float8_e4m3fn, device="cuda"), torch.empty(1, device="cuda")
+        for call in (lambda: native.swiglu_fwd(gd, ud, y), lambda: native.swiglu_fp8_fwd(gd, ud, q, s, "e4m3", 0.05)):
+            (name, _), = kernels_of(call)
+            assert "_flat" in name and tail in name, name
+        y_ref = eager.swiglu(g, u)
+        assert bits_equal(y, y_ref).all()
+        assert_codes_equal(q, ofp8.quant_static(y_ref.float().numpy(), 0.05, "e4m3"))
