@@ -16,9 +16,10 @@
 // threads cover at once, a thread per (head, chunk) of the token; while the
 // grid fits one round of resident workgroups, a thread per (head, chunk)
 // with the token's cos/sin row staged in LDS. Any other number of chunks, and
-// inputs small enough to be on chip still, take rope_heads: a thread per
+// 16-bit inputs small enough to be on chip still, take rope_heads: a thread per
 // (head, chunk) for any of both counts.
-// All accesses are 16 bytes; a wave covers whole 128-byte cache lines.
+// All accesses are 16 bytes; where a half is whole 128-byte lines, a wave covers
+// whole ones (rope_heads' SPLIT halves do not).
 #include "launch.hpp"
 
 namespace cck {
@@ -121,7 +122,17 @@ __global__ __launch_bounds__(256) void rope_scalar(const void* q, const void* k,
 // One token per workgroup, a thread per (head, chunk) of it, for any number of
 // chunks: t = h * chunks + c is split by `magic` = ceil(2^32 / chunks), exact
 // for t < 65536 (the launcher's bound). Threads loop when the token has more
-// than 1024 of them.
+// than 1024 of them. SPREAD: a few tokens take gridDim.y workgroups of 256 each. Against
+// one workgroup a token / the kernels that served these before (the scalar kernel,
+// and 256 threads walking the heads), graph-replayed on MI355X: bf16 40 / 40 heads of
+// 96 at 16 tokens 2.32 vs 2.53 / 2.35 us, at 128 2.53 vs 2.76 / 3.71; fp32 2.18 vs 2.78 /
+// 2.37; fp32 8 / 8 heads of 512 at 1 token 2.11 vs 2.53 / 2.25; fp32 64 / 8 heads of 128
+// at 16 2.14 vs 2.77 / 3.47. At 256 tokens no different (3.03 vs 3.08 us).
+//
+// The code starts on a page: between other kernels it runs from a cold
+// instruction cache, and the same instructions at other places of the code object
+// took up to 4 % longer there (64 / 8 heads of 128, 2048 tokens, in a decoder block
+// 14.6 us on a page, 15.0 and 15.2 elsewhere).
 //
 // The accesses come in two more policies than the streaming ones above:
 //   ONCHIP: cached loads, for inputs that the Infinity Cache still holds from
@@ -132,8 +143,8 @@ __global__ __launch_bounds__(256) void rope_scalar(const void* q, const void* k,
 //     write twice.
 enum RopePolicy : int { kRopeStream, kRopeOnChip, kRopeSplit };
 
-template <class C, RopePolicy P>
-__global__ __launch_bounds__(1024) void rope_heads(const void* q, const void* k, const float* __restrict__ cos_t,
+template <class C, RopePolicy P, bool SPREAD>
+__attribute__((aligned(4096))) __global__ __launch_bounds__(1024) void rope_heads(const void* q, const void* k, const float* __restrict__ cos_t,
                                                    const float* __restrict__ sin_t, void* q_out, void* k_out,
                                                    int64_t tokens, int64_t seq_len, int hq, int hkv, int chunks,
                                                    uint32_t magic) {
@@ -150,7 +161,7 @@ __global__ __launch_bounds__(1024) void rope_heads(const void* q, const void* k,
     const char* ks = static_cast<const char*>(k) + tok * k_bytes;
     const RowBuf<true, kStore> qo(static_cast<char*>(q_out) + tok * q_bytes, q_bytes);
     const RowBuf<true, kStore> ko(static_cast<char*>(k_out) + tok * k_bytes, k_bytes);
-    for (uint32_t t = threadIdx.x; t < n; t += blockDim.x) {
+    for (uint32_t t = threadIdx.x + (SPREAD ? blockIdx.y * 256u : 0u); t < n; t += SPREAD ? gridDim.y * 256u : blockDim.x) {
       const uint32_t h = __umulhi(t, magic), c = t - h * (uint32_t)chunks;
       const bool isq = h < (uint32_t)hq;
       const uint32_t off = (isq ? h : h - (uint32_t)hq) * 2u * half_bytes + c * 16u;
@@ -355,28 +366,49 @@ extern "C" int32_t launch_rope_fwd(const void* q, const void* k, const void* cos
     // 5.16 vs 5.79 at 512) and more (103.9 vs 108.4 us at 16384) do not.
     const int heads = hq + hkv;
     const int waves = chunks > 0 ? (heads * chunks + 63) / 64 : 0;
-    // rope_heads, for the chunk counts no kernel above is built for and for
-    // inputs that fit the Infinity Cache (kRopeOnChipBytes). Measured on MI355X
-    // through the Python API, rotating over three sets of buffers (and, after the
-    // slash, over 2 GB of them, which no cache holds): halves of 96 and 80 bytes,
-    // SPLIT against the scalar kernel, fp16 32 / 32 heads of 96 at [2, 2048] 16.4
-    // vs 39.9 us (101 MB; / 22.3), bf16 32 / 8 heads of 80 at [1, 8192] 21.4, with
-    // streaming accesses instead 33.6 and 39.1. Whole 64-byte pieces, ONCHIP
-    // against the streaming kernels: bf16 32 / 8 heads of 128 at [1, 2048] 7.6 vs
-    // 8.4 (/ 9.5 vs 9.1), [1, 4096] 13.2 vs 15.3 (/ 16.4 vs 15.6); fp32 [1, 2048] 13.3
-    // vs 15.3; 16 / 16 heads of 64 at [1, 8192] 11.5 vs 16.5 (/ 16.8 vs 17.0). q and k
-    // come from the projections just before, so the first figure counts while the
-    // cache holds them; the gain fades towards its size (84 MB of input: 26.4 vs 27.9 /
-    // 29.6 vs 27.9, 16 / 4 heads of 256 28.2 vs 28.0; 151 MB loses, 50.2 vs 48.3), so
-    // the line is at a quarter of the 256 MB.
+    // rope_heads, for the chunk counts no kernel above is built for, and for
+    // inputs that fit the Infinity Cache with room to spare (kRopeOnChipBytes),
+    // since the projections have just written q and k. Halves of 96 and 80 bytes,
+    // SPLIT against the scalar kernel: fp16 32 / 32 heads of 96 at [2, 2048] 16.4 vs 39.9
+    // us (101 MB), bf16 32 / 8 heads of 80 at [1, 8192] 21.4, with streaming accesses
+    // instead 33.6 and 39.1. Whole 64-byte pieces, ONCHIP against the streaming
+    // kernels (both on a page), as a decoder block's RoPE right after its q, k and v
+    // projections (in place, kernel times under rocprofv3, median of 50) / on three sets
+    // of buffers in turn / on 2 GB of them, which no cache holds, bf16:
+    //   32 / 8 heads of 128  2048 tokens 10.2 vs 10.4 / 7.7 vs 8.4 / 9.3 vs 8.9 us
+    //                        4096        15.5 vs 15.6 / 13.4 vs 15.3 / 16.1 vs 15.2
+    //                        6000        24.2 vs 25.0 (FP8 block 23.9 vs 24.5)
+    //   64 / 8 heads of 128  1024        9.5 vs 9.2 / 6.9 vs 7.8 / 8.7 vs 8.3
+    //                        2048        14.6 vs 14.8 / 12.3 vs 14.4 / 15.1 vs 14.4
+    //                        3500        23.0 vs 23.1 (FP8 block 25.2 vs 25.6)
+    //   28 / 4 heads of 128  4096        13.1 vs 14.1 / 11.3 vs 14.0 / 13.2 vs 13.6
+    //   32 / 8 heads of 64   8192        16.9 vs 18.3; 12000 28.2 vs 30.7
+    // So behind a projection it gains up to 7 % (most where 256 threads would not
+    // fill) and loses at most 3; q and k that have left the chip lose up to 8 %. The
+    // gain fades towards the cache's size (84 MB on three sets 26.4 vs 27.9, 151 MB
+    // 50.2 vs 48.3), so the line is at a quarter of the 256 MB. fp32 keeps streaming
+    // where a kernel is built for its chunks: in the block, 32 / 8 heads of 128 at
+    // 1024 / 2048 tokens 9.2 / 15.6 us ONCHIP against 8.3 / 14.6. It takes rope_heads,
+    // streaming, for tokens of more than 1024 pairs and for those that leave a
+    // quarter of the 256 threads idle: 64 / 8 heads of 128 at 128 tokens 2.9 vs 3.7, at
+    // 1024 14.2 vs 14.2; 12 / 12 of 64 at 4096 9.9 vs 11.3.
     constexpr int64_t kRopeOnChipBytes = 64ll << 20;
-    const bool on_chip = tokens * (int64_t)heads * d * C::kBytes <= kRopeOnChipBytes;
+    constexpr int64_t kRopeSpreadTokens = 128;
+    const bool fits = tokens * (int64_t)heads * d * C::kBytes <= kRopeOnChipBytes;
+    const bool built = chunks == 4 || chunks == 8 || chunks == 16 || chunks == 32;
+    const bool on_chip = fits && (C::kBytes == 2 || !built);
     auto run_heads = [&](auto policy) {
       const int64_t n = (int64_t)heads * chunks;
-      const int nt = n < 1024 ? (int)((n + 63) / 64 * 64) : 1024;
       const uint32_t magic = (uint32_t)(((uint64_t(1) << 32) + chunks - 1) / chunks);
-      rope_heads<C, (RopePolicy)decltype(policy)::value><<<flat_grid(tokens, 1, kMaxRowGroups), nt, 0, st>>>(
-          q, k, ct, sn, q_out, k_out, tokens, seq_len, hq, hkv, chunks, magic);
+      constexpr RopePolicy P = (RopePolicy)decltype(policy)::value;
+      if (n > 256 && tokens <= kRopeSpreadTokens) {
+        const dim3 grid((unsigned)tokens, (unsigned)((n + 255) / 256));
+        rope_heads<C, P, true><<<grid, 256, 0, st>>>(q, k, ct, sn, q_out, k_out, tokens, seq_len, hq, hkv, chunks, magic);
+      } else {
+        const int nt = n < 1024 ? (int)((n + 63) / 64 * 64) : 1024;
+        rope_heads<C, P, false><<<flat_grid(tokens, 1, kMaxRowGroups), nt, 0, st>>>(
+            q, k, ct, sn, q_out, k_out, tokens, seq_len, hq, hkv, chunks, magic);
+      }
     };
     // (chunks == 1 has no 32-bit magic and, like 2, packs many tokens into a workgroup.)
     const bool heads_ok = chunks > 2 && (int64_t)heads * chunks <= 65536;
@@ -398,6 +430,8 @@ extern "C" int32_t launch_rope_fwd(const void* q, const void* k, const void* cos
       run_heads(IntC<kRopeSplit>{});
     } else if (heads_ok && on_chip) {
       run_heads(IntC<kRopeOnChip>{});
+    } else if (heads_ok && fits && (heads * chunks > 1024 || (chunks == 8 && heads * chunks <= 192))) {
+      run_heads(IntC<kRopeStream>{});
     } else if (chunks == 8) {
       // Tokens of at most 32 heads (and more than 128): with at most 6
       // workgroups per CU (8 fit) this 256-thread shape measured 102.0 vs

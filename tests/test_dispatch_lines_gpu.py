@@ -182,3 +182,25 @@ def test_swiglu_streams_of_whole_vectors_have_no_tail(dtype):
         y_ref = eager.swiglu(g, u)
         assert bits_equal(y, y_ref).all()
         assert_codes_equal(q, ofp8.quant_static(y_ref.float().numpy(), 0.05, "e4m3"))
+
+
+# rope_heads streaming, with cached loads, with cached loads and stores; SPREAD last
+STREAM, ONCHIP, SPLIT = (f"RopePolicyE{p}EL" for p in (0, 1, 2))
+# (dtype, tokens, q heads, kv heads, head dim, kernel)
+ROPES = [(BF16, 128, 40, 40, 96, SPLIT + "b1E"), (BF16, 129, 40, 40, 96, SPLIT + "b0E"), (BF16, 1, 32, 8, 96, SPLIT + "b0E"),
+         (F32, 3, 8, 8, 512, ONCHIP + "b1E"), (F32, 300, 32, 8, 96, ONCHIP + "b0E"), (BF16, 3, 128, 8, 128, ONCHIP + "b1E"),
+         (BF16, 2048, 32, 8, 128, ONCHIP + "b0E"), (F32, 1100, 32, 8, 128, "rope_tokens"),
+         (F32, 3000, 12, 12, 64, STREAM + "b0E"), (F32, 100, 64, 8, 128, STREAM + "b1E"),
+         (F32, 300, 64, 8, 128, STREAM + "b0E"), (F32, 3000, 16, 16, 64, "rope_tokens")]
+
+
+@pytest.mark.parametrize("dtype,s,hq,hkv,d,kernel", ROPES)
+def test_rope(dtype, s, hq, hkv, d, kernel):
+    q, k, cos, sin = inputs.rope_inputs(1, s, hq, hkv, d, dtype=dtype, seed=s + d, theta=10000.0)
+    t = [v.cuda() for v in (q, k, cos, sin)]
+    qo, ko = torch.empty_like(t[0]), torch.empty_like(t[1])
+    _takes(lambda: native.rope_fwd(*t, qo, ko), kernel)
+    q_ref, k_ref = eager.rope(q, k, cos, sin)
+    assert bits_equal(qo, q_ref).all() and bits_equal(ko, k_ref).all()
+    native.rope_fwd(*t, t[0], t[1])
+    assert bits_equal(t[0], q_ref).all() and bits_equal(t[1], k_ref).all()
