@@ -13,9 +13,10 @@ expert is accepted only at an exact tie (torch's topk orders those its own
 way; the kernel takes the lower expert index).
 
 Up to 8 experts one lane holds a token; a group of four lanes (16-expert
-stripes) holds one of 9 to 32 experts, and of up to 64 from 4096 tokens on;
-a group of eight lanes one of 65 to 256 experts from 8192 tokens (up to 128
-experts) or 12288; otherwise a wave does: the cases cover each form's edges
+stripes) one of 9 to 16 experts, and of up to 32 past 24576 tokens; a group of
+eight lanes one of up to 32 experts from 8192 tokens and of up to 64 from 16384;
+a wave one of more than 128 experts where tokens or picks are few; a group of 16
+lanes the others: the cases cover each form's edges
 (expert counts around 8, 16, 32, 64, 128 and 256, k = E, token counts that
 leave a partial workgroup or cross the thresholds) and rows that are not
 16-byte aligned.

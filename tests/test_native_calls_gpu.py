@@ -1,8 +1,9 @@
 """The one-call form of the Python API against the long way (torch.empty and
 the validating *_fwd functions): the same outputs (shape, stride, dtype, device
 and bits) over the forms both take; what the long way refuses is refused with
-its error; tensor subclasses, torch modes and functorch transforms go the long
-way; calls on a side stream and from several threads."""
+its error (type and message); tensor subclasses, torch modes and functorch
+transforms go the long way; calls on a side stream, from several threads, on
+inputs that another thread changes, and under capture, with replays."""
 
 from __future__ import annotations
 
@@ -58,6 +59,12 @@ def _calls(dtype):
     }
 
 
+def _calls_names():
+    return ["norm", "norm1d", "norm_param", "norm_fp8", "norm_fp8_1d", "norm_fp8_static", "swiglu", "swiglu_0d",
+            "swiglu_fp8", "swiglu_fp8_static", "rope", "block", "token", "tensor", "static", "gather", "combine",
+            "gather_fp8", "permutation", "router", "router_raw"]
+
+
 def _outputs(call):
     out = call()
     out = out if isinstance(out, tuple) else (out,)
@@ -76,18 +83,64 @@ def test_equals_the_long_way(dtype, monkeypatch):
         assert _outputs(c) == one[name], name
 
 
-def test_refused_as_before():
+def _refused():
     x, w = _r(4, 64), _r(64)
-    for call in (lambda: K.rmsnorm_residual(x, x[:, ::2], w), lambda: K.rmsnorm_residual(x, x.half(), w),
+    return (lambda: K.rmsnorm_residual(x, x[:, ::2], w), lambda: K.rmsnorm_residual(x, x.half(), w),
                  lambda: K.rmsnorm_residual(x, x, w[:32]), lambda: K.swiglu(x.t(), x.t()),
                  lambda: K.swiglu(x, x[:2]), lambda: K.fp8_quant(x[0]), lambda: K.fp8_quant(x, "e3m4"),
                  lambda: K.fp8_quant(x, "e4m3", "token", 0.5), lambda: K.swiglu_fp8(x, x.cpu()),
                  lambda: K.fp8_quant(x.double()), lambda: K.token_gather(x, torch.zeros(3, dtype=torch.int32).cuda()),
                  lambda: K.moe_router(x, 65), lambda: K.compute_permutation(torch.zeros(3, 2).cuda(), 4),
                  lambda: K.compute_permutation(torch.zeros(3, 2, dtype=torch.int64).cuda(), 257),
-                 lambda: K.rope(x.view(1, 4, 1, 64), x.view(1, 4, 1, 64), w.float(), w.float())):
+                 lambda: K.rope(x.view(1, 4, 1, 64), x.view(1, 4, 1, 64), w.float(), w.float()))
+
+
+def test_refused_as_before():
+    for call in _refused():
         with pytest.raises((ValueError, RuntimeError, TypeError)):
             call()
+
+
+def _errors(calls):
+    out = []
+    for call in calls:
+        with pytest.raises((ValueError, RuntimeError, TypeError)) as e:
+            call()
+        out.append((e.type, str(e.value)))
+    return out
+
+
+def test_refused_with_the_errors_of_the_long_way(monkeypatch):
+    one = _errors(_refused())
+    for name in NAMES:
+        monkeypatch.setattr(native, name, lambda *a: None)
+    assert _errors(_refused()) == one
+
+
+@pytest.mark.parametrize("name", _calls_names())
+def test_captured_calls(name):
+    """A call captured into a graph, its outputs from the capture's pool: every
+    replay gives the eager result, with eager calls of the same function between
+    the replays."""
+    call = _calls(torch.bfloat16)[name]
+    as_tuple = lambda out: out if isinstance(out, tuple) else (out,)
+    bits = lambda out: [t.contiguous().view(-1).view(torch.uint8).clone() for t in as_tuple(out)]
+    ref = bits(call())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = call()
+    for _ in range(4):
+        for t in as_tuple(out):
+            t.view(-1).view(torch.uint8).fill_(0xA5)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(bits(out), ref))
+        assert all(torch.equal(a, b) for a, b in zip(bits(call()), ref))
 
 
 def test_modes_and_subclasses_go_the_long_way():

@@ -2,8 +2,9 @@
 whose per-op tests cover only aligned buffers. The reference accepts them and
 handles them with scalar kernels (swiglu.cu:135,155; rope.cu:294-330;
 fp8_quant.cu:122,226); here each launcher checks alignment on the host and
-takes its scalar kernel, and the result must meet the same bar as the aligned
-path: the per-op tests' oracles and tolerances, reused.
+takes the form that allows it (unaligned vectors or a scalar kernel), and the
+result must meet the same bar as the aligned path: the per-op tests' oracles and
+tolerances, reused.
 
 A buffer is made unaligned by viewing a larger allocation from element 1
 (2 bytes for bf16 / fp16, 4 for fp32, 1 for FP8 codes).
