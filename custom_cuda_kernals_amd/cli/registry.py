@@ -247,6 +247,8 @@ REGISTRY: dict[str, OpSpec] = {
             memory_profile="HBM-bound: 2 B in + 2 B out per bf16 element plus the tables (config 4: 673 MB).",
             design=("one workgroup per token, a thread per (head, chunk) for 33-128 heads (320 threads at "
                     "config 4's 40), cos / sin read once per chunk (staged in LDS while the grid fits one round)",
+                    "any number of chunks, and 16-bit inputs small enough to be on chip (cached loads): a thread "
+                    "per (head, chunk) of a run of tokens",
                     "per-token buffer-resource stores with SC1 | NT"),
             target=">= 75 % of 8 TB/s at q [8, 4096, 32, 128] + k [8, 4096, 8, 128] bf16; bit-exact",
             reference=("baselines/rope.py:103-145", "csrc/kernels/rope.cu", "csrc/includes/rope.h:23-36"),
@@ -309,11 +311,13 @@ REGISTRY: dict[str, OpSpec] = {
             dtypes=("float32", "float16", "bfloat16", "fp8 (gather)"),
             memory_profile="HBM-bound row moves (gather 67 MB, combine k = 2 50 MB at the reference's shapes).",
             design=("four or eight destination rows per gather workgroup; one vector per thread on a flat grid "
-                    "for rows of more than 512 vectors and from 2^22 destination vectors",
-                    "two expert rows in flight per combine step",
-                    "the permutation bookkeeping as one stable counting-sort launch (compute_permutation with "
-                    "num_experts)"),
-            target="gather and the permutation bit-exact; combine equal to the j-order fp32 sum",
+                    "for rows of more than 512 vectors and from 2^22 destination vectors; one slice of each row "
+                    "per XCD where source rows repeat, and for ragged rows",
+                    "two expert rows in flight per combine step; the columns past the last 32 summed by further "
+                    "workgroups of the launch up to k = 16, by a second launch beyond",
+                    "the permutation bookkeeping as a stable counting sort (compute_permutation with "
+                    "num_experts): one launch, three from 65536 entries"),
+            target="gather and the permutation bit-exact; combine equal to torch-CPU's fp32 sum",
             reference=("baselines/token_permute.py:55-70, 215-251", "csrc/kernels/token_permute.cu",
                        "csrc/includes/token_permute.h:17-41"),
             python_api=("token_gather", "token_combine", "compute_permutation"),

@@ -489,7 +489,9 @@ struct RowBuf<false, SPOL> {
 // may start at any byte. Measured on MI355X, a 256 MiB copy by 16-byte vectors
 // (nontemporal): aligned 84.0 us; loads 8 / 4 / 2 bytes off 85.1 / 84.9 /
 // 86.8; stores off 87.6 / 87.6 / 88.2; both off 88.8 / 88.8 / 91.9. The last
-// n < VEC elements of such a row are a partial vector, moved one by one.
+// n < VEC elements of such a row are a partial vector: a load that overlaps its
+// neighbour, and at most three stores of 8, 4 and 2 bytes (codes: 4, 2 and 1), or
+// the same values stored once more where a step takes the overlap whole.
 // ---------------------------------------------------------------------------
 typedef u32x4 u32x4_any __attribute__((aligned(1)));
 typedef u32x2 u32x2_any __attribute__((aligned(1)));

@@ -4,18 +4,21 @@
 //
 // Each function takes its Python function's arguments by position and returns
 // its outputs, or None when the call is not the ordinary one (plain contiguous
-// torch.Tensors of the supported dtypes on one GPU, consistent shapes, some
-// work to do, and no torch function or dispatch mode, no functorch transform
-// active): the Python function then goes the long way, through torch.empty and
-// the validating *_fwd functions, which raise the errors. So the checks here
-// only have to be at least as strict as theirs.
+// unnamed torch.Tensors of the supported dtypes on one GPU, consistent shapes,
+// some work to do, and no torch function or dispatch mode, no functorch
+// transform active; a default device, set for the process or by `with
+// torch.device(...)`, is such a function mode): the Python function then goes the
+// long way, through torch.empty and the validating *_fwd functions, which raise
+// the errors. So the checks here only have to be at least as strict as theirs.
 //
-// Outputs come from at::empty, the allocator, stream and device of
-// torch.empty. What bounds a small call is this host path. Host time of a call
-// on [8, 4096] bf16, back to back, the long way vs this: RMSNorm 7.0 vs 5.5 us,
-// with per-token FP8 11.5 vs 6.4, SwiGLU + FP8 9.5 vs 5.5, per-token FP8 7.1 vs
-// 5.4, per-tensor (two launches) 10.5 vs 9.0, RoPE 6.5 vs 5.7; torch's own x.add_(0)
-// takes 4.9, a launch through the *_fwd functions alone 4.0.
+// Outputs come from at::empty or at::empty_strided, the allocator, stream and
+// device of torch.empty. What bounds a small call is this host path. Host time of a call
+// on [8, 4096] bf16, back to back, median of three processes each (which differ by
+// up to 10 %), the long way vs this: RMSNorm 6.1 vs 5.5 us, with per-token FP8 10.8
+// vs 6.3, SwiGLU + FP8 9.5 vs 5.6, per-token FP8 7.2 vs 5.6, RoPE 6.3 vs 5.9, the
+// permutation 6.9 vs 5.2, the router 7.5 vs 5.2; torch's own x.add_(0) takes 4.9, a
+// launch through the *_fwd functions alone 4.0. Of this, 0.1 to 0.3 us look at the
+// inputs again after the allocations and give the outputs the inputs' strides.
 #pragma once
 
 #include <ATen/ATen.h>

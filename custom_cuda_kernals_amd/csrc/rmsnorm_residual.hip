@@ -514,7 +514,15 @@ int32_t launch_rmsnorm(const void* x, const void* res, const void* w, void* y, u
   // [3001, 4100] 59.4 vs 23.1 us (3.7 TB/s; 20.6 for aligned rows of 4104),
   // [16384, 101] 51.0 vs 14.3, [16384, 1005] 100.7 vs 28.1, [1524, 11005] 97.0 vs
   // 34.8, [838, 20005] 123.6 vs 41.3; plain [4091, 4101] 76.7 vs 35.2; fp32
-  // per-token [8184, 2050] 129.8 vs 54.1.
+  // per-token [8184, 2050] 129.8 vs 54.1. The 20.6 of the aligned rows says that
+  // raggedness is the smaller part: both lists go from 256 x 2 to 256 x 3, so a row
+  // of 513 vectors leaves 255 of the third slots empty and pays their registers (four
+  // workgroups a CU).
+  // Past the last shape the looping kernel shows: aligned rows vs ragged ones two
+  // columns longer, buffers on chip, bf16 per-token 64 rows of 24584 / 24586 10.3 vs
+  // 80.1 us, 1024 rows 44.3 vs 152.5, 1024 of 28672 / 28674 47.8 vs 175.7 (24570, the
+  // last with a shape: 46.5); fp32 1024 of 12292 / 12294 34.4 vs 124.8; plain rows, up to
+  // 32768: 64 of 32768 / 32770 8.5 vs 82.3, 1024 of them 50.4 vs 154.9.
   bool done = false;
   if (!vec_ok) {
     if (cols < C::VEC) {

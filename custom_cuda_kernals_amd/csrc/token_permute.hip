@@ -15,11 +15,16 @@
 //   * h == 1, where the reduced dimension is contiguous: ATen's row sum
 //     (aten_row_sum).
 //
-// Design: one workgroup per output row (64-512 threads, sized to the row).
-// The row's index (and weight) is workgroup-uniform and read once into SGPRs;
-// the row then moves as 16-byte vectors (one per thread for the gather; 2-4
-// per thread times two expert rows in flight for the combine), nontemporal. Gather is byte movement
-// (dtype-agnostic); combine unpacks to fp32, accumulates and packs.
+// Design: the rows move as 16-byte vectors. Combine: one workgroup per token
+// (64-512 threads, sized to the row), whose indices and weights are
+// workgroup-uniform and read once into SGPRs, 2-4 vectors per thread times two
+// expert rows in flight; it unpacks to fp32, accumulates and packs. Gather is
+// byte movement (dtype-agnostic) in one of four forms: several rows per
+// workgroup, one vector per thread (token_gather_rows, _pf); the destination as
+// one flat stream, an index per vector (token_gather_flat); and a slice of every
+// row per XCD, where rows repeat (token_gather_slices). Loads and stores are
+// nontemporal but for repeated source rows and small outputs; each kernel says
+// why.
 //
 // Index hygiene: an index outside [0, n_src) makes a gathered row all zeros
 // and drops that (t, j) term from a combine, instead of reading out of bounds.
@@ -907,10 +912,14 @@ __device__ inline void perm_rank_chunk(const int64_t* __restrict__ ids, int64_t 
 // its chunk (before) and the others (after), one LDS atomic per id. Each
 // workgroup reads all n ids once more than a per-chunk count would, so the
 // grid is capped: at n = 12288 (2048 tokens, top 6) that is 12 workgroups and
-// 1.2 MB of L2 reads. kCombine counts through perm_count; it is used for
-// k <= 2 only: with more picks per token (distinct experts per token), a
-// wave's 64 entries hold at most 64 / k of any one expert, and the combining
-// step costs more than it saves (6.9 against 6.0 us at 2048 tokens x top 6).
+// 1.2 MB of L2 reads. kCombine counts through perm_count. It pays only where a
+// wave's ids repeat: with every token on the same experts 5.4 against 7.9 us at
+// 4096 tokens x top 1 and 10.4 against 32.5 at 32768, and nothing at 2048 x top
+// 2 (5.92, 5.88); uniform ids lose by it (4096 x 1 of 8 experts 5.00 against
+// 4.91 us, 16384 x 2 of 64 10.1 against 8.7, 2048 x 6 of 64 6.45 against 5.56).
+// It is used for k <= 2: with more picks per token (distinct experts per
+// token), a wave's 64 entries hold at most 64 / k of any one expert, which
+// bounds what a skewed routing can cost without it.
 template <bool kCombine>
 __global__ __launch_bounds__(kPermThreads) void moe_permutation(const int64_t* __restrict__ ids, int64_t n, int64_t k,
                                                                 int n_experts, int64_t chunk,
@@ -959,10 +968,14 @@ __global__ __launch_bounds__(kPermThreads) void moe_permutation(const int64_t* _
 }
 
 // Three launches from kPermSplitMin entries on, so that each id is counted
-// once: the cost of the one-launch kernel grows with n x workgroups (uniform
-// ids, top 8 of 256: 14.0 against 22.9 us at 16384 tokens, 26.4 against 81.2
-// at 65536; the one launch is faster up to 49152 entries). The output
-// buffers carry the intermediate results between the launches (stream order
+// once: the cost of the one-launch kernel grows with n x workgroups. One
+// launch against three, uniform ids: top 8 of 256 10.8 against 11.3 us at 49152
+// entries, 12.2 / 11.5 at 57344, 13.3 / 11.7 at 65536, 23.2 / 13.7 at 131072;
+// top 4 of 64 10.5 / 10.5, 11.9 / 10.6 and 13.0 / 10.7 at the first three; top 2
+// of 64, which combines its counts, 10.1 / 10.4 at 32768 and 11.9 / 10.5 at
+// 40960; top 1 of 8 9.9 / 10.0 at 24576 and 11.3 / 10.1 at 32768. So the two
+// meet at 24576 to 53000 entries, and between there and kPermSplitMin a call
+// takes up to 2.3 us more than it would in three launches. The output buffers carry the intermediate results between the launches (stream order
 // separates them):
 //   1. moe_permutation_count: workgroup c counts its own chunk per bucket and
 //      stores the counts in permute_index's memory as uint32 [G][nb];

@@ -11,7 +11,8 @@
  *     null stream);
  *   - empty work (a dimension <= 0) returns 0 without touching the device;
  *   - unaligned pointers and sizes that are not a multiple of the 16-byte
- *     vector width are accepted (scalar kernels handle them).
+ *     vector width are accepted (unaligned vectors or, where a kernel has no
+ *     such form, scalar kernels handle them).
  *
  * The reference declares its launchers with cudaError_t / cudaStream_t; both
  * are 32-bit-enum / pointer sized, so these declarations are ABI-compatible
@@ -150,7 +151,7 @@ int32_t launch_token_gather_fwd(const void* src, const int64_t* indices, void* d
  * products rounded to fp32 and summed in torch-CPU's order for (x.float() * w).sum(dim=1)
  * (j order, in ATen's 16-step blocks beyond k = 16, on the leading 32 * floor(h / 32)
  * columns; ATen's four-slot order on the rest; a row sum when hidden_dim == 1), the
- * sum rounded to dtype. Two launches when hidden_dim is not a multiple of 32.
+ * sum rounded to dtype. Two launches when k > 16 and hidden_dim is not a multiple of 32.
  * expert_output: [N, hidden_dim], unpermute_index: int64 [n_tokens, k], weights:
  * float32 [n_tokens, k], combined: [n_tokens, hidden_dim]. A negative index
  * drops its term.
